@@ -228,7 +228,9 @@ typedef struct dlg_opts {
                                 totals in a ring of mapped host words (a round
                                 whose output outgrows its buffer does nothing and
                                 is queued again after the buffer grows).  0 auto
-                                (4), 1 one round at a time, at most 8            */
+                                (4), 1 one round at a time, at most 8.  Id ranges
+                                of at most 16,384 ids go by whole-row ORs instead
+                                (same results) when this and reorder = 2 are unset */
     int32_t reserved[1];
 } dlg_opts;
 

@@ -304,6 +304,9 @@ struct BatchHook : RoundHook {
         }
         record(c, round);
     }
+    void on_finished(const std::vector<int> &first_empty) override {
+        for (int i = 0; i < B; i++) iters[i] = first_empty[i];
+    }
     // an instance's iteration count is the first round that gave it nothing new
     void record(const std::vector<u64> &c, int round) {
         for (int i = 0; i < B; i++) {

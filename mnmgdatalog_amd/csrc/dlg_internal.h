@@ -456,6 +456,13 @@ struct MapRef {
 };
 u64 bitmap_emit_maps(dlg_ctx *ctx, const u32 *words, const std::vector<MapRef> &maps, bool transposed, u64 *out,
                      u64 expect);
+// The same for row-major maps that each start at a whole emission tile of
+// `words` (emit_tile_words(rows * wpr) words each, the padding clear, nwords
+// in all): read out as they lie.  `out` is resized; the count is checked
+// against `expect` before anything is written (synchronises).
+u64 emit_tile_words(u64 nwords);
+void bitmap_emit_tiled(dlg_ctx *ctx, u32 *words, const std::vector<MapRef> &maps, u64 nwords, DBuf<u64> &out,
+                       u64 expect);
 // A W-row block of a map, emitted in tuple order at out through a padded
 // scratch copy (transposed back when `transposed`).  Returns its set bits.
 u64 bitmap_emit_block(dlg_ctx *ctx, const u32 *words, u32 lo, u64 W, u64 wpr, bool transposed, DBuf<u32> &scratch,
@@ -538,6 +545,16 @@ void relabel_rows(dlg_ctx *ctx, const int32_t *in, u64 n, const u32 *sigma, u32 
 u64 rowmap_emit_renumbered(dlg_ctx *ctx, RowMap &m, DBuf<u64> &out, u64 expect, const u32 *sigma);
 // Fraction of the index's rows (k, v) whose reverse (v, k) is also a row.
 double reciprocal_fraction(dlg_ctx *ctx, const Index &ix);
+
+// ------------------------------------------------------------- TC row ORs (k_tcdense.hip)
+// TC over id ranges (one for a plain run, the batched form's `starts`, see
+// rowmap_init) of at most TD_MAX_W ids each: rounds of whole-row ORs.  The
+// sorted relation to `out`, its size to *total, the join rows added to *raw;
+// returns the round count.  `iters` (may be null): per range of `starts`, the
+// first round that gave it nothing new.
+constexpr u64 TD_MAX_W = 1ull << 14;
+int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, const std::vector<u32> *starts, int max_it,
+                 DBuf<u64> &out, u64 *total, u64 *raw, std::vector<int> *iters);
 
 // ------------------------------------------------------------- SG row ORs (k_sgrows.hip)
 struct SgRows {

@@ -62,6 +62,9 @@ struct RoundHook {
     // nn in all), so the tuples are never built.
     virtual bool by_source() const { return false; }
     virtual void on_round_sources(dlg_ctx *, const u32 *, const u32 *, u64, u64, int) {}
+    // TC by row ORs counts a round's new tuples per id range itself: after the
+    // last round, each range's first round without new tuples.
+    virtual void on_finished(const std::vector<int> &) {}
 };
 
 // Id-range width up to which TC / SG keep the full relation as a bitmap

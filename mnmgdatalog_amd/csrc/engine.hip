@@ -275,6 +275,20 @@ static bool tc_use_rows(const Opts &o, u64 n, const u32 *ib, const std::vector<u
     return wmax <= BITMAP_MAX_W && bits <= BITMAP_MAX_W * BITMAP_MAX_W;
 }
 
+// TC by row ORs (k_tcdense.hip): the bitmap layout with every id range narrow
+// enough, unless the caller tunes what only the row kernel has (its queue, a
+// locality order) or asks for the sorted index (whose join rows count each edge once).
+static bool tc_use_dense(const Opts &o, u64 n, const u32 *ib, const std::vector<u32> *blocks) {
+    if (!tc_use_rows(o, n, ib, blocks) || o.join != 0 || o.queue != 0 || o.reorder == 2) return false;
+    u64 wmax = (u64)(ib[1] - ib[0]) + 1;
+    if (blocks) {
+        wmax = 0;
+        for (size_t i = 0; i + 1 < blocks->size(); i++)
+            wmax = std::max<u64>(wmax, (u64)(*blocks)[i + 1] - (*blocks)[i]);
+    }
+    return wmax <= TD_MAX_W;
+}
+
 // The locality order of a plain TC run in the bitmap layout (order.cpp):
 // sigma (device, sigma[old - lo] = new - lo) from the rows, which are
 // downloaded for it, and the renumbered rows.
@@ -309,6 +323,20 @@ void tc_fixpoint(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, Phas
     pack_rows(ctx, d_rows, n, DLG_ORIENT_KV, edge.p);   // e(src, dst) keyed by src
     u32 ib[4];
     id_bounds(ctx, edge.p, n, ib);
+    if (tc_use_dense(o, n, ib, blocks)) {
+        edge.release();
+        J.release();
+        pc.mark(DLG_PH_JOIN);
+        u64 total = 0, raw = 0;
+        std::vector<int> first_empty;
+        out.iterations = tc_dense_run(ctx, d_rows, n, ib[0], ib[1], blocks, o.max_it, out.full, &total, &raw,
+                                      hook ? &first_empty : nullptr);
+        if (hook) hook->on_finished(first_empty);
+        pc.mark(DLG_PH_FINAL);
+        out.raw += (i64)raw;
+        out.nfull = total;
+        return;
+    }
     pc.mark(DLG_PH_HASHTABLE);
     Index ix(ctx);
     auto build_index = [&]() {

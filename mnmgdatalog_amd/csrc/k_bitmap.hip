@@ -335,14 +335,26 @@ __device__ __forceinline__ void load8(const u32 *words, u64 base, u32 *w) {
     w[4] = b.x; w[5] = b.y; w[6] = b.z; w[7] = b.w;
 }
 
+// BW: words per thread -- BE_W, or one for maps too small to give every CU a
+// tile of BE_TILE words.
+template <int BW>
+__device__ __forceinline__ void load_words(const u32 *words, u64 base, u32 (&w)[BW]) {
+    if constexpr (BW == BE_W) load8(words, base, w);
+    else {
+#pragma unroll
+        for (int i = 0; i < BW; i++) w[i] = words[base + i];
+    }
+}
+
+template <int BW = BE_W>
 __global__ __launch_bounds__(BE_T) void bm_count_k(const u32 *words, u64 *bsum) {
     __shared__ u64 sc[BE_T / WAVE + 1];
-    u64 base = (u64)blockIdx.x * BE_TILE + (u64)threadIdx.x * BE_W;
-    u32 w[BE_W];
-    load8(words, base, w);
+    u64 base = (u64)blockIdx.x * (BE_T * BW) + (u64)threadIdx.x * BW;
+    u32 w[BW];
+    load_words<BW>(words, base, w);
     u64 c = 0;
 #pragma unroll
-    for (int i = 0; i < BE_W; i++) c += __popc(w[i]);
+    for (int i = 0; i < BW; i++) c += __popc(w[i]);
     u64 tot;
     block_exclusive_scan<u64>(c, sc, &tot);
     if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
@@ -359,17 +371,22 @@ __global__ __launch_bounds__(BE_T) void bm_count_k(const u32 *words, u64 *bsum) 
 // MULTI: the words are several maps, each starting at a whole tile: map m
 // covers tiles [mt[m], mt[m + 1]) with ids from mlo[m] and mwpr[m] words per
 // row (nm maps); each workgroup finds its tile's map by a binary search.
+// gate: nothing is written unless *gate (the set bits counted) is `expect`.
 constexpr int BE_STAGE = 4096;
-template <bool SWAP, bool CLEAR, bool MULTI = false>
+template <bool SWAP, bool CLEAR, bool MULTI = false, int BW = BE_W>
 __global__ __launch_bounds__(BE_T) void bm_emit_k(u32 *words, const u64 *bpre, u32 lo, u64 wpr, u64 *out,
                                                   const u64 *mt = nullptr, const u32 *mlo = nullptr,
-                                                  const u64 *mwpr = nullptr, u32 nm = 0) {
+                                                  const u64 *mwpr = nullptr, u32 nm = 0,
+                                                  const u64 *gate = nullptr, u64 expect = 0) {
+    constexpr int BE_TILE = BE_T * BW;   // this variant's tile
+    static_assert(!CLEAR || BW == BE_W, "clearing goes by eight words");
+    if (gate && *gate != expect) return;
     __shared__ u64 sc[BE_T / WAVE + 1];
     __shared__ u64 s_buf[BE_STAGE];   // the stage, or the dense walk's three word tables
     static_assert(3 * BE_TILE * 4 <= BE_STAGE * 8, "word tables must fit the stage");
     u32 *s_w = (u32 *)s_buf, *s_pos = s_w + BE_TILE, *s_row = s_pos + BE_TILE;
     const u64 tile = (u64)blockIdx.x * BE_TILE;
-    const u64 base = tile + (u64)threadIdx.x * BE_W;
+    const u64 base = tile + (u64)threadIdx.x * BW;
     u64 mbase = 0;   // the tile's map's first word
     if (MULTI) {
         u32 a = 0, b = nm;   // the last map starting at or before this tile
@@ -382,11 +399,11 @@ __global__ __launch_bounds__(BE_T) void bm_emit_k(u32 *words, const u64 *bpre, u
         wpr = mwpr[a];
     }
     const u64 rtile = tile - mbase, rbase = base - mbase;   // word indexes within the map
-    u32 w[BE_W];
-    load8(words, base, w);
+    u32 w[BW];
+    load_words<BW>(words, base, w);
     u64 c = 0;
 #pragma unroll
-    for (int i = 0; i < BE_W; i++) c += __popc(w[i]);
+    for (int i = 0; i < BW; i++) c += __popc(w[i]);
     u64 tot;
     const u64 rel = block_exclusive_scan<u64>(c, sc, &tot);   // this thread's first output in the tile
     const u64 out0 = bpre[blockIdx.x];
@@ -395,14 +412,14 @@ __global__ __launch_bounds__(BE_T) void bm_emit_k(u32 *words, const u64 *bpre, u
         *(uint4 *)(words + base + 4) = make_uint4(0u, 0u, 0u, 0u);
     }
     if (tot == 0) return;
-    if (tot <= (u64)(2 * BE_STAGE)) {   // uniform: staged, one or two rounds
+    if (tot <= (u64)(BW == BE_W ? 2 * BE_STAGE : BE_STAGE)) {   // uniform: staged, one or two rounds
         const u64 k0 = rbase / wpr, cw0 = rbase - k0 * wpr;
         for (u64 r0 = 0; r0 < tot; r0 += BE_STAGE) {
             const u64 r1 = r0 + BE_STAGE < tot ? r0 + BE_STAGE : tot;
             if (c && rel < r1 && rel + c > r0) {
                 u64 p = rel, k = k0, cw = cw0;
 #pragma unroll
-                for (int i = 0; i < BE_W; i++) {
+                for (int i = 0; i < BW; i++) {
                     u32 x = w[i];
                     const u32 c0 = (u32)(cw * 32);
                     while (x) {
@@ -428,10 +445,10 @@ __global__ __launch_bounds__(BE_T) void bm_emit_k(u32 *words, const u64 *bpre, u
         u64 pos = rel;
         u64 k = rbase / wpr, cw = rbase - k * wpr;   // one division per thread; the words are consecutive
 #pragma unroll
-        for (int i = 0; i < BE_W; i++) {
-            s_w[threadIdx.x * BE_W + i] = w[i];
-            s_pos[threadIdx.x * BE_W + i] = (u32)pos;
-            s_row[threadIdx.x * BE_W + i] = (u32)k;
+        for (int i = 0; i < BW; i++) {
+            s_w[threadIdx.x * BW + i] = w[i];
+            s_pos[threadIdx.x * BW + i] = (u32)pos;
+            s_row[threadIdx.x * BW + i] = (u32)k;
             pos += __popc(w[i]);
             if (++cw == wpr) {
                 cw = 0;
@@ -572,7 +589,7 @@ static u64 words_count(dlg_ctx *ctx, const u32 *words, u64 nwords, DBuf<u64> &bs
     nb = (nwords + BE_TILE - 1) / BE_TILE;
     bsum.ensure(nb);
     DBuf<u64> tot(ctx, 1);
-    DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * nb * BE_TILE, bm_count_k, (unsigned)nb, BE_T, 0, words, bsum.p);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * nb * BE_TILE, bm_count_k<BE_W>, (unsigned)nb, BE_T, 0, words, bsum.p);
     scan_blocks(ctx, bsum.p, nb, tot.p);
     u64 h = 0;
     ctx->read_scalars(tot.p, 1, &h);
@@ -1395,7 +1412,7 @@ u64 bitmap_emit_maps(dlg_ctx *ctx, const u32 *words, const std::vector<MapRef> &
     DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * tails, bm_zero_tails_k, std::min<u32>(nm, 4096u), 256, 0, sc.p,
                (const u64 *)d_db, (const u64 *)d_nw, nm);
     DBuf<u64> bsum(ctx, t), tot(ctx, 1);
-    DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * t * BE_TILE, bm_count_k, (unsigned)t, BE_T, 0, (const u32 *)sc.p, bsum.p);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * t * BE_TILE, bm_count_k<BE_W>, (unsigned)t, BE_T, 0, (const u32 *)sc.p, bsum.p);
     scan_blocks(ctx, bsum.p, t, tot.p);
     u64 total = 0;
     ctx->read_scalars(tot.p, 1, &total);
@@ -1405,6 +1422,53 @@ u64 bitmap_emit_maps(dlg_ctx *ctx, const u32 *words, const std::vector<MapRef> &
                    BE_T, 0, sc.p, (const u64 *)bsum.p, 0u, (u64)1, out, (const u64 *)d_mt, (const u32 *)d_lo,
                    (const u64 *)d_wpr, nm);
     return total;
+}
+
+u64 emit_tile_words(u64 nwords) { return (nwords + BE_TILE - 1) / BE_TILE * BE_TILE; }
+
+// Maps too small to give every CU a tile of BE_TILE words go by tiles of BE_T
+// words: TC of 437 ids (3 large tiles) 31 us of emission by large tiles.
+template <int BW>
+static void emit_tiled(dlg_ctx *ctx, u32 *words, const std::vector<MapRef> &maps, u64 nwords, u64 *out, u64 expect) {
+    constexpr u64 tile = (u64)BE_T * BW;
+    const u64 nt = nwords / tile;
+    const u32 nm = (u32)maps.size();
+    DBuf<u64> bsum(ctx, nt), tot(ctx, 1), tab(ctx);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * nwords, bm_count_k<BW>, (unsigned)nt, BE_T, 0, (const u32 *)words, bsum.p);
+    scan_blocks(ctx, bsum.p, nt, tot.p);
+    const double bytes = 4.0 * nwords + 8.0 * expect;
+    std::vector<u64> h;
+    if (nm == 1) {
+        DLG_LAUNCH(ctx, DLG_K_MISC, bytes, (bm_emit_k<false, false, false, BW>), (unsigned)nt, BE_T, 0, words,
+                   (const u64 *)bsum.p, maps[0].lo, maps[0].wpr, out, (const u64 *)nullptr, (const u32 *)nullptr,
+                   (const u64 *)nullptr, 0u, (const u64 *)tot.p, expect);
+    } else {
+        const size_t L = nm + 1;   // each map's first tile, its words per row and (u32) its first id
+        h.assign(2 * L + (L + 1) / 2, 0);
+        u32 *hlo = (u32 *)(h.data() + 2 * L);
+        for (u32 m = 0; m < nm; m++) {
+            h[m] = maps[m].base / tile;
+            h[L + m] = maps[m].wpr;
+            hlo[m] = maps[m].lo;
+        }
+        h[nm] = nt;
+        tab.ensure(h.size());
+        HIPCHK(hipMemcpyAsync(tab.p, h.data(), 8 * h.size(), hipMemcpyHostToDevice, ctx->stream));
+        DLG_LAUNCH(ctx, DLG_K_MISC, bytes, (bm_emit_k<false, false, true, BW>), (unsigned)nt, BE_T, 0, words,
+                   (const u64 *)bsum.p, 0u, (u64)1, out, (const u64 *)tab.p, (const u32 *)(tab.p + 2 * L),
+                   (const u64 *)(tab.p + L), nm, (const u64 *)tot.p, expect);
+    }
+    u64 total = 0;
+    ctx->read_scalars(tot.p, 1, &total);
+    if (total != expect) fail(DLG_DEVICE_ERROR, "bitmap emission count mismatch");
+}
+
+void bitmap_emit_tiled(dlg_ctx *ctx, u32 *words, const std::vector<MapRef> &maps, u64 nwords, DBuf<u64> &out,
+                       u64 expect) {
+    out.ensure(expect ? expect : 1);
+    if (nwords == 0) return;
+    if (nwords < (u64)ctx->num_cus * BE_TILE) emit_tiled<1>(ctx, words, maps, nwords, out.p, expect);
+    else emit_tiled<BE_W>(ctx, words, maps, nwords, out.p, expect);
 }
 
 }  // namespace dlg

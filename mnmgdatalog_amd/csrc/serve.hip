@@ -80,7 +80,8 @@ double now_s(const dlg_server *s) { return secs(s->t0, Clock::now()); }
 // Predicted peak device bytes of one request, by the layout its run will
 // use.  TC and SG keep the full relation as a bitmap when the id range W is
 // at most BITMAP_MAX_W wide: F and its transposed copy for the read-out,
-// W * ceil(W / 32) words each (SG: F, the round's maps D and R), plus the
+// W * ceil(W / 32) words each (SG: F, the round's maps D and R; TC by row ORs
+// has three maps, at most 32 MiB more, which the slack covers), plus the
 // sorted output and the round buffers, about 32 B per output tuple, plus
 // the edge index.  Wider ranges keep F as sorted tuples with a hash set and
 // a final sort: about 48 B per output tuple.  The output is |TC| by SCC

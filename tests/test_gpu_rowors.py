@@ -1,0 +1,86 @@
+"""TC by row ORs (id ranges up to 2^14 ids): the relation, round count and join rows at the edges of its
+words, chunks, tasks and long-list rows, against the oracle and the row kernel (which `queue` selects)."""
+import numpy as np
+import pytest
+
+import mnmgdatalog_amd as dlg
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = dlg.Ctx(0)
+    yield c
+    c.close()
+
+
+def same(a, b):
+    assert (a["iterations"], a["output_size"]) == (b["iterations"], b["output_size"])
+    assert np.array_equal(a["rows"], b["rows"])
+
+
+def graph(width, edges, seed, hub=0):
+    """`edges` random edges over exactly `width` ids (both ends used), duplicates and self-loops among
+    them, the last `hub` ids all pointing at id 3."""
+    rng = np.random.default_rng(seed)
+    r = rng.integers(0, width, size=(edges, 2))
+    r = np.concatenate([r, r[:5], [[0, width - 1], [7 % width, 7 % width]]])
+    if hub:
+        r = np.concatenate([r, np.stack([np.arange(width - hub, width), np.full(hub, 3)], 1)])
+    return (r + rng.integers(-2**30, 2**30)).astype(np.int32)
+
+
+# words (32), uint4s (128), chunks (2,048) and their remainders; one task to thousands
+@pytest.mark.parametrize("width,edges", [(1, 1), (2, 3), (31, 40), (32, 40), (33, 50), (127, 160), (128, 160), (129, 200),
+                                         (2047, 2300), (2048, 2300), (2049, 2300), (4097, 4300)])
+def test_widths(ctx, orc, width, edges):
+    rows = graph(width, edges, width)
+    got = ctx.run("tc", rows)
+    same(got, orc.tc(rows))
+    assert got["raw_join_rows"] == ctx.run("tc", rows, queue=1)["raw_join_rows"]
+
+
+# the widest range taken, and the first one that is not; several chunks a row, sparse
+@pytest.mark.parametrize("width", [16383, 16384, 16385])
+def test_widest(ctx, orc, width):
+    rows = graph(width, 9000, width)
+    got = ctx.run("tc", rows)
+    same(got, orc.tc(rows))
+    assert got["raw_join_rows"] == ctx.run("tc", rows, queue=1)["raw_join_rows"]
+
+
+# 255 to 257 and thousands of predecessors: a sub-group's row, then a workgroup's
+@pytest.mark.parametrize("hub", [250, 256, 257, 300, 2500])
+def test_long_lists(ctx, orc, hub):
+    rows = graph(3000, 3500, hub, hub=hub)
+    got = ctx.run("tc", rows)
+    same(got, orc.tc(rows))
+    assert got["raw_join_rows"] == ctx.run("tc", rows, queue=1)["raw_join_rows"]
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 9])
+def test_truncated(ctx, orc, k):
+    rows = graph(700, 760, 11)
+    got, want = ctx.run("tc", rows, max_iterations=k), orc.tc(rows, max_iterations=k)
+    same(got, want)
+    assert got["raw_join_rows"] == ctx.run("tc", rows, queue=1, max_iterations=k)["raw_join_rows"]
+
+
+def test_many_rounds(ctx, orc):
+    rows = np.stack([np.arange(300), np.arange(1, 301)], 1).astype(np.int32)
+    got = ctx.run("tc", rows)
+    same(got, orc.tc(rows))
+    assert got["iterations"] == 300
+
+
+def test_batch_of_mixed_widths(ctx, orc):
+    """One id to several chunks a row, long lists, empty and single-edge instances side by side: each
+    as its plain run, with and without a round limit."""
+    inst = [graph(w, w + w // 8 + 1, w, hub=h) for w, h in ((1, 0), (33, 0), (640, 400), (129, 0), (2600, 0), (5000, 300))]
+    inst.insert(2, np.zeros((0, 2), np.int32))
+    inst.append(np.array([[5, 6]], np.int32))
+    for kw in ({}, {"max_iterations": 3}):
+        res, _ = ctx.batch_run("tc", inst, **kw)
+        for r, rows in zip(res, inst):
+            same(r, orc.tc(rows, **kw))
