@@ -84,3 +84,19 @@ def test_batch_of_mixed_widths(ctx, orc):
         res, _ = ctx.batch_run("tc", inst, **kw)
         for r, rows in zip(res, inst):
             same(r, orc.tc(rows, **kw))
+
+
+@pytest.mark.parametrize("prog", ["tc", "wcc"])
+def test_batch_digest_segments(ctx, prog):
+    """Instances of one tuple to several of the digest's segments of 2^15 tuples, and empty ones
+    between them: each instance's digest is its plain run's."""
+    sizes = [1, 0, 181, 182, 2, 0, 0, 300, 33] if prog == "tc" else [1, 40_000, 0, 2, 70_000]
+    inst = []
+    for i, w in enumerate(sizes):   # a cycle of w ids: w * w tuples; w self-loops: w components
+        k = np.arange(w)
+        inst.append((np.stack([k, (k + 1) % max(w, 1) if prog == "tc" else k], 1) + 100 * i).astype(np.int32))
+    res, _ = ctx.batch_run(prog, inst, keep_output=False, check_output=1)
+    for r, rows in zip(res, inst):
+        p = ctx.run(prog, rows, keep_output=False, check_output=1)
+        assert (r["output_size"], r["output_sum"]) == (p["output_size"], p["output_sum"])
+        assert r["output_order_breaks"] == p["output_order_breaks"] == 0
