@@ -377,12 +377,6 @@ struct RunSet {
 };
 // Unique elements of sorted `in` that no run of `rs` contains.
 u64 select_unique_not_in_runs(dlg_ctx *ctx, const u64 *in, u64 n, const RunSet &rs, u64 *out);
-// Second half of a compaction whose count kernel (tiles of 2048, flags as
-// ballot words, per-tile counts in bsum) already ran: scan, read the total
-// back, scatter.  Returns the kept count.
-u64 select_scatter(dlg_ctx *ctx, const u64 *in, u64 n, const u64 *flags, DBuf<u64> &bsum, DBuf<u64> &tot,
-                   u64 *out);
-
 // Exclusive scan of bsum[0..nb) in place by one block; the total to *d_total.
 void scan_blocks(dlg_ctx *ctx, u64 *bsum, u64 nb, u64 *d_total);
 
@@ -578,8 +572,21 @@ struct HashSet {
 void hashset_reserve(dlg_ctx *ctx, HashSet &hs, u64 need, double lf, const u64 *all, u64 n_all);
 // Insert tuples that are absent and pairwise distinct.
 void hashset_insert(dlg_ctx *ctx, HashSet &hs, const u64 *x, u64 n);
-// First of each equal run of sorted `in` that the set does not contain.
-u64 select_unique_not_in_hash(dlg_ctx *ctx, const u64 *in, u64 n, const HashSet &hs, u64 *out);
+// A relation as an append-only array (arrival order, n tuples) and the hash
+// set of them; the set takes up to `limit` tuples before both grow.
+struct HashRel {
+    DBuf<u64> all, count;
+    HashSet hs;
+    u64 n = 0, limit = 0;
+    double lf;
+    HashRel(dlg_ctx *c, double load_factor) : all(c), count(c), hs(c), lf(load_factor) {}
+};
+// The tuples of x (any order, duplicates allowed) that are absent, appended.  Returns their number.
+u64 hashrel_insert_list(dlg_ctx *ctx, HashRel &r, const u64 *x, u64 n);
+// The same for the rows of probe ⋈ index (probe null: the relation's own
+// tuples [off, off + n)); nodiag drops rows with key == value.  *raw += |probe ⋈ index|.
+u64 hashrel_insert_join(dlg_ctx *ctx, HashRel &r, const Index &ix, const u64 *probe, u64 off, u64 n, int proj,
+                        bool nodiag, JoinScratch &js, u64 *raw);
 // Merge of sorted a, b into out (a first on ties).
 void merge(dlg_ctx *ctx, const u64 *a, u64 na, const u64 *b, u64 nb, u64 *out);
 // The merge with one copy of each value kept (inputs sorted, duplicates
@@ -628,6 +635,8 @@ struct JoinScratch {
     explicit JoinScratch(dlg_ctx *c) : cnt(c), pstart(c), offs(c) {}
 };
 u64 join_count(dlg_ctx *ctx, const Index &ix, const u64 *probe, u64 n, JoinScratch &js);
+// Same without reading |J| back: it is left at js.offs[n] (n and ix.n not 0).
+void join_count_async(dlg_ctx *ctx, const Index &ix, const u64 *probe, u64 n, JoinScratch &js);
 void join_expand(dlg_ctx *ctx, const Index &ix, const u64 *probe, u64 n, const JoinScratch &js,
                  u64 total, int proj, u64 *out);
 // The same two phases over caller-provided scratch (no allocation): cnt and

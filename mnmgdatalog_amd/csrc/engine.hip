@@ -123,31 +123,23 @@ void check_rows_arg(int64_t n, const void *rows) {
     if ((u64)n >= 0x7fffffffull) fail(DLG_OVERFLOW, "more than 2^31-2 input rows");
 }
 
-// The full relation F, three layouts with identical results:
+// The full relation F as sorted arrays, two layouts with identical results:
 //  1  one sorted array; every round's new tuples are merged into it (the
 //     reference's scheme, tc.cu:268-286): each round rewrites all of F.
 //  2  sorted, disjoint runs whose sizes fall geometrically from the oldest to
 //     the newest; a round's new tuples become the newest run and runs of
 //     similar size are merged (a binary counter), so each tuple is rewritten
 //     O(log rounds) times; N = unique(J) \ F searches every run.
-//  3  an append-only array plus a device hash set of F: membership costs one
-//     or two slot reads however large F is, and F is sorted once at the end.
+// (Layout 3, the default for wide id ranges, is a HashRel: every join row
+// goes into a hash set as it is formed, and F is sorted once at the end.)
 // collapse() leaves the whole relation sorted in one array.
 struct FullRel {
     dlg_ctx *ctx;
-    int mode;                       // 1 one array, 2 tiered runs, 3 append + hash set
+    int mode;                       // 1 one array, 2 tiered runs
     std::vector<DBuf<u64>> runs;
     std::vector<u64> sizes;
     u64 total = 0;
-    // mode 3: every tuple of F in arrival order, and a hash set of them
-    DBuf<u64> all;
-    HashSet hs;
-    double lf;
-    int bits;
-    const u32 *bounds;
-    FullRel(dlg_ctx *c, const Opts &o, const u32 *b)
-        : ctx(c), mode(o.strategy == 1 ? 1 : (o.strategy == 2 ? 2 : 3)), all(c), hs(c), lf(o.lf),
-          bits(o.bits), bounds(b) {}
+    FullRel(dlg_ctx *c, const Opts &o) : ctx(c), mode(o.strategy == 1 ? 1 : 2) {}
 
     void merge_last_two() {
         size_t k = runs.size();
@@ -162,19 +154,6 @@ struct FullRel {
     // Takes buf[0..n) (sorted, disjoint from F); buf is left empty.
     void add(DBuf<u64> &buf, u64 n) {
         if (n == 0) return;
-        if (mode == 3) {
-            if (all.cap < total + n) {                       // grow x2, keep the contents
-                DBuf<u64> g(ctx, std::max<u64>(2 * (total + n), 1024));
-                copy_u64(ctx, g.p, all.p, total);
-                all = std::move(g);
-            }
-            copy_u64(ctx, all.p + total, buf.p, n);
-            hashset_reserve(ctx, hs, total + n, lf, all.p, total);
-            hashset_insert(ctx, hs, buf.p, n);
-            total += n;
-            buf.release();
-            return;
-        }
         total += n;
         runs.push_back(std::move(buf));
         sizes.push_back(n);
@@ -189,7 +168,6 @@ struct FullRel {
     }
     // N = first of each run of equal tuples in sorted J, minus F.
     u64 new_tuples(const u64 *J, u64 nj, u64 *N) {
-        if (mode == 3) return select_unique_not_in_hash(ctx, J, nj, hs, N);
         if (runs.size() == 1) return select(ctx, SEL_UNIQUE_NOT_IN, J, nj, runs[0].p, sizes[0], N);
         RunSet rs;
         rs.k = (int)runs.size();
@@ -201,14 +179,6 @@ struct FullRel {
     }
     // The whole relation, sorted, moved into `out`.
     void collapse(DBuf<u64> &out) {
-        if (mode == 3) {
-            hs.slots.release();
-            DBuf<u64> tmp(ctx);
-            if (total) radix_sort(ctx, all, total, tmp, bits, bounds);
-            if (!all.p) all.ensure(1);
-            out = std::move(all);
-            return;
-        }
         while (runs.size() >= 2) merge_last_two();
         if (runs.empty()) {
             out.ensure(1);
@@ -219,6 +189,17 @@ struct FullRel {
         }
     }
 };
+
+static bool use_hash_rel(const Opts &o) { return o.strategy != 1 && o.strategy != 2; }
+
+// A HashRel's tuples, sorted, moved into `out` (its table is given back first).
+static void hashrel_collapse(dlg_ctx *ctx, HashRel &r, int bits, const u32 *bounds, DBuf<u64> &out) {
+    r.hs.slots.release();
+    DBuf<u64> tmp(ctx);
+    if (r.n) radix_sort(ctx, r.all, r.n, tmp, bits, bounds);
+    if (!r.all.p) r.all.ensure(1);
+    out = std::move(r.all);
+}
 
 // Every tuple of a TC / SG fixpoint pairs two node ids of the input, so the
 // id range of the edge relation bounds both halves of every tuple; the radix
@@ -409,9 +390,34 @@ void tc_fixpoint(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, Phas
         out.iterations = it;
         return;
     }
+    if (use_hash_rel(o)) {
+        // N = the join rows that claim a slot, appended after Δ: Δ, N and F
+        // share one array, and a round is a count, a scan and an insertion
+        HashRel F(ctx, o.lf);
+        pc.mark(DLG_PH_DEDUP);
+        u64 beg = 0, nd = hashrel_insert_list(ctx, F, J.p, n);   // F = Δ0
+        J.release();
+        pc.mark(DLG_PH_JOIN);
+        while (true) {
+            u64 raw = 0;
+            const u64 nn = hashrel_insert_join(ctx, F, ix, nullptr, beg, nd, DLG_PROJ_HV_PV, false, js, &raw);   // (z, x)
+            out.raw += (i64)raw;
+            it++;
+            if (hook) hook->on_round(ctx, F.all.p + beg + nd, nn, it, false);
+            if (nn == 0) break;                         // |F| unchanged (tc.cu:294-300)
+            beg += nd;
+            nd = nn;
+            if (o.max_it > 0 && it >= o.max_it) break;
+        }
+        pc.mark(DLG_PH_MERGE);
+        out.nfull = F.n;
+        hashrel_collapse(ctx, F, o.bits, ib, out.full);
+        out.iterations = it;
+        return;
+    }
     pc.mark(DLG_PH_DEDUP);
     u64 nd = sort_unique_into(ctx, J, n, tmp, delta, SEL_UNIQUE, nullptr, 0, o.bits, ib);
-    FullRel F(ctx, o, ib);                              // F = Δ0, added after the first join
+    FullRel F(ctx, o);                                  // F = Δ0, added after the first join
     while (true) {
         pc.mark(DLG_PH_JOIN);
         u64 nj = join_into(ctx, ix, delta.p, nd, DLG_PROJ_HV_PV, js, J);   // (z, x)
@@ -487,13 +493,41 @@ void sg_fixpoint(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, Phas
         out.iterations = it;
         return;
     }
+    if (use_hash_rel(o)) {
+        HashRel F(ctx, o.lf);
+        pc.mark(DLG_PH_JOIN);
+        u64 raw = 0;
+        u64 beg = 0, nd = hashrel_insert_join(ctx, F, ix, edge.p, 0, ne, DLG_PROJ_HV_PV, true, js, &raw);   // base (y, x)
+        edge.release();
+        while (true) {
+            pc.mark(DLG_PH_JOIN);
+            const u64 n1 = join_into(ctx, ix, F.all.p + beg, nd, DLG_PROJ_PV_HV, js, J);   // (b, x)
+            raw += n1;
+            pc.mark(DLG_PH_DEDUP);
+            const u64 nt = sort_unique_into(ctx, J, n1, tmp, T, SEL_UNIQUE, nullptr, 0, o.bits, ib);
+            pc.mark(DLG_PH_JOIN);
+            const u64 nn = hashrel_insert_join(ctx, F, ix, T.p, 0, nt, DLG_PROJ_PV_HV, false, js, &raw);   // (x, y)
+            it++;
+            if (hook) hook->on_round(ctx, F.all.p + beg + nd, nn, it, false);
+            if (nn == 0) break;                     // sg.cu:376-389
+            beg += nd;
+            nd = nn;
+            if (o.max_it > 0 && it >= o.max_it) break;
+        }
+        pc.mark(DLG_PH_MERGE);
+        out.raw += (i64)raw;
+        out.nfull = F.n;
+        hashrel_collapse(ctx, F, o.bits, ib, out.full);
+        out.iterations = it;
+        return;
+    }
     pc.mark(DLG_PH_JOIN);
     u64 nb = join_into(ctx, ix, edge.p, ne, DLG_PROJ_HV_PV, js, J);   // (y, x)
     out.raw += (i64)nb;
     edge.release();
     pc.mark(DLG_PH_DEDUP);
     u64 nd = sort_unique_into(ctx, J, nb, tmp, delta, SEL_UNIQUE_NODIAG, nullptr, 0, o.bits, ib);
-    FullRel F(ctx, o, ib);                              // F = base, added after the first join
+    FullRel F(ctx, o);                                  // F = base, added after the first join
     while (true) {
         pc.mark(DLG_PH_JOIN);
         u64 n1 = join_into(ctx, ix, delta.p, nd, DLG_PROJ_PV_HV, js, J);  // (b, x)

@@ -193,13 +193,20 @@ static void join_count_launch(dlg_ctx *ctx, const Index &ix, const u64 *probe, u
     }
 }
 
-u64 join_count(dlg_ctx *ctx, const Index &ix, const u64 *probe, u64 n, JoinScratch &js) {
-    if (n == 0 || ix.n == 0) return 0;
+void join_count_async(dlg_ctx *ctx, const Index &ix, const u64 *probe, u64 n, JoinScratch &js) {
     js.cnt.ensure(n);
     js.pstart.ensure(n);
     js.offs.ensure(n + 1);
     join_count_launch(ctx, ix, probe, n, js.cnt.p, js.pstart.p);
-    return scan_u32_u64(ctx, js.cnt.p, n, js.offs.p);
+    scan_u32_u64_async(ctx, js.cnt.p, n, js.offs.p, js.offs.p + n);
+}
+
+u64 join_count(dlg_ctx *ctx, const Index &ix, const u64 *probe, u64 n, JoinScratch &js) {
+    if (n == 0 || ix.n == 0) return 0;
+    join_count_async(ctx, ix, probe, n, js);
+    u64 h = 0;
+    ctx->read_scalars(js.offs.p + n, 1, &h);
+    return h;
 }
 
 u64 join_count_with(dlg_ctx *ctx, const Index &ix, const u64 *probe, u64 n, u32 *cnt, u32 *pstart, u64 *offs,

@@ -233,9 +233,38 @@ u64 scan_partials(u64 n) {
     return nb ? nb : 1;
 }
 
-// The three launches of a scan over caller-provided partials (scan_partials(n) u64s).
+// A whole scan by one workgroup, for inputs of up to SCAN_SMALL elements:
+// one launch of about 3 us instead of three.
+constexpr int SCAN_SMALL_T = 1024;
+constexpr u64 SCAN_SMALL = (u64)SCAN_SMALL_T * SCAN_I;
+template <typename T>
+__global__ __launch_bounds__(SCAN_SMALL_T) void scan_small_k(const T *in, u64 n, u64 *out, u64 *d_total) {
+    __shared__ u64 sc[SCAN_SMALL_T / WAVE + 1];
+    const u64 base = (u64)threadIdx.x * SCAN_I;
+    T v[SCAN_I];
+    u64 s = 0;
+#pragma unroll
+    for (int i = 0; i < SCAN_I; i++) {
+        v[i] = base + i < n ? in[base + i] : 0;
+        s += v[i];
+    }
+    u64 tot;
+    u64 ex = block_exclusive_scan<u64>(s, sc, &tot);   // every read is done before the first write: out may alias in
+#pragma unroll
+    for (int i = 0; i < SCAN_I; i++) {
+        if (base + i < n) out[base + i] = ex;
+        ex += v[i];
+    }
+    if (threadIdx.x == 0 && d_total) *d_total = tot;
+}
+
+// The launches of a scan over caller-provided partials (scan_partials(n) u64s).
 template <typename T>
 static void scan_to_u64_with(dlg_ctx *ctx, const T *in, u64 n, u64 *out, u64 *bsum, u64 *d_total) {
+    if (n <= SCAN_SMALL) {
+        DLG_LAUNCH(ctx, DLG_K_SCAN, (sizeof(T) + 8.0) * n, scan_small_k<T>, 1, SCAN_SMALL_T, 0, in, n, out, d_total);
+        return;
+    }
     const u64 nb = scan_partials(n);
     DLG_LAUNCH(ctx, DLG_K_SCAN, (double)sizeof(T) * n + 8.0 * nb, scan_reduce_k<T>, (unsigned)nb, SCAN_T, 0,
                in, n, bsum);
@@ -1082,18 +1111,6 @@ __global__ __launch_bounds__(SEL_T) void select_count_runs_k(const u64 *in, u64 
     u64 tot;
     block_exclusive_scan<u64>(c, sc, &tot);
     if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
-}
-
-u64 select_scatter(dlg_ctx *ctx, const u64 *in, u64 n, const u64 *flags, DBuf<u64> &bsum, DBuf<u64> &tot,
-                   u64 *out) {
-    u64 nb = (n + SEL_TILE - 1) / SEL_TILE;
-    scan_blocks(ctx, bsum.p, nb, tot.p);
-    u64 total = 0;
-    ctx->read_scalars(tot.p, 1, &total);
-    if (total == 0) return 0;
-    DLG_LAUNCH(ctx, DLG_K_SELECT, 8.0 * ((n + 63) / 64) + 16.0 * total, select_scatter_k<false>,
-               (unsigned)nb, SEL_T, 0, in, n, flags, (const u64 *)bsum.p, (void *)out);
-    return total;
 }
 
 u64 select_unique_not_in_runs(dlg_ctx *ctx, const u64 *in, u64 n, const RunSet &rs, u64 *out) {

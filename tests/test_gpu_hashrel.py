@@ -1,0 +1,61 @@
+"""TC and SG over wide id ranges: join rows inserted into the hash set as they are formed, against the
+oracle and the sorted-run layout (strategy 2)."""
+import numpy as np
+import pytest
+
+import mnmgdatalog_amd as dlg
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = dlg.Ctx(0)
+    yield c
+    c.close()
+
+
+def same(a, b):
+    assert (a["iterations"], a["output_size"]) == (b["iterations"], b["output_size"])
+    assert np.array_equal(a["rows"], b["rows"])
+
+
+# tiles of 256 rows and their remainders; the tuple that equals the empty slot marker (INT32_MAX twice)
+@pytest.mark.parametrize("prog", ["tc", "sg"])
+@pytest.mark.parametrize("edges", [1, 255, 256, 257, 3000])
+@pytest.mark.parametrize("lf", [0.0, 0.1, 0.95])
+def test_small(ctx, orc, prog, edges, lf):
+    rng = np.random.default_rng(edges)
+    rows = (rng.integers(0, max(2, edges), size=(edges, 2)) * 100_003).astype(np.int32)
+    rows = np.concatenate([rows, rows[:3], [[2**31 - 1, 2**31 - 1], [5, 2**31 - 1]]]).astype(np.int32)
+    kw = {"load_factor": lf} if lf else {}
+    got = ctx.run(prog, rows, **kw)
+    same(got, getattr(orc, prog)(rows))
+    assert got["raw_join_rows"] == ctx.run(prog, rows, strategy=2)["raw_join_rows"]
+
+
+# far more join rows than new tuples (the rows past the set's room wait for it to grow), hubs
+@pytest.mark.parametrize("prog", ["tc", "sg"])
+def test_many_duplicates(ctx, orc, prog):
+    rng = np.random.default_rng(3)
+    rows = rng.integers(0, 120, size=(3000, 2))
+    rows = np.concatenate([rows, [[0, 1_000_000]]]).astype(np.int32)
+    rows[:-1] *= 3001
+    got = ctx.run(prog, rows, strategy=3)
+    same(got, getattr(orc, prog)(rows))
+    assert got["raw_join_rows"] == ctx.run(prog, rows, strategy=2)["raw_join_rows"]
+
+
+@pytest.mark.parametrize("k", [1, 2, 4])
+def test_truncated(ctx, orc, k):
+    rows = (np.random.default_rng(8).integers(0, 500, size=(520, 2)) * 4096).astype(np.int32)
+    same(ctx.run("tc", rows, max_iterations=k), orc.tc(rows, max_iterations=k))
+    same(ctx.run("sg", rows, max_iterations=k), orc.sg(rows, max_iterations=k))
+
+
+def test_large_rounds(ctx):
+    """Rounds of more than 2^19 probes (tiles of 2,048 rows), against the sorted-run layout."""
+    rows = dlg.gen_erdos_renyi(900_000, 800_000, 4)
+    got, want = ctx.run("tc", rows), ctx.run("tc", rows, strategy=2)
+    same(got, want)
+    assert got["raw_join_rows"] == want["raw_join_rows"]
