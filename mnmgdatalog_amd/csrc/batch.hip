@@ -447,6 +447,64 @@ static void split_rows(dlg_ctx *ctx, const u64 *d, const std::vector<u64> &b, co
     ctx->sync();
 }
 
+// The rounds of a batch's WCC union, pushed from the frontier: per round the
+// frontier is counted by instance, and an instance whose rule fires drops out
+// of it.  (Graphs too large for whole-graph pulls, and the other round forms.)
+static void wcc_batch_rounds(dlg_ctx *ctx, WccState &s, const WccGraph &g, const Opts &o, PhaseClock &pc,
+                             const u32 *vstart, const std::vector<u32> &hv, std::vector<int> &iters, int &rounds) {
+    const u64 V = g.V;
+    const int B = (int)hv.size() - 1;
+    wcc_setup(ctx, s, V);
+    DBuf<u32> cnt(ctx, B), live(ctx, B);
+    std::vector<i64> prev(B), cur(B);
+    std::vector<char> done(B, 0);
+    std::vector<u32> hlive(B, 1);
+    for (int i = 0; i < B; i++) prev[i] = (i64)(hv[i + 1] - hv[i]);   // wcc.cu:236-242
+    int live_n = B;
+    u64 nf = V;
+    DBuf<u32> tnode(ctx, V ? V : 1), tlabel(ctx, V ? V : 1);
+    std::vector<u32> hc(B);
+    while (live_n > 0) {
+        pc.mark(DLG_PH_JOIN);
+        rounds++;
+        u64 nn = nf ? wcc_round(ctx, s, g.ix, g.nbr.p, nf, (u32)rounds) : 0;
+        fill_u32(ctx, cnt.p, B, 0u);
+        if (nn)
+            DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * nn, frontier_hist_k, sgrid(ctx, nn), ctx->block_size, 0,
+                       (const u32 *)s.fnode.p, nn, (const u32 *)vstart, (u32)B, cnt.p);
+        HIPCHK(hipMemcpyAsync(hc.data(), cnt.p, 4 * B, hipMemcpyDeviceToHost, ctx->stream));
+        ctx->sync();
+        bool froze = false;
+        for (int i = 0; i < B; i++) {
+            if (done[i]) continue;
+            iters[i]++;
+            cur[i] = hc[i];
+            if (cur[i] == prev[i]) {                  // wcc.cu:366-383, per instance
+                done[i] = 1;
+                hlive[i] = 0;
+                live_n--;
+                froze = froze || hc[i] > 0;
+            } else {
+                prev[i] = cur[i];
+            }
+        }
+        nf = nn;
+        if (froze && nf) {
+            HIPCHK(hipMemcpyAsync(live.p, hlive.data(), 4 * B, hipMemcpyHostToDevice, ctx->stream));
+            fill_u32(ctx, s.counter.p, 1, 0u);
+            DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * nf, frontier_filter_k, sgrid(ctx, nf), ctx->block_size, 0,
+                       (const u32 *)s.fnode.p, (const u32 *)s.flabel.p, nf, (const u32 *)vstart,
+                       (u32)B, (const u32 *)live.p, tnode.p, tlabel.p, s.counter.p);
+            HIPCHK(hipMemcpyAsync(ctx->h_scalars, s.counter.p, 4, hipMemcpyDeviceToHost, ctx->stream));
+            ctx->sync();
+            nf = *(u32 *)ctx->h_scalars;
+            s.fnode.swap(tnode);
+            s.flabel.swap(tlabel);
+        }
+        if (o.max_it > 0 && rounds >= o.max_it) break;
+    }
+}
+
 void batch_run(dlg_ctx *ctx, int prog, int B, const int32_t *const *rows, const int64_t *n,
                       const Opts &o, dlg_result *res, dlg_batch_stats *st) {
     Layout L = make_layout(B, rows, n);
@@ -507,7 +565,7 @@ void batch_run(dlg_ctx *ctx, int prog, int B, const int32_t *const *rows, const 
         WccGraph g(ctx);
         wcc_graph_build(ctx, d_rows.p, N, o, pc, g);
         u64 V = g.V;
-        DBuf<u32> gkey(ctx, V ? V : 1), vstart(ctx, B + 1), cnt(ctx, B), live(ctx, B), largest(ctx, B);
+        DBuf<u32> gkey(ctx, V ? V : 1), vstart(ctx, B + 1), largest(ctx, B);
         if (V)
             DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * V, group_keys_k, sgrid(ctx, V), ctx->block_size, 0,
                        (const u64 *)g.ix.rows.p, (const u32 *)g.ix.gstart.p, V, gkey.p);
@@ -520,54 +578,15 @@ void batch_run(dlg_ctx *ctx, int prog, int B, const int32_t *const *rows, const 
         HIPCHK(hipMemcpyAsync(vstart.p, hv.data(), 4 * (B + 1), hipMemcpyHostToDevice, ctx->stream));
         pc.mark(DLG_PH_INIT);
         WccState s(ctx);
-        wcc_setup(ctx, s, V);
-        std::vector<i64> prev(B), cur(B);
         std::vector<int> iters(B, 0);
-        std::vector<char> done(B, 0);
-        std::vector<u32> hlive(B, 1);
-        for (int i = 0; i < B; i++) prev[i] = (i64)(hv[i + 1] - hv[i]);   // wcc.cu:236-242
-        int live_n = B;
-        u64 nf = V;
-        DBuf<u32> tnode(ctx, V ? V : 1), tlabel(ctx, V ? V : 1);
-        std::vector<u32> hc(B);
-        while (live_n > 0) {
+        const bool whole = o.strategy == 0 && o.relax == WCC_AUTO && g.ne <= WD_MAX_EDGES;
+        if (whole) {
             pc.mark(DLG_PH_JOIN);
-            rounds++;
-            u64 nn = nf ? wcc_round(ctx, s, g.ix, g.nbr.p, nf, (u32)rounds) : 0;
-            fill_u32(ctx, cnt.p, B, 0u);
-            if (nn)
-                DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * nn, frontier_hist_k, sgrid(ctx, nn), ctx->block_size, 0,
-                           (const u32 *)s.fnode.p, nn, (const u32 *)vstart.p, (u32)B, cnt.p);
-            HIPCHK(hipMemcpyAsync(hc.data(), cnt.p, 4 * B, hipMemcpyDeviceToHost, ctx->stream));
-            ctx->sync();
-            bool froze = false;
-            for (int i = 0; i < B; i++) {
-                if (done[i]) continue;
-                iters[i]++;
-                cur[i] = hc[i];
-                if (cur[i] == prev[i]) {                  // wcc.cu:366-383, per instance
-                    done[i] = 1;
-                    hlive[i] = 0;
-                    live_n--;
-                    froze = froze || hc[i] > 0;
-                } else {
-                    prev[i] = cur[i];
-                }
-            }
-            nf = nn;
-            if (froze && nf) {
-                HIPCHK(hipMemcpyAsync(live.p, hlive.data(), 4 * B, hipMemcpyHostToDevice, ctx->stream));
-                fill_u32(ctx, s.counter.p, 1, 0u);
-                DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * nf, frontier_filter_k, sgrid(ctx, nf), ctx->block_size, 0,
-                           (const u32 *)s.fnode.p, (const u32 *)s.flabel.p, nf, (const u32 *)vstart.p,
-                           (u32)B, (const u32 *)live.p, tnode.p, tlabel.p, s.counter.p);
-                HIPCHK(hipMemcpyAsync(ctx->h_scalars, s.counter.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-                ctx->sync();
-                nf = *(u32 *)ctx->h_scalars;
-                s.fnode.swap(tnode);
-                s.flabel.swap(tlabel);
-            }
-            if (o.max_it > 0 && rounds >= o.max_it) break;
+            std::vector<u32> hit;
+            rounds = wcc_rounds_whole(ctx, s, V, g.ix, g.nbr.p, o.max_it, vstart.p, (u32)B, &hit);
+            for (int i = 0; i < B; i++) iters[i] = (int)hit[i];
+        } else {
+            wcc_batch_rounds(ctx, s, g, o, pc, vstart.p, hv, iters, rounds);
         }
         // components per instance
         pc.mark(DLG_PH_FINAL);

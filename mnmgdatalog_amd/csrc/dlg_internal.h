@@ -674,6 +674,13 @@ u64 wcc_relax_tuples(dlg_ctx *ctx, const Index &ix, const u32 *nbr, const u64 *d
                      u64 *next);
 // #components, largest component size and the (label, 0) tuples in `out`.
 u64 wcc_finalize(dlg_ctx *ctx, WccState &s, const Index &ix, DBuf<u64> &out, i64 *largest);
+// All rounds by whole-graph pulls, one launch each (s needs no set-up):
+// returns the iteration count (labels in s.L).  Taken up to WD_MAX_EDGES edges.
+constexpr u64 WD_MAX_EDGES = 1ull << 25;
+// With vstart (device, B + 1 entries: instance i holds the nodes [vstart[i],
+// vstart[i + 1])), each instance stops by its own rule, its round count in iters.
+int wcc_rounds_whole(dlg_ctx *ctx, WccState &s, u64 V, const Index &ix, const u32 *nbr, int max_it,
+                     const u32 *vstart = nullptr, u32 B = 0, std::vector<u32> *iters = nullptr);
 // All rounds through replays of a captured graph of `kr` rounds; returns the
 // iteration count (labels in s.L).  `ne` = edges of the index.
 int wcc_rounds_graph(dlg_ctx *ctx, WccState &s, const Index &ix, const u32 *nbr, u64 ne, int max_it,

@@ -744,13 +744,16 @@ static void run_sj(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, dl
 void wcc_solve(dlg_ctx *ctx, const WccGraph &g, const Opts &o, PhaseClock &pc, dlg_result *res) {
     pc.mark(DLG_PH_INIT);
     WccState s(ctx);
-    wcc_setup(ctx, s, g.V);
-    int it = 0;
-    const bool graph = o.strategy == 2 || (o.strategy == 0 && o.relax == WCC_AUTO && g.ne <= (1ull << 25));
+    int it = -1;
     pc.mark(DLG_PH_JOIN);
-    if (graph) {
+    if (o.strategy == 0 && o.relax == WCC_AUTO && g.ne <= WD_MAX_EDGES)
+        it = wcc_rounds_whole(ctx, s, g.V, g.ix, g.nbr.p, o.max_it);
+    const bool graph = o.strategy == 2 || (o.strategy == 0 && o.relax == WCC_AUTO && g.ne <= (1ull << 25));
+    if (it < 0) wcc_setup(ctx, s, g.V);
+    if (it < 0 && graph) {
         it = wcc_rounds_graph(ctx, s, g.ix, g.nbr.p, g.ne, o.max_it, 16);
-    } else {
+    } else if (it < 0) {
+        it = 0;
         u64 nf = g.V;
         u64 prev = g.V;                                    // wcc.cu:236-242
         while (true) {

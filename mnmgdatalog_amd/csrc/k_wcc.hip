@@ -32,6 +32,7 @@
 #include "dlg_internal.h"
 
 #include <algorithm>
+#include <deque>
 
 namespace dlg {
 
@@ -506,6 +507,338 @@ u64 wcc_finalize(dlg_ctx *ctx, WccState &s, const Index &ix, DBuf<u64> &out, i64
                (const u32 *)flags.p, (const u64 *)offs.p, V, (const u64 *)ix.rows.p,
                (const u32 *)ix.gstart.p, out.p);
     return ncomp;
+}
+
+}  // namespace dlg
+
+// =====================================================================
+// Whole-graph rounds: for graphs of moderate size every round pulls every
+// node from the labels of the round before (two label arrays in turn: exactly
+// the Jacobi round) in ONE launch -- no frontier, no degree scan, no append,
+// no label atomics.  Rounds are queued ahead of the host: kernel r publishes
+// round r - 1's count, applies the stop rule to it and, when it fires, lets the
+// kernels after it do nothing (round r itself writes the other array, so the
+// labels of the last counted round stay in theirs).
+// A thread takes a node of up to WD_THREAD edges, a wave one of up to WD_WAVE, a
+// workgroup WD_SEG edges of a larger one (a hub's segments meet in an atomic
+// minimum).
+// Bound by the latency of start -> neighbour -> label (L2) for small graphs, by
+// the label reads for large ones.
+// Whole calls against the captured push rounds, which stay for `strategy` 2:
+// 160,000 nodes, 355,000 edges, ~500 rounds 15.4 -> 2.0 ms (a round 4.6 us
+// instead of 41); 12.4M nodes, 28.8M edges, 4,303 rounds 2,693 -> 344 ms;
+// R-MAT 2^17 to 2^20 nodes 1.36 -> 0.82 and 4.3 -> 4.1 ms; a star of 200,000
+// 1.0 -> 0.56 ms (1.1 with its hub in one workgroup).  Never slower up to
+// WD_MAX_EDGES, the range the captured rounds were taken for.
+// Batches: 400 instances 2.8 -> 1.6 ms on the device.
+namespace dlg {
+
+constexpr int WD_T = 256, WD_SLOTS = 64, WD_SETS = 4, WD_LINE = 8;
+constexpr u32 WD_THREAD = 16, WD_WAVE = 1024, WD_SEG = 8192;
+constexpr int WD_DEPTH = 4;   // rounds queued ahead of the host
+static_assert(WD_DEPTH + 2 <= dlg_ctx::MAPPED_SLOTS, "every queued round has a mapped slot of its own");
+
+struct WdState {
+    unsigned long long cnt[WD_SETS][WD_SLOTS][WD_LINE];   // lowered nodes, by round and slice
+    u64 prev;    // |Δ| of the round before (wcc.cu:236-242)
+    u32 done;    // the stop rule fired (every instance's)
+    u32 nmid, nhub;   // middle nodes, hub segments
+};
+
+// The batched form's instances (contiguous node ranges), each with its own
+// stop rule: an instance's labels stay where its last round left them, in
+// the array of that round's parity, and the end picks them from there.
+struct WdInst {
+    const u32 *of;       // each node's instance (null: one graph)
+    u32 B;
+    u32 *cnt;            // WD_SETS sets of B counts
+    u32 *prev, *done, *iters;
+};
+
+// The nodes that a wave takes, and the segments (node, first edge) that a
+// workgroup takes.
+__global__ __launch_bounds__(WD_T) void wd_lists_k(const u32 *gstart, u64 V, u32 *mid, uint2 *hub, WdState *st) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    const u64 stride = (u64)gridDim.x * WD_T, lim = (V + WAVE - 1) / WAVE * WAVE;   // whole waves iterate together
+    for (u64 i = (u64)blockIdx.x * WD_T + threadIdx.x; i < lim; i += stride) {
+        const u32 a = i < V ? gstart[i] : 0u, d = i < V ? gstart[i + 1] - a : 0u;
+        const bool is_mid = d > WD_THREAD && d <= WD_WAVE;
+        const u64 bm = __ballot(is_mid);
+        u32 b = 0;
+        if (lane == 0 && bm) b = atomicAdd(&st->nmid, (u32)__popcll(bm));
+        b = (u32)__shfl((int)b, 0, WAVE);
+        if (is_mid) mid[b + (u32)__popcll(bm & lanemask_lt())] = (u32)i;
+        if (d > WD_WAVE) {
+            u32 j = atomicAdd(&st->nhub, (d + WD_SEG - 1) / WD_SEG);
+            for (u32 e = 0; e < d; e += WD_SEG) hub[j++] = make_uint2((u32)i, a + e);
+        }
+    }
+}
+
+// Identity labels in both arrays: a hub's segments lower a label of two rounds
+// ago, which is never below the last one.
+__global__ void wd_init_k(WdState *st, u32 *L, u32 *Ln, u64 V) {
+    const u64 i0 = (u64)blockIdx.x * blockDim.x + threadIdx.x, stride = (u64)gridDim.x * blockDim.x;
+    for (u64 i = i0; i < V; i += stride) L[i] = Ln[i] = (u32)i;
+    for (u64 i = i0; i < (u64)WD_SETS * WD_SLOTS * WD_LINE; i += stride) (&st->cnt[0][0][0])[i] = 0;
+    if (i0 == 0) {
+        st->prev = V;
+        st->done = st->nmid = st->nhub = 0;
+    }
+}
+
+__global__ void wd_sizes_k(const WdState *st, u64 *host, u64 seq) {
+    if (threadIdx.x != 0) return;
+    host[0] = st->nmid;
+    host[1] = st->nhub;
+    __threadfence_system();
+    *(volatile u64 *)(host + dlg_ctx::MAPPED_SEQ) = seq;
+    __threadfence_system();
+}
+
+__device__ __forceinline__ u32 wd_wave_min(u32 v) {
+#pragma unroll
+    for (int d = WAVE / 2; d > 0; d >>= 1) v = min(v, (u32)__shfl_xor((int)v, d, WAVE));
+    return v;
+}
+
+// Nodes the threads lowered: into the round's count, by slice, or (instances)
+// by the node's instance.
+template <bool MULTI>
+__device__ __forceinline__ void wd_count(WdState *st, const WdInst &in, u32 round, u32 wg, bool low, u32 inst, u32 *s_v) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    if (MULTI) {
+        wave_count_by_key(in.cnt + (u64)(round % WD_SETS) * in.B, inst, low);
+        return;
+    }
+    const u32 c = (u32)__popcll(__ballot(low));
+    if (lane == 0) s_v[threadIdx.x / WAVE] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        u32 t = 0;
+        for (int w = 0; w < WD_T / WAVE; w++) t += s_v[w];
+        if (t) atomicAdd(&st->cnt[round % WD_SETS][wg % WD_SLOTS][0], (unsigned long long)t);
+    }
+}
+
+// Publishes round `round` - 1: the stop rule (wcc.cu:366-383) on its count, or
+// on each instance's; host[1] = nothing is left to run.
+template <bool MULTI>
+__device__ __forceinline__ void wd_publish(WdState *st, const WdInst &in, u32 round, u64 *host, u64 seq) {
+    __shared__ u32 s_live;
+    if (MULTI) {
+        if (threadIdx.x == 0) s_live = 0;
+        __syncthreads();
+        const u32 *cur = in.cnt + (u64)((round - 1) % WD_SETS) * in.B;
+        u32 *next = in.cnt + (u64)((round + 1) % WD_SETS) * in.B;
+        u32 live = 0;
+        for (u32 i = threadIdx.x; i < in.B; i += WD_T) {
+            next[i] = 0;
+            if (in.done[i]) continue;
+            in.iters[i] = round - 1;
+            if (cur[i] == in.prev[i]) in.done[i] = 1;
+            else live++;
+            in.prev[i] = cur[i];
+        }
+        if (live) atomicAdd(&s_live, live);
+        __syncthreads();
+        if (threadIdx.x == 0) host[1] = st->done = s_live == 0;
+    } else if (threadIdx.x < WAVE) {   // WD_SLOTS == WAVE: a slice per lane
+        u64 c = st->cnt[(round - 1) % WD_SETS][threadIdx.x][0];
+        st->cnt[(round + 1) % WD_SETS][threadIdx.x][0] = 0;
+#pragma unroll
+        for (int d = WAVE / 2; d > 0; d >>= 1) c += __shfl_xor(c, d, WAVE);
+        if (threadIdx.x == 0) {
+            host[1] = st->done = st->done || c == st->prev;
+            st->prev = c;
+        }
+    }
+    if (threadIdx.x == 0) {
+        __threadfence_system();
+        *(volatile u64 *)(host + dlg_ctx::MAPPED_SEQ) = seq;
+        __threadfence_system();
+    }
+}
+
+// Round `round` from L into Ln, the round before published first (or only
+// the publication).  Workgroups: the publisher, the nodes by thread, the
+// middle nodes by wave, the hubs' segments by workgroup.
+template <bool MULTI>
+__global__ __launch_bounds__(WD_T) void wd_round_k(const u32 *gstart, const u32 *nbr, u64 V, const u32 *L, u32 *Ln,
+                                                   const u32 *mid, u32 nmid, const uint2 *hub, WdState *st, WdInst in,
+                                                   u32 round, int publish_only, u64 *host, u64 seq) {
+    __shared__ u32 s_v[WD_T / WAVE];
+    const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
+    if (blockIdx.x == 0) {
+        if (round > 1) wd_publish<MULTI>(st, in, round, host, seq);
+        return;
+    }
+    if (publish_only || st->done) return;
+    const u32 wg = blockIdx.x - 1, nthr = (u32)((V + WD_T - 1) / WD_T), nwav = (nmid + WD_T / WAVE - 1) / (WD_T / WAVE);
+    bool low = false;   // this thread lowered a node, of instance `inst`
+    u32 inst = 0;
+    if (wg < nthr) {
+        const u64 i = (u64)wg * WD_T + threadIdx.x;
+        if (i < V) {
+            const u32 a = gstart[i], d = gstart[i + 1] - a;
+            if (MULTI) inst = in.of[i];
+            if (d <= WD_THREAD && !(MULTI && in.done[inst])) {
+                const u32 old = L[i];
+                u32 m = old;
+                for (u32 e = 0; e < d; e += 4) {   // four neighbours in flight (a lane past the end reads the last again)
+                    u32 v[4];
+#pragma unroll
+                    for (u32 k = 0; k < 4; k++) v[k] = nbr[a + min(e + k, d - 1)];
+#pragma unroll
+                    for (u32 k = 0; k < 4; k++) m = min(m, L[v[k]]);
+                }
+                Ln[i] = m;
+                low = m < old;
+            }
+        }
+    } else if (wg < nthr + nwav) {
+        const u32 j = (wg - nthr) * (WD_T / WAVE) + (u32)wv;
+        if (j < nmid) {
+            const u32 i = mid[j], a = gstart[i], d = gstart[i + 1] - a;
+            if (MULTI) inst = in.of[i];
+            if (!(MULTI && in.done[inst])) {   // wave-uniform
+                u32 m = 0xffffffffu;
+                for (u32 e = (u32)lane; e < d; e += WAVE) m = min(m, L[nbr[a + e]]);
+                m = wd_wave_min(m);
+                if (lane == 0) {
+                    const u32 old = L[i];
+                    m = min(m, old);
+                    Ln[i] = m;
+                    low = m < old;
+                }
+            }
+        }
+    } else {
+        const uint2 h = hub[wg - nthr - nwav];
+        const u32 i = h.x, end = min(h.y + WD_SEG, gstart[i + 1]);
+        if (MULTI) {   // one reading for the workgroup: the flag may be set while it runs
+            inst = in.of[i];
+            if (threadIdx.x == 0) s_v[0] = in.done[inst];
+            __syncthreads();
+            const bool stop = s_v[0] != 0;
+            __syncthreads();
+            if (stop) return;
+        }
+        u32 m = 0xffffffffu;
+        for (u32 e = h.y + threadIdx.x; e < end; e += 4 * WD_T) {
+            u32 v[4];
+#pragma unroll
+            for (u32 k = 0; k < 4; k++) v[k] = nbr[min(e + k * WD_T, end - 1)];
+#pragma unroll
+            for (u32 k = 0; k < 4; k++) m = min(m, L[v[k]]);
+        }
+        m = wd_wave_min(m);
+        if (lane == 0) s_v[wv] = m;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int w = 1; w < WD_T / WAVE; w++) m = min(m, s_v[w]);
+            const u32 old = L[i];
+            // the node's first segment to go below its last label counts it
+            low = atomicMin(&Ln[i], min(m, old)) >= old && m < old;
+        }
+        __syncthreads();   // s_v is rewritten below
+    }
+    wd_count<MULTI>(st, in, round, wg, low, inst, s_v);
+}
+
+// Each node's instance (vstart[i] <= v < vstart[i + 1]); the instances' state.
+__global__ void wd_inst_k(const u32 *vstart, WdInst in, u64 V, u32 *of) {
+    const u64 i0 = (u64)blockIdx.x * blockDim.x + threadIdx.x, stride = (u64)gridDim.x * blockDim.x;
+    for (u64 v = i0; v < V; v += stride) {
+        u32 a = 0, b = in.B;
+        while (b - a > 1) {
+            const u32 m = (a + b) >> 1;
+            if (vstart[m] <= (u32)v) a = m; else b = m;
+        }
+        of[v] = a;
+    }
+    for (u64 i = i0; i < (u64)WD_SETS * in.B; i += stride) in.cnt[i] = 0;
+    for (u64 i = i0; i < in.B; i += stride) {
+        in.prev[i] = vstart[i + 1] - vstart[i];
+        in.done[i] = in.iters[i] = 0;
+    }
+}
+// The labels of each node's instance's last round.
+__global__ void wd_pick_k(u32 *L, const u32 *Ln, u64 V, WdInst in) {
+    const u64 stride = (u64)gridDim.x * blockDim.x;
+    for (u64 v = (u64)blockIdx.x * blockDim.x + threadIdx.x; v < V; v += stride)
+        if (in.iters[in.of[v]] & 1u) L[v] = Ln[v];
+}
+
+int wcc_rounds_whole(dlg_ctx *ctx, WccState &s, u64 V, const Index &ix, const u32 *nbr, int max_it, const u32 *vstart,
+                     u32 B, std::vector<u32> *iters) {
+    s.V = V;
+    if (iters) iters->assign(B, 1);
+    if (V == 0) return 1;   // empty graph: the first round already sees 0 == 0
+    s.L.ensure(V);
+    s.counter.ensure(4);
+    static_assert(WD_SLOTS == WAVE, "the publisher's wave sums a slice per lane");
+    DBuf<u64> stbuf(ctx, (sizeof(WdState) + 7) / 8);
+    WdState *st = (WdState *)stbuf.p;
+    s.Ln.ensure(V);
+    u32 *buf[2] = {s.L.p, s.Ln.p};   // round r leaves its labels in buf[r & 1]
+    DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * V, wd_init_k, sgrid(ctx, V), ctx->block_size, 0, st, buf[0], buf[1], V);
+    DBuf<u32> mid(ctx, ix.n / WD_THREAD + 1);
+    DBuf<uint2> hub(ctx, ix.n / WD_WAVE + ix.n / WD_SEG + 1);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * V, wd_lists_k, (unsigned)std::min<u64>((V + WD_T - 1) / WD_T, (u64)ctx->num_cus * 8),
+               WD_T, 0, (const u32 *)ix.gstart.p, V, mid.p, hub.p, st);
+    WdInst in{nullptr, B, nullptr, nullptr, nullptr, nullptr};
+    DBuf<u32> of(ctx), ist(ctx);
+    if (vstart) {
+        of.ensure(V);
+        ist.ensure((u64)(WD_SETS + 3) * B);
+        in.of = of.p;
+        in.cnt = ist.p;
+        in.prev = ist.p + (u64)WD_SETS * B;
+        in.done = in.prev + B;
+        in.iters = in.done + B;
+        DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * V, wd_inst_k, sgrid(ctx, V), ctx->block_size, 0, vstart, in, V, of.p);
+    }
+    u64 seq = ++ctx->mapped_seq;
+    DLG_LAUNCH(ctx, DLG_K_MISC, 0.0, wd_sizes_k, 1, 64, 0, (const WdState *)st, ctx->mapped_dev(seq), seq);
+    ctx->wait_mapped(seq);
+    const u32 nmid = (u32)ctx->mapped_host(seq)[0], nhub = (u32)ctx->mapped_host(seq)[1];
+    const unsigned g = 1u + (unsigned)((V + WD_T - 1) / WD_T) + (nmid + WD_T / WAVE - 1) / (WD_T / WAVE) + nhub;
+    std::deque<u64> q;   // sequence numbers of the rounds not read yet
+    int launched = 0, it = 0;
+    auto launch = [&](bool publish_only) {
+        const u32 r = (u32)launched + 1;
+        seq = r > 1 ? ++ctx->mapped_seq : 0;   // round 1 has no round before it
+        auto go = [&](auto kern) {
+            // 4 B neighbour + 4 B label per edge; a start and two labels per node
+            DLG_LAUNCH(ctx, DLG_K_WCC_RELAX, publish_only ? 0.0 : 8.0 * ix.n + 16.0 * V, kern, publish_only ? 1u : g, WD_T,
+                       0, (const u32 *)ix.gstart.p, nbr, V, (const u32 *)buf[(r - 1) & 1], buf[r & 1],
+                       (const u32 *)mid.p, nmid, (const uint2 *)hub.p, st, in, r, publish_only ? 1 : 0,
+                       ctx->mapped_dev(seq), seq);
+        };
+        if (vstart) go(wd_round_k<true>);
+        else go(wd_round_k<false>);
+        if (r > 1) q.push_back(seq);
+        if (!publish_only) launched++;
+    };
+    while (true) {
+        while (launched < it + 1 + WD_DEPTH && (max_it <= 0 || launched < max_it)) launch(false);
+        if (q.empty()) launch(true);   // the last round asked for
+        ctx->wait_mapped(q.front());
+        const bool done = ctx->mapped_host(q.front())[1] != 0;
+        q.pop_front();
+        it++;
+        if (done || (max_it > 0 && it >= max_it)) break;
+    }
+    if (vstart) {
+        DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * V, wd_pick_k, sgrid(ctx, V), ctx->block_size, 0, s.L.p, (const u32 *)s.Ln.p, V,
+                   in);
+        HIPCHK(hipMemcpyAsync(iters->data(), in.iters, 4 * (size_t)B, hipMemcpyDeviceToHost, ctx->stream));
+        ctx->sync();
+    } else if (it & 1) {
+        s.L.swap(s.Ln);
+    }
+    return it;
 }
 
 }  // namespace dlg

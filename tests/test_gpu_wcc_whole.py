@@ -1,0 +1,66 @@
+"""WCC by whole-graph pulls: nodes at the edges of the thread, wave and workgroup classes, round limits,
+and batches whose instances stop by their own rule, against the oracle and the pushed rounds."""
+import numpy as np
+import pytest
+
+import mnmgdatalog_amd as dlg
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = dlg.Ctx(0)
+    yield c
+    c.close()
+
+
+def same(a, b):
+    assert (a["iterations"], a["output_size"], a["secondary"]) == (b["iterations"], b["output_size"], b["secondary"])
+    assert np.array_equal(a["rows"], b["rows"])
+
+
+def stars(degrees, seed):
+    """Hubs of the given degrees (distinct leaves, some shared between neighbouring hubs), ids shuffled."""
+    r, at = [], len(degrees)
+    for h, d in enumerate(degrees):
+        r.append(np.stack([np.full(d, h), np.arange(at, at + d)], 1))
+        at += d - (h % 2)
+    r = np.concatenate(r)
+    return np.random.default_rng(seed).permutation(r.max() + 1).astype(np.int32)[r]
+
+
+@pytest.mark.parametrize("degrees", [[1], [15, 16, 17], [16] * 40 + [17] * 40, [1023, 1024, 1025], [8191, 8192, 8193],
+                                     [1025, 3, 20_000, 64, 16_384, 16_385, 17]])
+def test_degree_classes(ctx, orc, degrees):
+    rows = stars(degrees, len(degrees))
+    same(ctx.run("wcc", rows), orc.wcc(rows))
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 700])
+def test_paths(ctx, orc, n):
+    rows = np.stack([np.arange(n), np.arange(1, n + 1)], 1).astype(np.int32)
+    same(ctx.run("wcc", rows), orc.wcc(rows))
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 7])
+def test_truncated(ctx, k):
+    rows = np.concatenate([dlg.gen_grid(30, 0.55, 0.01, 20, 3), stars([2000, 9000], 2) + 5000])
+    same(ctx.run("wcc", rows, max_iterations=k), ctx.run("wcc", rows, max_iterations=k, strategy=2))
+
+
+@pytest.mark.parametrize("limit", [0, 1, 3, 6])
+def test_batch_stops_each_by_its_own_rule(ctx, limit):
+    """Paths (many rounds), stars (few, with hub segments), grids and empty instances side by side."""
+    inst = [np.stack([np.arange(w), np.arange(1, w + 1)], 1).astype(np.int32) for w in (1, 5, 60, 300)]
+    inst += [stars([17, 16], 1), stars([1500], 2), stars([20_000, 9], 3), np.zeros((0, 2), np.int32)]
+    inst += [dlg.gen_grid(24, 0.55, 0.01, 20, s) for s in range(3)]
+    kw = {"max_iterations": limit} if limit else {}
+    res, _ = ctx.batch_run("wcc", inst, **kw)
+    for r, rows in zip(res, inst):
+        want = ctx.run("wcc", rows, strategy=2, **kw)
+        if len(rows) == 0:
+            assert r["output_size"] == 0
+            continue
+        same(r, want)
+        assert r["nodes"] == want["nodes"]
