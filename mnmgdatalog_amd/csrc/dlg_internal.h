@@ -41,6 +41,9 @@ hipEvent_t timing_event();   // an event for timing only (no system-scope fence)
 // block of the library).  Null on failure.
 void *host_block_alloc(size_t bytes);
 void host_block_free(void *p);
+// One context more (+1) or fewer (-1): with the last one, the page-locked
+// blocks kept for later results go back to the runtime.
+void host_contexts(int change);
 // Looks up, once per device and with that device current, the address of the
 // no-allocation entry points' static scratch array (noalloc.hip); called by
 // dlg_ctx_create.  A failure is kept and reported by those entry points.
@@ -117,6 +120,7 @@ struct dlg_ctx {
     // have a slot of their own.
     uint64_t *h_mapped = nullptr, *d_mapped = nullptr;
     uint64_t mapped_seq = 0;
+    bool counted = false;   // among the contexts that keep page-locked host blocks
     static constexpr int MAPPED_SEQ = 7, MAPPED_WORDS = 8, MAPPED_SLOTS = 8;
     static constexpr int MAPPED_SPIN_US = 2000;   // busy-wait this long, then yield between checks
     uint64_t *mapped_host(uint64_t seq) const { return h_mapped + MAPPED_WORDS * (seq % MAPPED_SLOTS); }
