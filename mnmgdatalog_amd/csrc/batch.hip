@@ -495,9 +495,9 @@ static void wcc_batch_rounds(dlg_ctx *ctx, WccState &s, const WccGraph &g, const
             DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * nf, frontier_filter_k, sgrid(ctx, nf), ctx->block_size, 0,
                        (const u32 *)s.fnode.p, (const u32 *)s.flabel.p, nf, (const u32 *)vstart,
                        (u32)B, (const u32 *)live.p, tnode.p, tlabel.p, s.counter.p);
-            HIPCHK(hipMemcpyAsync(ctx->h_scalars, s.counter.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-            ctx->sync();
-            nf = *(u32 *)ctx->h_scalars;
+            u32 kept = 0;
+            ctx->read_words(s.counter.p, 1, &kept);
+            nf = kept;
             s.fnode.swap(tnode);
             s.flabel.swap(tlabel);
         }

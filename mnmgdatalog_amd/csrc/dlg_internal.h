@@ -110,8 +110,6 @@ struct dlg_ctx {
     std::vector<dlg::ProfRec> pending;
     std::vector<hipEvent_t> event_free;
     hipEvent_t cur_a = nullptr;
-    // pinned host scalar area for size read-backs
-    uint64_t *h_scalars = nullptr;
     // pinned host words that kernels write directly (mapped), as a ring of
     // MAPPED_SLOTS slots of MAPPED_WORDS words: a fixpoint round's totals go
     // to slot seq % MAPPED_SLOTS, then (after a system-scope fence) the
@@ -138,7 +136,9 @@ struct dlg_ctx {
     // (spinning: no sleep between the kernel's write and the host's next
     // launch); fails if the stream runs dry without it.
     void wait_mapped(uint64_t seq);
-    // read `count` u64 scalars from device memory into host (synchronises)
+    // read a few words / u64 scalars (at most MAPPED_SEQ u64s) from device
+    // memory, after everything queued before (synchronises)
+    void read_words(const uint32_t *d, int words, void *h);
     void read_scalars(const uint64_t *d, int count, uint64_t *h);
 };
 
@@ -354,6 +354,18 @@ void radix_sort(dlg_ctx *ctx, u64 *data, u64 n, DBuf<u64> &tmp, int bits = 0, bo
 // every element; otherwise a pass over the data computes them.
 void radix_sort(dlg_ctx *ctx, DBuf<u64> &data, u64 n, DBuf<u64> &tmp, int bits = 0,
                 const u32 *bounds = nullptr, bool key_only = false);
+// Inputs of up to this many tuples are sorted, and compacted, by one workgroup
+// in one launch.
+constexpr u64 SORT_SMALL_MAX = 8192;
+// in[0, n), n <= SORT_SMALL_MAX, sorted into out (may be in) with one copy of
+// each (returns their number), or whole with the index of each key's first
+// tuple in heads (returns the keys' number).
+u64 sort_unique_small(dlg_ctx *ctx, const u64 *in, u64 n, u64 *out);
+u64 sort_heads_small(dlg_ctx *ctx, const u64 *in, u64 n, u64 *out, u32 *heads);
+// in[0, n) sorted into out (resized; `in` is left alone).
+void radix_sort_into(dlg_ctx *ctx, const u64 *in, u64 n, DBuf<u64> &out, DBuf<u64> &tmp);
+// data[0, n) sorted in place with one copy of each; returns their number.
+u64 sort_unique(dlg_ctx *ctx, u64 *data, u64 n);
 // Digest of tuples as output rows in `orient` (dlg_result.output_sum) and the
 // number of i with d[i] >= d[i + 1] (synchronises).
 void rows_digest(dlg_ctx *ctx, const u64 *d, u64 n, int orient, u64 *sum, u64 *breaks);

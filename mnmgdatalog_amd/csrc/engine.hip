@@ -79,8 +79,9 @@ static u64 sort_unique_into(dlg_ctx *ctx, DBuf<u64> &buf, u64 n, DBuf<u64> &tmp,
                             int mode, const u64 *other, u64 n_other, int bits,
                             const u32 *bounds = nullptr) {
     if (n == 0) return 0;
-    radix_sort(ctx, buf, n, tmp, bits, bounds);
     out.ensure(n);
+    if (mode == SEL_UNIQUE && n <= SORT_SMALL_MAX) return sort_unique_small(ctx, buf.p, n, out.p);
+    radix_sort(ctx, buf, n, tmp, bits, bounds);
     return select(ctx, mode, buf.p, n, other, n_other, out.p);
 }
 
@@ -985,14 +986,8 @@ dlg_status dlg_sort_unique(dlg_ctx *c, uint64_t *d, int64_t n, int64_t *out_n) {
     if (!c || !out_n || n < 0 || (n && !d)) return DLG_INVALID_INPUT;
     *out_n = 0;
     API_BEGIN(c)
-    if (n) {
-        DBuf<u64> tmp(c), out(c, (size_t)n);
-        radix_sort(c, d, (u64)n, tmp);
-        u64 k = select(c, SEL_UNIQUE, d, (u64)n, nullptr, 0, out.p);
-        copy_u64(c, d, out.p, k);
-        c->sync();
-        *out_n = (int64_t)k;
-    }
+    *out_n = (int64_t)sort_unique(c, d, (u64)n);
+    c->sync();
     API_END(c)
 }
 
@@ -1003,9 +998,16 @@ dlg_status dlg_set_difference(dlg_ctx *c, const uint64_t *a, int64_t na, const u
     *out_n = 0;
     API_BEGIN(c)
     if (na) {
-        DBuf<u64> o(c, (size_t)na);
-        u64 k = select(c, SEL_NOT_IN, a, (u64)na, b, (u64)nb, o.p);
-        copy_u64(c, out, o.p, k);
+        // straight into out, unless it may overlap an input
+        auto meets = [&](const uint64_t *p, int64_t m) { return out < p + m && p < out + na; };
+        u64 k;
+        if (meets(a, na) || meets(b, nb)) {
+            DBuf<u64> o(c, (size_t)na);
+            k = select(c, SEL_NOT_IN, a, (u64)na, b, (u64)nb, o.p);
+            copy_u64(c, out, o.p, k);
+        } else {
+            k = select(c, SEL_NOT_IN, a, (u64)na, b, (u64)nb, out);
+        }
         c->sync();
         *out_n = (int64_t)k;
     }

@@ -71,14 +71,21 @@ void index_build(dlg_ctx *ctx, Index &ix, const u64 *rel, u64 n, double lf, bool
     if (n >= 0xffffffffull) fail(DLG_OVERFLOW, "index: relation larger than 2^32-2 rows");
     if (!(lf > 0.0)) lf = ctx->load_factor;
     lf = std::min(0.95, std::max(0.05, lf));
-    ix.rows.ensure(n);
-    if (rel != ix.rows.p) copy_u64(ctx, ix.rows.p, rel, n);
-    if (!presorted) {
-        DBuf<u64> tmp(ctx);
-        radix_sort(ctx, ix.rows, n, tmp);
-    }
     ix.gstart.ensure(n + 1);
-    u64 G = select(ctx, SEL_KEY_HEAD, ix.rows.p, n, nullptr, 0, ix.gstart.p);
+    u64 G;
+    if (!presorted && n <= SORT_SMALL_MAX) {
+        ix.rows.ensure(n);
+        G = sort_heads_small(ctx, rel, n, ix.rows.p, ix.gstart.p);
+    } else {
+        if (!presorted) {   // the relation is read by the first pass, not copied
+            DBuf<u64> tmp(ctx);
+            radix_sort_into(ctx, rel, n, ix.rows, tmp);
+        } else {
+            ix.rows.ensure(n);
+            if (rel != ix.rows.p) copy_u64(ctx, ix.rows.p, rel, n);
+        }
+        G = select(ctx, SEL_KEY_HEAD, ix.rows.p, n, nullptr, 0, ix.gstart.p);
+    }
     DLG_LAUNCH(ctx, DLG_K_MISC, 4.0, set_last_k, 1, 64, 0, ix.gstart.p, G, (u32)n);
     ix.groups = G;
     if (sorted_lookup) return;
@@ -416,14 +423,16 @@ __global__ void lookup_values_rank_k(const u64 *rows, u64 n, const u64 *dir, u32
 // the directory then takes at most 2 bytes per key over the hash table's slots.
 constexpr u64 RANK_IDS_PER_KEY = 64, RANK_SLACK = 1ull << 20;
 
+// The first and last row (rows are sorted).
+static void index_ends(dlg_ctx *ctx, const Index &ix, u64 *ends) {
+    ctx->read_scalars(ix.rows.p, 1, ends);
+    ctx->read_scalars(ix.rows.p + (ix.n - 1), 1, ends + 1);
+}
+
 bool index_rank_lookup_applies(dlg_ctx *ctx, const Index &ix) {
     if (ix.n == 0) return true;
     u64 ends[2];
-    HIPCHK(hipMemcpyAsync(ctx->h_scalars, ix.rows.p, 8, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync((char *)ctx->h_scalars + 8, ix.rows.p + (ix.n - 1), 8, hipMemcpyDeviceToHost,
-                          ctx->stream));
-    ctx->sync();
-    std::memcpy(ends, ctx->h_scalars, 16);
+    index_ends(ctx, ix, ends);
     const u64 W = (u64)(u32)(ends[1] >> 32) - (u32)(ends[0] >> 32) + 1;   // rows are sorted
     return W <= RANK_IDS_PER_KEY * ix.groups + RANK_SLACK;
 }
@@ -436,11 +445,7 @@ void index_lookup_values(dlg_ctx *ctx, const Index &ix, u32 *out) {
         return;
     }
     u64 ends[2];
-    HIPCHK(hipMemcpyAsync(ctx->h_scalars, ix.rows.p, 8, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync((char *)ctx->h_scalars + 8, ix.rows.p + (ix.n - 1), 8, hipMemcpyDeviceToHost,
-                          ctx->stream));
-    ctx->sync();
-    std::memcpy(ends, ctx->h_scalars, 16);
+    index_ends(ctx, ix, ends);
     const u32 lo = (u32)(ends[0] >> 32);
     const u64 W = (u64)(u32)(ends[1] >> 32) - lo + 1;   // rows are sorted: first and last key
     if (W <= RANK_IDS_PER_KEY * ix.groups + RANK_SLACK) {

@@ -546,7 +546,7 @@ __global__ __launch_bounds__(T) void rs_downsweep_k(const u64 *in, u64 *out, u64
 static int bit_width(u32 v) { return v ? 32 - __builtin_clz(v) : 0; }
 
 template <int BITS, int T, int I>
-static void radix_passes(dlg_ctx *ctx, u64 *&src, u64 *&dst, u64 n, RadixKey key, int total_bits) {
+static u64 *radix_passes(dlg_ctx *ctx, const u64 *src, u64 *dst, u64 *other, u64 n, RadixKey key, int total_bits) {
     constexpr int BINS = 1 << BITS, TILE = T * I;
     u32 nb = (u32)((n + TILE - 1) / TILE);
     DBuf<u32> counts(ctx, (size_t)BINS * nb);
@@ -554,12 +554,14 @@ static void radix_passes(dlg_ctx *ctx, u64 *&src, u64 *&dst, u64 n, RadixKey key
     for (int shift = 0; shift < total_bits; shift += BITS) {
         key.shift = (u32)shift;
         DLG_LAUNCH(ctx, DLG_K_SORT_UPSWEEP, 8.0 * n + 4.0 * BINS * nb, (rs_upsweep_k<BITS, T, I>), nb,
-                   T, 0, (const u64 *)src, n, key, counts.p, nb);
+                   T, 0, src, n, key, counts.p, nb);
         scan_u32_inplace(ctx, counts.p, (u64)BINS * nb, bsum);
         DLG_LAUNCH(ctx, DLG_K_SORT_DOWNSWEEP, 16.0 * n + 4.0 * BINS * nb, (rs_downsweep_k<BITS, T, I>),
-                   nb, T, 0, (const u64 *)src, dst, n, key, (const u32 *)counts.p, nb);
-        std::swap(src, dst);
+                   nb, T, 0, src, dst, n, key, (const u32 *)counts.p, nb);
+        src = dst;
+        std::swap(dst, other);
     }
+    return other;
 }
 
 // ---------------------------------------------------------- one-sweep passes
@@ -590,8 +592,9 @@ constexpr u64 OS_VALUE = (1ull << 56) - 1;
 // A pass whose digits span fewer than 8 bits (the top one) has few distinct
 // digits: its count goes through ballot matching, one atomic per distinct
 // digit per wave.  Each thread loads OH_I keys of a tile before counting
-// any.  The kernel is bound by its vector instructions, so the digits come
-// from 32-bit bit-field extracts of the two halves.
+// any, and the next tile's keys are in flight meanwhile (62 -> 58 us for 10M
+// keys).  The kernel is bound by its vector instructions and LDS atomics, so the
+// digits come from 32-bit bit-field extracts of the two halves.
 constexpr int OH_T = 256, OH_I = 8, OH_TILE = OH_T * OH_I;
 
 __global__ __launch_bounds__(OH_T) void os_hist_k(const u64 *in, u64 n, RadixKey key, u32 passes, u32 top_bits,
@@ -602,12 +605,24 @@ __global__ __launch_bounds__(OH_T) void os_hist_k(const u64 *in, u64 n, RadixKey
     __syncthreads();
     const int wave = threadIdx.x / WAVE;
     const u32 p = passes - 1;
-    for (u64 base = (u64)blockIdx.x * OH_TILE; base < n; base += (u64)gridDim.x * OH_TILE) {   // block-uniform
-        u64 x[OH_I];
+    u64 nx[OH_I];   // the next tile's keys, in flight while this one's are counted
+    const u64 step = (u64)gridDim.x * OH_TILE;
+    {
+        const u64 base = (u64)blockIdx.x * OH_TILE;
 #pragma unroll
         for (int r = 0; r < OH_I; r++) {
             const u64 i = base + (u64)r * OH_T + threadIdx.x;
-            x[r] = i < n ? in[i] : 0ull;
+            nx[r] = in[i < n ? i : n - 1];
+        }
+    }
+    for (u64 base = (u64)blockIdx.x * OH_TILE; base < n; base += step) {   // block-uniform
+        u64 x[OH_I];
+#pragma unroll
+        for (int r = 0; r < OH_I; r++) x[r] = nx[r];
+#pragma unroll
+        for (int r = 0; r < OH_I; r++) {   // never predicated: past the end, the last key again (not counted)
+            const u64 i = base + step + (u64)r * OH_T + threadIdx.x;
+            nx[r] = in[i < n ? i : n - 1];
         }
 #pragma unroll
         for (int r = 0; r < OH_I; r++) {
@@ -788,7 +803,7 @@ __global__ __launch_bounds__(T) void os_pass_k(const u64 *in, u64 *out, u64 n, R
 
 // All passes of an 8-bit sort: histograms of every pass in one read, then one
 // kernel per pass (one read, one write of the keys).
-static void radix_onesweep(dlg_ctx *ctx, u64 *&src, u64 *&dst, u64 n, RadixKey key, int total_bits) {
+static u64 *radix_onesweep(dlg_ctx *ctx, const u64 *src, u64 *dst, u64 *other, u64 n, RadixKey key, int total_bits) {
     constexpr int OT = OS_T, OI = OS_I, OTILE = OS_TILE;
     const u32 passes = (u32)((total_bits + 7) / 8);
     const u64 tiles = (n + OTILE - 1) / OTILE;
@@ -805,31 +820,199 @@ static void radix_onesweep(dlg_ctx *ctx, u64 *&src, u64 *&dst, u64 n, RadixKey k
     const u32 top_bits = (u32)(total_bits - 8 * (int)(passes - 1));
     // 4 blocks per CU (32 KiB of LDS each), each looping over tiles
     const unsigned hg = (unsigned)std::min<u64>((n + OH_TILE - 1) / OH_TILE, (u64)ctx->num_cus * 4);
-    DLG_LAUNCH(ctx, DLG_K_SORT_UPSWEEP, 8.0 * n, os_hist_k, hg, OH_T, 0, (const u64 *)src, n, key, passes, top_bits,
+    DLG_LAUNCH(ctx, DLG_K_SORT_UPSWEEP, 8.0 * n, os_hist_k, hg, OH_T, 0, src, n, key, passes, top_bits,
                (unsigned long long *)hist.p);
     DLG_LAUNCH(ctx, DLG_K_SORT_UPSWEEP, 8.0 * 256 * passes, os_starts_k, 1, 256, 0, (const u64 *)hist.p, passes,
                starts);
     for (u32 p = 0; p < passes; p++) {
         key.shift = 8 * p;
         DLG_LAUNCH(ctx, DLG_K_SORT_DOWNSWEEP, 16.0 * n, (os_pass_k<OT, OI>), (unsigned)tiles, OT, 0,
-                   (const u64 *)src, dst, n, key, (const u64 *)(starts + 256 * p), status.p, tickets + p, p, err);
-        std::swap(src, dst);
+                   src, dst, n, key, (const u64 *)(starts + 256 * p), status.p, tickets + p, p, err);
+        src = dst;
+        std::swap(dst, other);
     }
     u32 e = 0;
-    HIPCHK(hipMemcpyAsync(ctx->h_scalars, err, 4, hipMemcpyDeviceToHost, ctx->stream));
-    ctx->sync();
-    e = *(u32 *)ctx->h_scalars;
+    ctx->read_words(err, 1, &e);
     if (e) fail(DLG_DEVICE_ERROR, "radix sort: a tile's look-back did not complete");
+    return other;
 }
 
+// The passes from src (left alone) into dst, then between dst and other (which
+// may be src); returns the one that holds the sorted keys.
 template <int BITS>
-static void radix_passes_sized(dlg_ctx *ctx, u64 *&src, u64 *&dst, u64 n, RadixKey key, int total_bits) {
-    if (BITS == 8 && n >= RS_BIG_MIN)
-        radix_onesweep(ctx, src, dst, n, key, total_bits);
-    else if (n >= RS_BIG_MIN)
-        radix_passes<BITS, RS_BIG_T, RS_BIG_I>(ctx, src, dst, n, key, total_bits);
-    else
-        radix_passes<BITS, RS_SMALL_T, RS_SMALL_I>(ctx, src, dst, n, key, total_bits);
+static u64 *radix_passes_sized(dlg_ctx *ctx, const u64 *src, u64 *dst, u64 *other, u64 n, RadixKey key, int total_bits) {
+    if (BITS == 8 && n >= RS_BIG_MIN) return radix_onesweep(ctx, src, dst, other, n, key, total_bits);
+    if (n >= RS_BIG_MIN) return radix_passes<BITS, RS_BIG_T, RS_BIG_I>(ctx, src, dst, other, n, key, total_bits);
+    return radix_passes<BITS, RS_SMALL_T, RS_SMALL_I>(ctx, src, dst, other, n, key, total_bits);
+}
+
+// ---------------------------------------------------------- sorts by one workgroup
+// Up to SS_MAX keys: bounds, every 8-bit pass (ranks as in os_pass_k, keys
+// exchanged through LDS) and, as asked, the compaction of the equal runs or the
+// key runs' heads, in ONE launch.  Bound by its own latency, about 3 us a pass;
+// the launches it replaces (bounds, four a pass, count, scan, scatter) and their
+// read-backs took 18 us a pass and about 40 us more: 7,001 tuples of 24 bits 26
+// against 95 us, a round of a program's own operators at that size 405 -> 235 us.
+// From SORT_SMALL_MAX on, one CU's ranking takes longer than the launches.
+constexpr int SS_T = 1024;
+enum { SS_SORT = 0, SS_UNIQUE = 1, SS_HEADS = 2 };
+
+// in[0, n) sorted into out (may be in): every tuple (SS_SORT), one of each
+// (SS_UNIQUE), or every tuple and the index of each key's first one in heads
+// (SS_HEADS); SS_UNIQUE and SS_HEADS publish their count.
+template <int I>
+__global__ __launch_bounds__(SS_T) void sort_small_k(const u64 *in, u32 n, u64 *out, int mode, int key_only, u32 *heads,
+                                                     u64 *host, u64 seq) {
+    constexpr int BINS = 256, W = SS_T / WAVE;
+    __shared__ u64 stage[SS_T * I];
+    __shared__ u32 wcnt[W][BINS];
+    __shared__ u32 bstart[BINS];
+    __shared__ u32 sc[W + 1];
+    __shared__ u32 smm[4][W];
+    const int lane = threadIdx.x & (WAVE - 1), wave = threadIdx.x / WAVE;
+    const u32 w0 = (u32)wave * (WAVE * I);   // the wave's keys: w0 + r * 64 + lane, in input order
+    u64 keys[I];
+    u32 mnh = 0xffffffffu, mxh = 0u, mnl = 0xffffffffu, mxl = 0u;
+#pragma unroll
+    for (int r = 0; r < I; r++) {
+        const u32 i = w0 + (u32)r * WAVE + lane;
+        keys[r] = i < n ? in[i] : 0ull;
+        if (i < n) {
+            mnh = min(mnh, tkey(keys[r])); mxh = max(mxh, tkey(keys[r]));
+            mnl = min(mnl, tval(keys[r])); mxl = max(mxl, tval(keys[r]));
+        }
+    }
+#pragma unroll
+    for (int d = WAVE / 2; d > 0; d >>= 1) {
+        mnh = min(mnh, (u32)__shfl_xor((int)mnh, d, WAVE));
+        mxh = max(mxh, (u32)__shfl_xor((int)mxh, d, WAVE));
+        mnl = min(mnl, (u32)__shfl_xor((int)mnl, d, WAVE));
+        mxl = max(mxl, (u32)__shfl_xor((int)mxl, d, WAVE));
+    }
+    if (lane == 0) {
+        smm[0][wave] = mnh; smm[1][wave] = mxh; smm[2][wave] = mnl; smm[3][wave] = mxl;
+    }
+    __syncthreads();
+    for (int w = 0; w < W; w++) {
+        mnh = min(mnh, smm[0][w]); mxh = max(mxh, smm[1][w]);
+        mnl = min(mnl, smm[2][w]); mxl = max(mxl, smm[3][w]);
+    }
+    RadixKey key;
+    key.min_hi = mnh;
+    key.min_lo = mnl;
+    key.vb = key_only ? 0u : 32u - (u32)__builtin_clz((mxl - mnl) | 1u) - (mxl == mnl ? 1u : 0u);
+    const u32 hb = 32u - (u32)__builtin_clz((mxh - mnh) | 1u) - (mxh == mnh ? 1u : 0u);
+    const u32 bits = key.vb + hb;
+    for (u32 shift = 0; shift < bits; shift += 8) {   // block-uniform
+        key.shift = shift;
+        for (int i = threadIdx.x; i < W * BINS; i += SS_T) (&wcnt[0][0])[i] = 0;
+        __syncthreads();
+        u32 pk[I];
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            const bool valid = w0 + (u32)r * WAVE + lane < n;
+            const u32 d = radix_digit8(keys[r], key), nd = ~d;
+            const u64 vm = __ballot(valid);
+            u32 mlo = (u32)vm, mhi = (u32)(vm >> 32);
+#pragma unroll
+            for (int b = 0; b < 8; b++) {
+                const u32 clr = (u32)__builtin_amdgcn_sbfe((int)nd, b, 1);
+                const u64 set = __ballot(clr == 0u);
+                mlo &= (u32)set ^ clr;
+                mhi &= (u32)(set >> 32) ^ clr;
+            }
+            const u32 before = __builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, 0u));
+            const u32 cnt = wcnt[wave][d];
+            if (valid && before == 0) wcnt[wave][d] = cnt + (u32)__popc(mlo) + (u32)__popc(mhi);
+            pk[r] = d | ((cnt + before) << 8);
+            __builtin_amdgcn_wave_barrier();
+        }
+        __syncthreads();
+        u32 tot = 0;
+        if (threadIdx.x < BINS) {
+#pragma unroll
+            for (int w = 0; w < W; w++) {
+                const u32 c = wcnt[w][threadIdx.x];
+                wcnt[w][threadIdx.x] = tot;
+                tot += c;
+            }
+        }
+        const u32 ex = block_exclusive_scan<u32>(tot, sc, nullptr);
+        if (threadIdx.x < BINS) bstart[threadIdx.x] = ex;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < I; r++)
+            if (w0 + (u32)r * WAVE + lane < n) {
+                const u32 d = pk[r] & 0xffu;
+                stage[bstart[d] + wcnt[wave][d] + (pk[r] >> 8)] = keys[r];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            const u32 i = w0 + (u32)r * WAVE + lane;
+            if (i < n) keys[r] = stage[i];
+        }
+    }
+    if (bits == 0) {   // all equal (or sorted by a key they share): as they came
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            const u32 i = w0 + (u32)r * WAVE + lane;
+            if (i < n) stage[i] = keys[r];
+        }
+        __syncthreads();
+    }
+    if (mode != SS_UNIQUE) {
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            const u32 i = w0 + (u32)r * WAVE + lane;
+            if (i < n) out[i] = keys[r];
+        }
+        if (mode == SS_SORT) return;
+    }
+    u32 keep = 0;
+#pragma unroll
+    for (int r = 0; r < I; r++) {   // each thread's I consecutive tuples
+        const u32 i = threadIdx.x * I + r;
+        if (i < n && (i == 0 || (mode == SS_HEADS ? tkey(stage[i]) != tkey(stage[i - 1]) : stage[i] != stage[i - 1])))
+            keep |= 1u << r;
+    }
+    u32 total;
+    u32 at = block_exclusive_scan<u32>((u32)__popc(keep), sc, &total);
+#pragma unroll
+    for (int r = 0; r < I; r++)
+        if ((keep >> r) & 1u) {
+            const u32 i = threadIdx.x * I + r;
+            if (mode == SS_HEADS) heads[at++] = i;
+            else out[at++] = stage[i];
+        }
+    if (threadIdx.x == 0) {
+        host[0] = total;
+        __threadfence_system();
+        *(volatile u64 *)(host + dlg_ctx::MAPPED_SEQ) = seq;
+        __threadfence_system();
+    }
+}
+
+static u64 sort_small(dlg_ctx *ctx, const u64 *in, u64 n, u64 *out, int mode, bool key_only, u32 *heads) {
+    const u64 seq = mode == SS_SORT ? 0 : ++ctx->mapped_seq;
+    auto go = [&](auto kern) {
+        DLG_LAUNCH(ctx, DLG_K_SORT_DOWNSWEEP, 16.0 * n, kern, 1, SS_T, 0, in, (u32)n, out, mode, key_only ? 1 : 0, heads,
+                   ctx->mapped_dev(seq), seq);
+    };
+    if (n <= SS_T) go(sort_small_k<1>);
+    else if (n <= 2 * SS_T) go(sort_small_k<2>);
+    else if (n <= 4 * SS_T) go(sort_small_k<4>);
+    else go(sort_small_k<8>);
+    if (mode == SS_SORT) return n;
+    ctx->wait_mapped(seq);
+    return ((const volatile u64 *)ctx->mapped_host(seq))[0];
+}
+
+u64 sort_unique_small(dlg_ctx *ctx, const u64 *in, u64 n, u64 *out) {
+    return sort_small(ctx, in, n, out, SS_UNIQUE, false, nullptr);
+}
+u64 sort_heads_small(dlg_ctx *ctx, const u64 *in, u64 n, u64 *out, u32 *heads) {
+    return sort_small(ctx, in, n, out, SS_HEADS, false, heads);
 }
 
 void tuple_bounds(dlg_ctx *ctx, const u64 *data, u64 n, u32 *h) {
@@ -837,9 +1020,7 @@ void tuple_bounds(dlg_ctx *ctx, const u64 *data, u64 n, u32 *h) {
     DBuf<u32> mm(ctx, 4 + 4 * (u64)g);   // the bounds, then the workgroups' partials
     if (g) DLG_LAUNCH(ctx, DLG_K_SORT_HIST, 8.0 * n, minmax_k, g, 256, 0, data, n, mm.p + 4);
     DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * g, minmax_final_k, 1, 256, 0, (const u32 *)(mm.p + 4), g, mm.p);
-    HIPCHK(hipMemcpyAsync(ctx->h_scalars, mm.p, 16, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    std::memcpy(h, ctx->h_scalars, 16);
+    ctx->read_words(mm.p, 4, h);
 }
 
 // Per block: the digest sum and the order breaks of a grid-stride share,
@@ -890,9 +1071,14 @@ void rows_digest(dlg_ctx *ctx, const u64 *d, u64 n, int orient, u64 *sum, u64 *b
     *breaks = h[1];
 }
 
-void radix_sort(dlg_ctx *ctx, DBuf<u64> &data, u64 n, DBuf<u64> &tmp, int bits, const u32 *bounds,
-                bool key_only) {
-    if (n < 2) return;
+// in[0, n) sorted into a or b (b may be in): returns the one that holds the
+// result -- `in` itself when there is nothing to do.
+static const u64 *radix_from(dlg_ctx *ctx, const u64 *in, u64 n, u64 *a, u64 *b, int bits, const u32 *bounds, bool key_only) {
+    if (n < 2) return in;
+    if (n <= SORT_SMALL_MAX) {
+        sort_small(ctx, in, n, b, SS_SORT, key_only, nullptr);
+        return b;
+    }
     if (bits <= 0) bits = ctx->radix_bits;
     if (bits < 4) bits = 4;
     if (bits > 8) bits = 8;
@@ -902,37 +1088,55 @@ void radix_sort(dlg_ctx *ctx, DBuf<u64> &data, u64 n, DBuf<u64> &tmp, int bits, 
         fail(DLG_OVERFLOW, "radix_sort: more than 2^32-1 tuples need 8-bit digits");
     u32 h[4];
     if (bounds) std::memcpy(h, bounds, sizeof(h));
-    else tuple_bounds(ctx, data.p, n, h);
+    else tuple_bounds(ctx, in, n, h);
     RadixKey key;
     key.min_hi = h[0];
     key.min_lo = h[2];
     key.vb = key_only ? 0u : (u32)bit_width(h[3] - h[2]);   // key_only: a stable sort by key alone
     key.shift = 0;
     int total_bits = (int)key.vb + bit_width(h[1] - h[0]);
-    if (total_bits == 0) return;  // all equal
-    tmp.ensure(n);
-    u64 *src = data.p, *dst = tmp.p;
+    if (total_bits == 0) return in;  // all equal
     switch (bits) {
-        case 4: radix_passes_sized<4>(ctx, src, dst, n, key, total_bits); break;
-        case 5: radix_passes_sized<5>(ctx, src, dst, n, key, total_bits); break;
-        case 6: radix_passes_sized<6>(ctx, src, dst, n, key, total_bits); break;
-        case 7: radix_passes_sized<7>(ctx, src, dst, n, key, total_bits); break;
-        default: radix_passes_sized<8>(ctx, src, dst, n, key, total_bits); break;
+        case 4: return radix_passes_sized<4>(ctx, in, a, b, n, key, total_bits);
+        case 5: return radix_passes_sized<5>(ctx, in, a, b, n, key, total_bits);
+        case 6: return radix_passes_sized<6>(ctx, in, a, b, n, key, total_bits);
+        case 7: return radix_passes_sized<7>(ctx, in, a, b, n, key, total_bits);
+        default: return radix_passes_sized<8>(ctx, in, a, b, n, key, total_bits);
     }
-    if (src != data.p) data.swap(tmp);   // result is in the other buffer: swap ownership
+}
+
+void radix_sort(dlg_ctx *ctx, DBuf<u64> &data, u64 n, DBuf<u64> &tmp, int bits, const u32 *bounds,
+                bool key_only) {
+    if (n < 2) return;
+    if (n > SORT_SMALL_MAX) tmp.ensure(n);   // the one-workgroup sort works in place
+    const u64 *r = radix_from(ctx, data.p, n, tmp.p, data.p, bits, bounds, key_only);
+    if (r != data.p) data.swap(tmp);   // result is in the other buffer: swap ownership
+}
+
+void radix_sort_into(dlg_ctx *ctx, const u64 *in, u64 n, DBuf<u64> &out, DBuf<u64> &tmp) {
+    out.ensure(n ? n : 1);
+    if (n > SORT_SMALL_MAX) tmp.ensure(n);
+    const u64 *r = radix_from(ctx, in, n, tmp.p, out.p, 0, nullptr, false);
+    if (r == in) copy_u64(ctx, out.p, in, n);
+    else if (r != out.p) out.swap(tmp);
 }
 
 void radix_sort(dlg_ctx *ctx, u64 *data, u64 n, DBuf<u64> &tmp, int bits, bool key_only) {
-    DBuf<u64> view(ctx);
-    view.p = data;          // borrowed: released without returning it to the pool
-    view.cap = n;
-    radix_sort(ctx, view, n, tmp, bits, nullptr, key_only);
-    if (view.p != data) {   // sorted copy ended in tmp's old block; bring it back
-        copy_u64(ctx, data, view.p, n);
-        tmp.swap(view);     // tmp owns that block again
-    }
-    view.p = nullptr;
-    view.cap = 0;
+    if (n < 2) return;
+    if (n > SORT_SMALL_MAX) tmp.ensure(n);
+    const u64 *r = radix_from(ctx, data, n, tmp.p, data, bits, nullptr, key_only);
+    if (r != data) copy_u64(ctx, data, r, n);   // sorted copy ended in tmp; bring it back
+}
+
+u64 sort_unique(dlg_ctx *ctx, u64 *data, u64 n) {
+    if (n == 0) return 0;
+    if (n <= SORT_SMALL_MAX) return sort_unique_small(ctx, data, n, data);
+    DBuf<u64> tmp(ctx, n);
+    const u64 *r = radix_from(ctx, data, n, tmp.p, data, 0, nullptr, false);
+    if (r != data) return select(ctx, SEL_UNIQUE, r, n, nullptr, 0, data);   // compacted straight back
+    const u64 k = select(ctx, SEL_UNIQUE, data, n, nullptr, 0, tmp.p);
+    copy_u64(ctx, data, tmp.p, k);
+    return k;
 }
 
 // =============================================================== select
@@ -944,24 +1148,9 @@ __device__ __forceinline__ bool found_sorted(const u64 *a, u64 lo, u64 hi, u64 x
 }
 
 template <int MODE>
-__global__ __launch_bounds__(SEL_T) void select_count_k(const u64 *in, u64 n, const u64 *other,
-                                                        u64 no, u64 *flags, u64 *bsum) {
-    __shared__ u64 s_lo, s_hi;
+__global__ __launch_bounds__(SEL_T) void select_count_k(const u64 *in, u64 n, u64 *flags, u64 *bsum) {
     __shared__ u64 sc[SEL_T / WAVE + 1];
     const u64 base = (u64)blockIdx.x * SEL_TILE;
-    constexpr bool NEED_OTHER = (MODE == SEL_UNIQUE_NOT_IN || MODE == SEL_NOT_IN);
-    if (NEED_OTHER) {
-        if (threadIdx.x < WAVE) {   // the first wave finds the tile's range of `other`
-            const u64 last = base + SEL_TILE - 1 < n ? base + SEL_TILE - 1 : n - 1;
-            const u64 lo = wave_lower_bound(other, 0, no, in[base]);
-            const u64 hi = wave_upper_bound(other, lo, no, in[last]);
-            if (threadIdx.x == 0) {
-                s_lo = lo;
-                s_hi = hi;
-            }
-        }
-        __syncthreads();
-    }
     u64 c = 0;
 #pragma unroll
     for (int r = 0; r < SEL_I; r++) {
@@ -971,20 +1160,106 @@ __global__ __launch_bounds__(SEL_T) void select_count_k(const u64 *in, u64 n, co
             u64 x = in[idx];
             if (MODE == SEL_KEY_HEAD) {
                 keep = idx == 0 || tkey(in[idx - 1]) != tkey(x);
-            } else if (MODE == SEL_NOT_IN) {
-                keep = !found_sorted(other, s_lo, s_hi, x);
             } else if (MODE == SEL_NODIAG) {
                 keep = tkey(x) != tval(x);
             } else {
                 keep = idx == 0 || in[idx - 1] != x;
                 if (MODE == SEL_UNIQUE_NODIAG) keep = keep && tkey(x) != tval(x);
-                if (MODE == SEL_UNIQUE_NOT_IN && keep) keep = !found_sorted(other, s_lo, s_hi, x);
             }
         }
         u64 m = __ballot(keep);
         u64 w0 = base + (u64)r * SEL_T + (threadIdx.x & ~(WAVE - 1));
         if ((threadIdx.x & (WAVE - 1)) == 0 && w0 < n) flags[w0 / WAVE] = m;
         c += keep ? 1 : 0;
+    }
+    u64 tot;
+    block_exclusive_scan<u64>(c, sc, &tot);
+    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
+}
+
+// The same flags for the modes that drop what sorted `other` holds (UNIQUE:
+// equal runs too).  The tile goes by SEL_PARTS parts; a part's stretch of
+// `other` begins at split[part] (select_split_k) and, up to SEL_STAGE elements,
+// comes into LDS with coalesced reads (all of them in flight together) and is
+// searched there; a larger one is searched in global memory.
+// 16M elements against 33M: 86 us (4.6 TB/s) against 291 us with every search in
+// global memory, each tile's range found by a wave; 176 us with the staging's
+// loads one after the other.
+constexpr int SEL_PARTS = 4, SEL_PART = SEL_TILE / SEL_PARTS, SEL_PER = SEL_I / SEL_PARTS;
+constexpr u32 SEL_BATCH = 8;
+constexpr u64 SEL_STAGE = SEL_BATCH * SEL_T;
+
+// split[p] = the first of `other` not below in[p SEL_PART], and, past the last
+// part, the first above in[n - 1]: one thread each (a wave's 64 pivots per step
+// would read 64 lines per search).
+__global__ __launch_bounds__(256) void select_split_k(const u64 *in, u64 n, const u64 *other, u64 no, u64 parts, u64 *split) {
+    const u64 p = (u64)blockIdx.x * 256 + threadIdx.x;
+    if (p < parts) split[p] = lower_bound_u64(other, 0, no, in[p * SEL_PART]);
+    else if (p == parts) split[p] = upper_bound_u64(other, 0, no, in[n - 1]);
+}
+
+template <bool UNIQUE>
+__global__ __launch_bounds__(SEL_T) void select_minus_k(const u64 *in, u64 n, const u64 *other, const u64 *split, u64 parts,
+                                                        u64 *flags, u64 *bsum) {
+    __shared__ u64 s_other[SEL_STAGE];
+    __shared__ u64 sc[SEL_T / WAVE + 1];
+    const u64 base = (u64)blockIdx.x * SEL_TILE;
+    u64 c = 0;
+    for (int part = 0; part < SEL_PARTS; part++) {
+        const u64 p = (u64)blockIdx.x * SEL_PARTS + part;
+        if (p >= parts) break;   // block-uniform
+        const u64 lo = split[p];
+        // the next part's first element may be this part's last one too
+        const u64 hi = split[p + 1] + (p + 1 < parts && split[p + 1] < split[parts] ? 1 : 0);
+        const bool staged = hi - lo <= SEL_STAGE;
+        const u64 i0 = base + (u64)part * SEL_PART + threadIdx.x;
+        u64 x[SEL_PER], before[SEL_PER];
+#pragma unroll
+        for (int r = 0; r < SEL_PER; r++) {
+            const u64 i = i0 + (u64)r * SEL_T;
+            x[r] = i < n ? in[i] : 0ull;
+            if (UNIQUE) before[r] = i > 0 && i < n ? in[i - 1] : 0ull;
+        }
+        const u32 m = (u32)(hi - lo);
+        if (staged && m) {
+            u64 v[SEL_BATCH];
+#pragma unroll
+            for (u32 k = 0; k < SEL_BATCH; k++)
+                if (k * SEL_T < m) v[k] = other[lo + min(k * SEL_T + threadIdx.x, m - 1)];   // uniform
+#pragma unroll
+            for (u32 k = 0; k < SEL_BATCH; k++)
+                if (k * SEL_T < m) s_other[k * SEL_T + threadIdx.x] = v[k];
+        }
+        __syncthreads();
+        bool found[SEL_PER];
+        if (staged) {
+            u32 at[SEL_PER];
+#pragma unroll
+            for (int r = 0; r < SEL_PER; r++) at[r] = 0;
+            for (u32 len = m; len > 1; len -= len / 2) {   // block-uniform: the searches step together
+                const u32 half = len / 2;
+                u64 v[SEL_PER];
+#pragma unroll
+                for (int r = 0; r < SEL_PER; r++) v[r] = s_other[at[r] + half - 1];
+#pragma unroll
+                for (int r = 0; r < SEL_PER; r++) at[r] += v[r] < x[r] ? half : 0u;
+            }
+#pragma unroll
+            for (int r = 0; r < SEL_PER; r++) found[r] = m && s_other[at[r]] == x[r];
+        } else {
+#pragma unroll
+            for (int r = 0; r < SEL_PER; r++) found[r] = found_sorted(other, lo, hi, x[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < SEL_PER; r++) {
+            const u64 i = i0 + (u64)r * SEL_T;
+            const bool keep = i < n && !found[r] && (!UNIQUE || i == 0 || before[r] != x[r]);
+            const u64 bal = __ballot(keep);
+            const u64 w0 = i & ~(u64)(WAVE - 1);
+            if ((threadIdx.x & (WAVE - 1)) == 0 && w0 < n) flags[w0 / WAVE] = bal;
+            c += keep;
+        }
+        __syncthreads();   // the stretch is searched: the next part's comes in
     }
     u64 tot;
     block_exclusive_scan<u64>(c, sc, &tot);
@@ -1022,6 +1297,87 @@ __global__ __launch_bounds__(SEL_T) void select_scatter_k(const u64 *in, u64 n, 
     }
 }
 
+// The whole compaction by one workgroup, for up to SORT_SMALL_MAX elements:
+// flags, scan, scatter and the count's publication in one launch.  A thread
+// takes 8 consecutive elements; its searches of `other` step together.
+template <int MODE>
+__global__ __launch_bounds__(1024) void select_small_k(const u64 *in, u32 n, const u64 *other, u64 no, void *out, u64 *host,
+                                                       u64 seq) {
+    constexpr int I = (int)(SORT_SMALL_MAX / 1024);
+    constexpr bool NEED_OTHER = (MODE == SEL_UNIQUE_NOT_IN || MODE == SEL_NOT_IN);
+    __shared__ u64 s_piv[NEED_OTHER ? 1024 : 1];
+    __shared__ u32 sc[1024 / WAVE + 1];
+    const u64 stride = (no + 1023) / 1024;   // `other` in 1024 segments, their last elements in LDS
+    if (NEED_OTHER) {
+        const u64 e = ((u64)threadIdx.x + 1) * stride;
+        s_piv[threadIdx.x] = other[(e < no ? e : no) - 1];
+        __syncthreads();
+    }
+    const u32 i0 = threadIdx.x * I;
+    u64 x[I];
+#pragma unroll
+    for (int r = 0; r < I; r++) x[r] = i0 + r < n ? in[i0 + r] : 0ull;
+    const u64 before = i0 > 0 && i0 < n ? in[i0 - 1] : 0ull;
+    u32 keep = 0;
+#pragma unroll
+    for (int r = 0; r < I; r++) {
+        if (i0 + r >= n) continue;
+        const u64 prev = r ? x[r ? r - 1 : 0] : before;
+        const bool first = i0 + r == 0;
+        bool k = true;
+        if (MODE == SEL_KEY_HEAD) k = first || tkey(prev) != tkey(x[r]);
+        else if (MODE == SEL_UNIQUE || MODE == SEL_UNIQUE_NODIAG || MODE == SEL_UNIQUE_NOT_IN) k = first || prev != x[r];
+        if (MODE == SEL_UNIQUE_NODIAG || MODE == SEL_NODIAG) k = k && tkey(x[r]) != tval(x[r]);
+        keep |= k ? 1u << r : 0u;
+    }
+    if (NEED_OTHER) {
+        // each element's segment among the pivots in LDS, then its place in the
+        // segment: log2(no / 1024) dependent reads of global memory instead of log2(no)
+        u64 lo[I];
+#pragma unroll
+        for (int r = 0; r < I; r++) {
+            u32 a = 0;   // pivots below x
+#pragma unroll
+            for (u32 h = 512; h; h >>= 1) a += s_piv[a + h - 1] < x[r] ? h : 0u;
+            lo[r] = (u64)a * stride;   // the last pivot below x may be the last of all: then x is in no segment
+        }
+        for (u64 len = stride; len > 1; len -= len / 2) {   // block-uniform: the searches step together
+            const u64 half = len / 2;
+            u64 v[I];
+#pragma unroll
+            for (int r = 0; r < I; r++) v[r] = lo[r] + half - 1 < no ? other[lo[r] + half - 1] : ~0ull;
+#pragma unroll
+            for (int r = 0; r < I; r++) lo[r] += v[r] < x[r] ? half : 0;
+        }
+#pragma unroll
+        for (int r = 0; r < I; r++)
+            if (lo[r] < no && other[lo[r]] == x[r]) keep &= ~(1u << r);
+    }
+    u32 total;
+    u32 at = block_exclusive_scan<u32>((u32)__popc(keep), sc, &total);   // every read is done before the first write
+#pragma unroll
+    for (int r = 0; r < I; r++)
+        if ((keep >> r) & 1u) {
+            if (MODE == SEL_KEY_HEAD) ((u32 *)out)[at++] = i0 + r;
+            else ((u64 *)out)[at++] = x[r];
+        }
+    if (threadIdx.x == 0) {
+        host[0] = total;
+        __threadfence_system();
+        *(volatile u64 *)(host + dlg_ctx::MAPPED_SEQ) = seq;
+        __threadfence_system();
+    }
+}
+
+template <int MODE>
+static u64 select_small(dlg_ctx *ctx, const u64 *in, u64 n, const u64 *other, u64 n_other, void *out) {
+    const u64 seq = ++ctx->mapped_seq;
+    DLG_LAUNCH(ctx, DLG_K_SELECT, 16.0 * n, select_small_k<MODE>, 1, 1024, 0, in, (u32)n, other, n_other, out,
+               ctx->mapped_dev(seq), seq);
+    ctx->wait_mapped(seq);
+    return ((const volatile u64 *)ctx->mapped_host(seq))[0];
+}
+
 u64 select(dlg_ctx *ctx, int mode, const u64 *in, u64 n, const u64 *other, u64 n_other,
            void *out) {
     if (n == 0) return 0;
@@ -1031,37 +1387,42 @@ u64 select(dlg_ctx *ctx, int mode, const u64 *in, u64 n, const u64 *other, u64 n
         if (out != (const void *)in) copy_u64(ctx, (u64 *)out, in, n);
         return n;
     }
+    if (n <= SORT_SMALL_MAX) switch (mode) {
+        case SEL_UNIQUE: return select_small<SEL_UNIQUE>(ctx, in, n, other, n_other, out);
+        case SEL_UNIQUE_NODIAG: return select_small<SEL_UNIQUE_NODIAG>(ctx, in, n, other, n_other, out);
+        case SEL_UNIQUE_NOT_IN: return select_small<SEL_UNIQUE_NOT_IN>(ctx, in, n, other, n_other, out);
+        case SEL_NOT_IN: return select_small<SEL_NOT_IN>(ctx, in, n, other, n_other, out);
+        case SEL_KEY_HEAD: return select_small<SEL_KEY_HEAD>(ctx, in, n, other, n_other, out);
+        case SEL_NODIAG: return select_small<SEL_NODIAG>(ctx, in, n, other, n_other, out);
+        default: fail(DLG_INVALID_INPUT, "select: bad mode");
+    }
     u64 nb = (n + SEL_TILE - 1) / SEL_TILE;
     DBuf<u64> flags(ctx, (n + WAVE - 1) / WAVE + 1);
     DBuf<u64> bsum(ctx, nb);
     DBuf<u64> tot(ctx, 1);
-    double rb = 8.0 * n + 8.0 * ((n + 63) / 64);
-    switch (mode) {
-        case SEL_UNIQUE:
-            DLG_LAUNCH(ctx, DLG_K_SELECT, rb, select_count_k<SEL_UNIQUE>, (unsigned)nb, SEL_T, 0,
-                       in, n, other, n_other, flags.p, bsum.p);
-            break;
-        case SEL_UNIQUE_NODIAG:
-            DLG_LAUNCH(ctx, DLG_K_SELECT, rb, select_count_k<SEL_UNIQUE_NODIAG>, (unsigned)nb,
-                       SEL_T, 0, in, n, other, n_other, flags.p, bsum.p);
-            break;
-        case SEL_UNIQUE_NOT_IN:
-            DLG_LAUNCH(ctx, DLG_K_SELECT, rb, select_count_k<SEL_UNIQUE_NOT_IN>, (unsigned)nb,
-                       SEL_T, 0, in, n, other, n_other, flags.p, bsum.p);
-            break;
-        case SEL_NOT_IN:
-            DLG_LAUNCH(ctx, DLG_K_SELECT, rb, select_count_k<SEL_NOT_IN>, (unsigned)nb, SEL_T, 0,
-                       in, n, other, n_other, flags.p, bsum.p);
-            break;
-        case SEL_KEY_HEAD:
-            DLG_LAUNCH(ctx, DLG_K_SELECT, rb, select_count_k<SEL_KEY_HEAD>, (unsigned)nb, SEL_T,
-                       0, in, n, other, n_other, flags.p, bsum.p);
-            break;
-        case SEL_NODIAG:
-            DLG_LAUNCH(ctx, DLG_K_SELECT, rb, select_count_k<SEL_NODIAG>, (unsigned)nb, SEL_T, 0,
-                       in, n, other, n_other, flags.p, bsum.p);
-            break;
-        default: fail(DLG_INVALID_INPUT, "select: bad mode");
+    const double rb = 8.0 * n + 8.0 * ((n + 63) / 64);
+    if (mode == SEL_NOT_IN || mode == SEL_UNIQUE_NOT_IN) {
+        const u64 parts = (n + SEL_PART - 1) / SEL_PART;
+        DBuf<u64> split(ctx, parts + 1);
+        DLG_LAUNCH(ctx, DLG_K_SELECT, 16.0 * parts, select_split_k, grid_for(parts + 1, 256), 256, 0, in, n, other, n_other,
+                   parts, split.p);
+        if (mode == SEL_NOT_IN)
+            DLG_LAUNCH(ctx, DLG_K_SELECT, rb + 8.0 * n_other, select_minus_k<false>, (unsigned)nb, SEL_T, 0, in, n, other,
+                       (const u64 *)split.p, parts, flags.p, bsum.p);
+        else
+            DLG_LAUNCH(ctx, DLG_K_SELECT, rb + 8.0 * n_other, select_minus_k<true>, (unsigned)nb, SEL_T, 0, in, n, other,
+                       (const u64 *)split.p, parts, flags.p, bsum.p);
+    } else {
+        auto go = [&](auto kern) {
+            DLG_LAUNCH(ctx, DLG_K_SELECT, rb, kern, (unsigned)nb, SEL_T, 0, in, n, flags.p, bsum.p);
+        };
+        switch (mode) {
+            case SEL_UNIQUE: go(select_count_k<SEL_UNIQUE>); break;
+            case SEL_UNIQUE_NODIAG: go(select_count_k<SEL_UNIQUE_NODIAG>); break;
+            case SEL_KEY_HEAD: go(select_count_k<SEL_KEY_HEAD>); break;
+            case SEL_NODIAG: go(select_count_k<SEL_NODIAG>); break;
+            default: fail(DLG_INVALID_INPUT, "select: bad mode");
+        }
     }
     scan_blocks(ctx, bsum.p, nb, tot.p);
     u64 total = 0;

@@ -347,9 +347,9 @@ __global__ void wcc_emit_k(const u32 *flags, const u64 *offs, u64 V, const u64 *
 }
 
 static u64 read_counter(dlg_ctx *ctx, WccState &s) {
-    HIPCHK(hipMemcpyAsync(ctx->h_scalars, s.counter.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-    ctx->sync();
-    return *(u32 *)ctx->h_scalars;
+    u32 h = 0;
+    ctx->read_words(s.counter.p, 1, &h);
+    return h;
 }
 
 u64 wcc_first_round(dlg_ctx *ctx, WccState &s, const Index &ix, const u32 *nbr) {
@@ -397,10 +397,7 @@ u64 wcc_round(dlg_ctx *ctx, WccState &s, const Index &ix, const u32 *nbr, u64 nf
                    (const u64 *)s.offs.p, total, nbr, s.L.p, s.mark.p, round, s.nnode.p,
                    s.counter.p);
     }
-    u64 h = 0;
-    HIPCHK(hipMemcpyAsync(ctx->h_scalars, s.counter.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-    ctx->sync();
-    h = *(u32 *)ctx->h_scalars;
+    const u64 h = read_counter(ctx, s);
     if (h) {
         DLG_LAUNCH(ctx, DLG_K_WCC_RELAX, 12.0 * h, wcc_gather_k, sgrid(ctx, h), ctx->block_size, 0,
                    (const u32 *)s.nnode.p, h, (const u32 *)s.L.p, s.flabel.p);
@@ -463,9 +460,7 @@ u64 wcc_relax_tuples(dlg_ctx *ctx, const Index &ix, const u32 *nbr, const u64 *d
                    0, delta, nd, (const u32 *)js.pstart.p, (const u64 *)js.offs.p, total, (const u64 *)ix.rows.p,
                    nbr, ncc, cc, bad.p);
     u32 hb = 0;
-    HIPCHK(hipMemcpyAsync(ctx->h_scalars, bad.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-    ctx->sync();
-    hb = *(u32 *)ctx->h_scalars;
+    ctx->read_words(bad.p, 1, &hb);
     if (hb) fail(DLG_INVALID_INPUT, "dlg_wcc_relax: a join row's node is not in cc (edges not symmetric, or cc "
                                     "not one tuple per key in key order)");
     // cc' keeps cc's node order, so both are sorted: Δ' = cc' minus cc
@@ -499,9 +494,7 @@ u64 wcc_finalize(dlg_ctx *ctx, WccState &s, const Index &ix, DBuf<u64> &out, i64
     DLG_LAUNCH(ctx, DLG_K_WCC_FINAL, 8.0 * V, wcc_comp_flags_k, sgrid(ctx, V), ctx->block_size, 0,
                (const u32 *)ccount.p, V, flags.p, s.counter.p);
     u64 ncomp = scan_u32_u64(ctx, flags.p, V, offs.p);
-    HIPCHK(hipMemcpyAsync(ctx->h_scalars, s.counter.p, 4, hipMemcpyDeviceToHost, ctx->stream));
-    ctx->sync();
-    *largest = (i64) * (u32 *)ctx->h_scalars;
+    *largest = (i64)read_counter(ctx, s);
     out.ensure(ncomp ? ncomp : 1);
     DLG_LAUNCH(ctx, DLG_K_WCC_FINAL, 16.0 * V, wcc_emit_k, sgrid(ctx, V), ctx->block_size, 0,
                (const u32 *)flags.p, (const u64 *)offs.p, V, (const u64 *)ix.rows.p,
@@ -1045,10 +1038,9 @@ int wcc_rounds_graph(dlg_ctx *ctx, WccState &s, const Index &ix, const u32 *nbr,
             if (ctx->prof) ctx->prof_begin();
             HIPCHK(hipGraphLaunch(exec, ctx->stream));
             if (ctx->prof) ctx->prof_end(DLG_K_WCC_RELAX, 0.0);
-            HIPCHK(hipMemcpyAsync(ctx->h_scalars, st, sizeof(WccDev), hipMemcpyDeviceToHost, ctx->stream));
-            ctx->sync();
             WccDev cur;
-            std::memcpy(&cur, ctx->h_scalars, sizeof(cur));
+            static_assert(sizeof(WccDev) <= 8 * dlg_ctx::MAPPED_SEQ, "the state fits a mapped slot");
+            ctx->read_words((const u32 *)st, (int)(sizeof(WccDev) / 4), &cur);
             it = (int)cur.it;
             if (cur.done) break;
         }

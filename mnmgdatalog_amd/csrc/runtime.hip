@@ -290,11 +290,28 @@ void dlg_ctx::wait_mapped(uint64_t seq) {
     std::atomic_thread_fence(std::memory_order_acquire);   // the totals were written before the number
 }
 
-void dlg_ctx::read_scalars(const uint64_t *d, int count, uint64_t *h) {
-    HIPCHK(hipMemcpyAsync(h_scalars, d, sizeof(uint64_t) * count, hipMemcpyDeviceToHost, stream));
-    HIPCHK(hipStreamSynchronize(stream));
-    std::memcpy(h, h_scalars, sizeof(uint64_t) * count);
+// A few words to a mapped slot, its number after them.
+__global__ static void read_words_k(const uint32_t *d, int words, uint32_t *host, uint64_t seq) {
+    if ((int)threadIdx.x < words) host[threadIdx.x] = d[threadIdx.x];
+    __threadfence_system();
+    if (threadIdx.x == 0) {   // the wave's stores above are done
+        ((volatile uint64_t *)host)[dlg_ctx::MAPPED_SEQ] = seq;
+        __threadfence_system();
+    }
 }
+
+// A copy and a stream synchronisation took about 20 us of a fixpoint's every
+// read-back; a one-wave kernel that writes the mapped slot, waited for by
+// spinning, takes about 8.
+void dlg_ctx::read_words(const uint32_t *d, int words, void *h) {
+    const uint64_t seq = ++mapped_seq;
+    hipLaunchKernelGGL(read_words_k, dim3(1), dim3(64), 0, stream, d, words, (uint32_t *)mapped_dev(seq), seq);
+    HIPCHK(hipGetLastError());
+    wait_mapped(seq);
+    std::memcpy(h, (const void *)mapped_host(seq), 4 * (size_t)words);
+}
+
+void dlg_ctx::read_scalars(const uint64_t *d, int count, uint64_t *h) { read_words((const uint32_t *)d, 2 * count, h); }
 
 // ------------------------------------------------------------------ C ABI
 extern "C" {
@@ -317,7 +334,6 @@ dlg_status dlg_ctx_create(int device, dlg_ctx **out) {
         c->arch = prop.gcnArchName;
         HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         c->pool = new Pool(device);
-        HIPCHK(hipHostMalloc((void **)&c->h_scalars, 64 * sizeof(uint64_t), hipHostMallocDefault));
         const size_t mw = (size_t)dlg_ctx::MAPPED_WORDS * dlg_ctx::MAPPED_SLOTS;
         HIPCHK(hipHostMalloc((void **)&c->h_mapped, mw * sizeof(uint64_t), hipHostMallocMapped));
         std::memset(c->h_mapped, 0, mw * sizeof(uint64_t));   // no sequence number yet
@@ -344,7 +360,6 @@ void dlg_ctx_destroy(dlg_ctx *c) {
     }
     for (auto e : c->event_free) (void)hipEventDestroy(e);
     delete c->pool;
-    if (c->h_scalars) (void)hipHostFree(c->h_scalars);
     if (c->h_mapped) (void)hipHostFree(c->h_mapped);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     if (c->counted) host_contexts(-1);
