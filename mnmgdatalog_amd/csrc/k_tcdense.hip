@@ -65,7 +65,7 @@ struct TdArgs {
     const u32 *nlong;
     unsigned long long *cnt; // TD_SETS sets of nslots slots: new tuples, their next join rows
     u32 *iters;              // per block: the first round without new tuples
-    u32 *done;               // a round found nothing: later ones do nothing
+    u32 *done;               // the round that published an empty one (0: none yet): later rounds do nothing
     u32 nslots, nblk, ntaskwg, per;   // task workgroups; tasks per sub-group
 };
 
@@ -129,6 +129,13 @@ __device__ __forceinline__ u32 td_update(uint4 acc, u32 *F, u32 *dn, u64 at, boo
     return (u32)(__popc(n.x) + __popc(n.y) + __popc(n.z) + __popc(n.w));
 }
 
+// Whether round `round` has work.  Its own publisher may set `done` while it
+// runs, which must not part a workgroup's waves: only earlier rounds' count.
+__device__ __forceinline__ bool td_live(const TdArgs &a, u32 round) {
+    const u32 d = *(volatile const u32 *)a.done;
+    return d == 0u || d >= round;
+}
+
 // Round `round` (its predecessor's totals published first: those of round 0
 // are the edges'), or only the publication (`publish_only`).
 __global__ __launch_bounds__(TD_T) void td_round_k(TdArgs a, const u32 *dc, u32 *dn, const unsigned char *fc,
@@ -152,7 +159,7 @@ __global__ __launch_bounds__(TD_T) void td_round_k(TdArgs a, const u32 *dc, u32 
             next[(u64)i * TD_SLOT + 1] = 0;
         }
         if (was_done) c = w = 0;
-    } else if (*a.done == 0u && !publish_only) {
+    } else if (td_live(a, round) && !publish_only) {
         const u32 wg = blockIdx.x - 1;
         if (wg < a.ntaskwg) {
             const u32 b = a.wgblk ? a.wgblk[wg] : 0u;
@@ -233,7 +240,7 @@ __global__ __launch_bounds__(TD_T) void td_round_k(TdArgs a, const u32 *dc, u32 
         w += s_w[i];
     }
     if (blockIdx.x == 0) {
-        if (round > 1 && c == 0) *a.done = 1u;
+        if (round > 1 && c == 0 && *a.done == 0u) *a.done = round;
         host[0] = c;
         host[1] = w;
         __threadfence_system();

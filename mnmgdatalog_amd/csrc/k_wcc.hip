@@ -534,7 +534,7 @@ static_assert(WD_DEPTH + 2 <= dlg_ctx::MAPPED_SLOTS, "every queued round has a m
 struct WdState {
     unsigned long long cnt[WD_SETS][WD_SLOTS][WD_LINE];   // lowered nodes, by round and slice
     u64 prev;    // |Δ| of the round before (wcc.cu:236-242)
-    u32 done;    // the stop rule fired (every instance's)
+    u32 done;    // the round that published the stop rule's firing, every instance's (0: not yet)
     u32 nmid, nhub;   // middle nodes, hub segments
 };
 
@@ -635,14 +635,18 @@ __device__ __forceinline__ void wd_publish(WdState *st, const WdInst &in, u32 ro
         }
         if (live) atomicAdd(&s_live, live);
         __syncthreads();
-        if (threadIdx.x == 0) host[1] = st->done = s_live == 0;
+        if (threadIdx.x == 0) {
+            if (s_live == 0 && !st->done) st->done = round;
+            host[1] = st->done != 0;
+        }
     } else if (threadIdx.x < WAVE) {   // WD_SLOTS == WAVE: a slice per lane
         u64 c = st->cnt[(round - 1) % WD_SETS][threadIdx.x][0];
         st->cnt[(round + 1) % WD_SETS][threadIdx.x][0] = 0;
 #pragma unroll
         for (int d = WAVE / 2; d > 0; d >>= 1) c += __shfl_xor(c, d, WAVE);
         if (threadIdx.x == 0) {
-            host[1] = st->done = st->done || c == st->prev;
+            if (c == st->prev && !st->done) st->done = round;
+            host[1] = st->done != 0;
             st->prev = c;
         }
     }
@@ -666,7 +670,9 @@ __global__ __launch_bounds__(WD_T) void wd_round_k(const u32 *gstart, const u32 
         if (round > 1) wd_publish<MULTI>(st, in, round, host, seq);
         return;
     }
-    if (publish_only || st->done) return;
+    // its own publisher may set `done` meanwhile, which must not part a workgroup's waves: earlier rounds' only
+    const u32 stop = *(volatile const u32 *)&st->done;
+    if (publish_only || (stop && stop < round)) return;
     const u32 wg = blockIdx.x - 1, nthr = (u32)((V + WD_T - 1) / WD_T), nwav = (nmid + WD_T / WAVE - 1) / (WD_T / WAVE);
     bool low = false;   // this thread lowered a node, of instance `inst`
     u32 inst = 0;
@@ -713,9 +719,9 @@ __global__ __launch_bounds__(WD_T) void wd_round_k(const u32 *gstart, const u32 
             inst = in.of[i];
             if (threadIdx.x == 0) s_v[0] = in.done[inst];
             __syncthreads();
-            const bool stop = s_v[0] != 0;
+            const bool fin = s_v[0] != 0;
             __syncthreads();
-            if (stop) return;
+            if (fin) return;
         }
         u32 m = 0xffffffffu;
         for (u32 e = h.y + threadIdx.x; e < end; e += 4 * WD_T) {
