@@ -412,7 +412,8 @@ struct Bitmap {
 };
 // Geometry for ids [lo, hi]; the map is cleared unless `clear` is false (its
 // padding always is).
-void bitmap_init(dlg_ctx *ctx, Bitmap &bm, u32 lo, u32 hi, bool transposed, bool clear = true);
+// Rows are a multiple of `align` words.
+void bitmap_init(dlg_ctx *ctx, Bitmap &bm, u32 lo, u32 hi, bool transposed, bool clear = true, u64 align = 1);
 // The single join R(a, b), R(b, c) straight into a row-major map (row c, bit
 // a), from `rows` = R keyed by its second column, sorted, n rows, with dense
 // offsets over the map's id range (W + 1 entries).  Every row is written.
@@ -576,6 +577,15 @@ void sg_rows_setup(dlg_ctx *ctx, const Index &ix, const Bitmap &F, SgRows &sr);
 // row-major map R, then N = (T ⋈ E) \ F: new bits into F and D (both
 // transposed); R is left empty.  Returns |N|; *raw += both joins' rows.
 u64 sg_rows_round(dlg_ctx *ctx, SgRows &sr, Bitmap &R, Bitmap &F, Bitmap &D, u64 *raw);
+
+// ------------------------------------------------------------- SG two row ORs (k_sgor.hip)
+// SG's rounds over id ranges that it takes (their maps are addressed by 32-bit
+// byte offsets, a row of zeros behind them: up to about 185,000 ids): F and D hold the base
+// rule's tuples (the same, rows of a multiple of 4 words); `edges` are the
+// distinct edges, released once read.  F is left complete, D's contents are lost; its size to
+// *total, the rounds' join rows added to *raw; returns the round count.
+constexpr bool sg_or_takes(u64 W) { return W * ((W + 127) / 128 * 16) + 16 <= 1ull << 32; }
+int sg_or_run(dlg_ctx *ctx, DBuf<u64> &edges, u64 n, Bitmap &F, Bitmap &D, int max_it, u64 *total, u64 *raw);
 
 // ------------------------------------------------------------- hash set (k_hashset.hip)
 struct HashSet {

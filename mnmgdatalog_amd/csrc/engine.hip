@@ -459,14 +459,29 @@ void sg_fixpoint(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, Phas
     int it = 0;
     if (use_bitmap(o, ne, ib)) {
         // F, the round's T and the round's N as bitmaps; both joins of a
-        // round are row operations on them (k_sgrows.hip), Δ never leaves its
-        // map D.  The base rule's rows go straight into F and D (k_bitmap.hip).
+        // round are row operations on them, Δ never leaves its map D.  Ranges
+        // that k_sgor.hip addresses take its row ORs (faster on every input
+        // tried); wider ones, and runs whose every round is handed out, the
+        // row kernels of k_sgrows.hip.  The base rule's rows go straight into F and D (k_bitmap.hip).
         // SG is symmetric (both rules are), so F equals its transpose and is
         // emitted without a sort.
         Bitmap F(ctx), R(ctx), D(ctx);
-        bitmap_init(ctx, F, ib[0], ib[1], true);
+        const bool two_ors = !hook && sg_or_takes((u64)(ib[1] - ib[0]) + 1);
+        bitmap_init(ctx, F, ib[0], ib[1], true, true, two_ors ? 4 : 1);
+        bitmap_init(ctx, D, ib[0], ib[1], true, true, two_ors ? 4 : 1);
+        if (two_ors) {   // both joins of a round as row ORs (k_sgor.hip)
+            if (!ix.sorted) index_dense(ctx, ix, F.lo, F.W);
+            u64 raw = 0, total = 0;
+            pc.mark(DLG_PH_JOIN);
+            bitmap_join_mark(ctx, ix, edge.p, ne, js, DLG_PROJ_HV_PV, true, F, &D, &raw);   // base (y, x)
+            out.iterations = sg_or_run(ctx, edge, ne, F, D, o.max_it, &total, &raw);
+            pc.mark(DLG_PH_FINAL);
+            out.raw += (i64)raw;
+            out.nfull = total;
+            bitmap_emit(ctx, F, out.full, total, true);
+            return;
+        }
         bitmap_init(ctx, R, ib[0], ib[1], false);
-        bitmap_init(ctx, D, ib[0], ib[1], true);
         SgRows sr(ctx);
         sg_rows_setup(ctx, ix, F, sr);
         if (!ix.sorted) index_dense(ctx, ix, F.lo, F.W);   // the joins' count pass reads offsets

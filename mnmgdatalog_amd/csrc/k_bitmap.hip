@@ -472,10 +472,10 @@ __global__ __launch_bounds__(BE_T) void bm_emit_k(u32 *words, const u64 *bpre, u
     }
 }
 
-void bitmap_init(dlg_ctx *ctx, Bitmap &bm, u32 lo, u32 hi, bool transposed, bool clear) {
+void bitmap_init(dlg_ctx *ctx, Bitmap &bm, u32 lo, u32 hi, bool transposed, bool clear, u64 align) {
     bm.lo = lo;
     bm.W = (u64)(hi - lo) + 1;
-    bm.wpr = (bm.W + 31) / 32;
+    bm.wpr = ((bm.W + 31) / 32 + align - 1) / align * align;
     bm.S = bm.wpr * 32;
     bm.nwords = bm.W * bm.wpr;
     bm.nbits = bm.nwords * 32;

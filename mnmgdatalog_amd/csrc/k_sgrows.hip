@@ -1,4 +1,5 @@
-// k_sgrows.hip -- a round of SG as row operations on bitmaps.
+// k_sgrows.hip -- a round of SG as row operations on bitmaps: for id ranges wider
+// than k_sgor.hip takes, and for runs whose every round is handed out.
 //
 // A round of SG (sg.cu:300-375) derives
 //     T(b, x) = Δ(a, b) ⋈ edge(a, x)            (the round's T map R, row-major: row b)
