@@ -580,12 +580,20 @@ u64 sg_rows_round(dlg_ctx *ctx, SgRows &sr, Bitmap &R, Bitmap &F, Bitmap &D, u64
 
 // ------------------------------------------------------------- SG two row ORs (k_sgor.hip)
 // SG's rounds over id ranges that it takes (their maps are addressed by 32-bit
-// byte offsets, a row of zeros behind them: up to about 185,000 ids): F and D hold the base
-// rule's tuples (the same, rows of a multiple of 4 words); `edges` are the
-// distinct edges, released once read.  F is left complete, D's contents are lost; its size to
-// *total, the rounds' join rows added to *raw; returns the round count.
+// byte offsets, a row of zeros behind them: up to about 185,000 ids).
 constexpr bool sg_or_takes(u64 W) { return W * ((W + 127) / 128 * 16) + 16 <= 1ull << 32; }
-int sg_or_run(dlg_ctx *ctx, DBuf<u64> &edges, u64 n, Bitmap &F, Bitmap &D, int max_it, u64 *total, u64 *raw);
+struct SgOr {   // adjacency, the map T, flags and counters
+    DBuf<u64> zero, off;
+    DBuf<unsigned char> df;
+    DBuf<u32> pred, list, T;
+    explicit SgOr(dlg_ctx *c) : zero(c), off(c), df(c), pred(c), list(c), T(c) {}
+};
+// From the n distinct edges, for F's geometry (rows of a multiple of 4 words).
+void sg_or_setup(dlg_ctx *ctx, const u64 *edges, u64 n, const Bitmap &F, SgOr &so);
+// F and D hold the base rule's tuples (the same).  F is left complete, D's
+// contents are lost; F's size to *total, the rounds' join rows added to *raw;
+// returns the round count.
+int sg_or_run(dlg_ctx *ctx, SgOr &so, Bitmap &F, Bitmap &D, int max_it, u64 *total, u64 *raw);
 
 // ------------------------------------------------------------- hash set (k_hashset.hip)
 struct HashSet {

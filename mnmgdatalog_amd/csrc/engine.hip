@@ -466,30 +466,39 @@ void sg_fixpoint(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, Phas
         // SG is symmetric (both rules are), so F equals its transpose and is
         // emitted without a sort.
         Bitmap F(ctx), R(ctx), D(ctx);
-        const bool two_ors = !hook && sg_or_takes((u64)(ib[1] - ib[0]) + 1);
-        bitmap_init(ctx, F, ib[0], ib[1], true, true, two_ors ? 4 : 1);
-        bitmap_init(ctx, D, ib[0], ib[1], true, true, two_ors ? 4 : 1);
-        if (two_ors) {   // both joins of a round as row ORs (k_sgor.hip)
-            if (!ix.sorted) index_dense(ctx, ix, F.lo, F.W);
-            u64 raw = 0, total = 0;
-            pc.mark(DLG_PH_JOIN);
-            bitmap_join_mark(ctx, ix, edge.p, ne, js, DLG_PROJ_HV_PV, true, F, &D, &raw);   // base (y, x)
-            out.iterations = sg_or_run(ctx, edge, ne, F, D, o.max_it, &total, &raw);
+        SgOr so(ctx);
+        bool two_ors = !hook && sg_or_takes((u64)(ib[1] - ib[0]) + 1);
+        const u64 align = two_ors ? 4 : 1;
+        bitmap_init(ctx, F, ib[0], ib[1], true, true, align);
+        bitmap_init(ctx, D, ib[0], ib[1], true, true, align);
+        if (two_ors) {
+            try {
+                sg_or_setup(ctx, edge.p, ne, F, so);
+            } catch (const Error &e) {   // the row kernels may still have enough memory
+                if (e.status != DLG_OUT_OF_MEMORY) throw;
+                two_ors = false;
+                so = SgOr(ctx);
+            }
+        }
+        SgRows sr(ctx);
+        if (!two_ors) {
+            bitmap_init(ctx, R, ib[0], ib[1], false, true, align);
+            sg_rows_setup(ctx, ix, F, sr);
+        }
+        if (!ix.sorted) index_dense(ctx, ix, F.lo, F.W);   // the joins' count pass reads offsets
+        u64 raw = 0, total = 0;
+        pc.mark(DLG_PH_JOIN);
+        bitmap_join_mark(ctx, ix, edge.p, ne, js, DLG_PROJ_HV_PV, true, F, &D, &raw);   // base (y, x)
+        edge.release();
+        if (two_ors) {
+            out.iterations = sg_or_run(ctx, so, F, D, o.max_it, &total, &raw);
             pc.mark(DLG_PH_FINAL);
             out.raw += (i64)raw;
             out.nfull = total;
             bitmap_emit(ctx, F, out.full, total, true);
             return;
         }
-        bitmap_init(ctx, R, ib[0], ib[1], false);
-        SgRows sr(ctx);
-        sg_rows_setup(ctx, ix, F, sr);
-        if (!ix.sorted) index_dense(ctx, ix, F.lo, F.W);   // the joins' count pass reads offsets
-        u64 raw = 0;
-        pc.mark(DLG_PH_JOIN);
-        bitmap_join_mark(ctx, ix, edge.p, ne, js, DLG_PROJ_HV_PV, true, F, &D, &raw);   // base (y, x)
-        edge.release();
-        u64 total = bitmap_count(ctx, D);
+        total = bitmap_count(ctx, D);
         while (true) {
             pc.mark(DLG_PH_JOIN);
             const u64 nn = sg_rows_round(ctx, sr, R, F, D, &raw);   // Δ in D -> T in R -> N in D (and F)

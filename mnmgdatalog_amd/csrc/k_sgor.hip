@@ -28,7 +28,7 @@
 //
 // Whole calls against the row kernels of k_sgrows.hip, which walk Δ's bits and
 // OR each one's successors into a row in LDS: the tetrahedral mesh of 46,656
-// vertices (52 rounds, 2.0e9 tuples) 49 -> 28 ms; meshes of 729 and 64,000
+// vertices (52 rounds, 2.0e9 tuples) 49 -> 26 ms; meshes of 729 and 64,000
 // vertices 0.88 -> 0.53 and 89 -> 38; power-law graphs of 40,000 ids 88 -> 5.5 and
 // of 131,000 ids 195 -> 26; sparse ranges of 175,000 ids (269 rounds) 504 -> 308;
 // a ladder of 3,000 rounds 137 -> 42; none of 30 inputs slower.
@@ -460,46 +460,52 @@ __global__ void so_list_k(const u64 *in, u64 n, u32 *list) {
     for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) list[i] = (u32)in[i];
 }
 
-int sg_or_run(dlg_ctx *ctx, DBuf<u64> &edges, u64 n, Bitmap &F, Bitmap &D, int max_it, u64 *total, u64 *raw) {
-    if (F.wpr % 4 || D.wpr != F.wpr || D.W != F.W || D.lo != F.lo || !sg_or_takes(F.W))
-        fail(DLG_INVALID_INPUT, "sg_or_run: two maps of one geometry, rows of whole uint4s");
+// Words of `zero`: the counters, T's flags, the degrees (in: W, out: W) and `done`.
+constexpr u64 SO_COUNT_WORDS = (u64)SO_SETS * SO_SLOTS * SO_SLOT;
+static u64 so_chunks(const Bitmap &F) { return (F.wpr + SO_CW - 1) / SO_CW; }
+static u64 so_flag_words(const Bitmap &F) { return F.W * ((so_chunks(F) + SO_G - 1) / SO_G) * 2; }
+
+void sg_or_setup(dlg_ctx *ctx, const u64 *edges, u64 n, const Bitmap &F, SgOr &so) {
+    if (F.wpr % 4 || !sg_or_takes(F.W)) fail(DLG_INVALID_INPUT, "sg_or_setup: a map of rows of whole uint4s");
+    const u64 W = F.W, tfw = so_flag_words(F), zw = SO_COUNT_WORDS + tfw + (2 * W + 2) / 2;
+    DBuf<u64> key(ctx, n ? n : 1), tmp(ctx);
+    so.zero.ensure(zw);
+    so.off.ensure(W + 1);
+    so.df.ensure(W * so_chunks(F));
+    so.pred.ensure(n ? n : 1);
+    so.list.ensure(n ? n : 1);
+    so.T.ensure(F.nwords + 4);   // and four words of zeros, read for what is not flagged
+    fill_u32(ctx, so.T.p + F.nwords, 4, 0u);
+    fill_u64(ctx, so.zero.p, zw, 0ull);
+    u32 *indeg = (u32 *)(so.zero.p + SO_COUNT_WORDS + tfw), *outdeg = indeg + W;
+    DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * n, so_hist_k, sgrid(ctx, n), ctx->block_size, 0, edges, n, F.lo, indeg, outdeg);
+    scan_u32_u64_async(ctx, indeg, W, so.off.p, so.off.p + W);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 20.0 * n, so_fill_k, sgrid(ctx, n), ctx->block_size, 0, edges, n, F.lo,
+               (const u64 *)so.off.p, indeg, so.pred.p);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * n, so_key_k, sgrid(ctx, n), ctx->block_size, 0, edges, n, F.lo, key.p);
+    const u32 bounds[4] = {0, ((u32)W - 1) >> SX_LOG, 0, ((u32)W << SX_LOG) - 1};
+    radix_sort(ctx, key, n, tmp, 0, bounds);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * n, so_list_k, sgrid(ctx, n), ctx->block_size, 0, (const u64 *)key.p, n, so.list.p);
+}
+
+int sg_or_run(dlg_ctx *ctx, SgOr &so, Bitmap &F, Bitmap &D, int max_it, u64 *total, u64 *raw) {
+    if (D.wpr != F.wpr || D.W != F.W || D.lo != F.lo) fail(DLG_INVALID_INPUT, "sg_or_run: two maps of one geometry");
     SoArgs a;
     a.W = (u32)F.W;
     a.wpr = (u32)F.wpr;
-    a.nc = (a.wpr + SO_CW - 1) / SO_CW;
+    a.nc = (u32)so_chunks(F);
     const u32 ng = (a.nc + SO_G - 1) / SO_G;
-    const u64 cw = (u64)SO_SETS * SO_SLOTS * SO_SLOT, tfw = (u64)a.W * ng * 2;
-    // one block of cleared words: counters, T's flags, degrees, done
-    const u64 zw = cw + tfw + (2 * (u64)a.W + 2) / 2;
-    DBuf<u64> zero(ctx, zw), off(ctx, (u64)a.W + 1);
-    fill_u64(ctx, zero.p, zw, 0ull);
-    a.cnt = (unsigned long long *)zero.p;
-    a.tf = (unsigned char *)(zero.p + cw);
-    u32 *indeg = (u32 *)(zero.p + cw + tfw), *outdeg = indeg + a.W;
-    a.done = outdeg + a.W;
-    a.outdeg = outdeg;
-    DBuf<unsigned char> df(ctx, (u64)a.W * a.nc);
-    DBuf<u32> pred(ctx, n ? n : 1), list(ctx, n ? n : 1), T(ctx, F.nwords + 4);   // and four words of zeros, read for what is not flagged
-    fill_u32(ctx, T.p + F.nwords, 4, 0u);
+    a.cnt = (unsigned long long *)so.zero.p;
+    a.tf = (unsigned char *)(so.zero.p + SO_COUNT_WORDS);
+    a.outdeg = (const u32 *)(so.zero.p + SO_COUNT_WORDS + so_flag_words(F)) + a.W;
+    a.done = (u32 *)a.outdeg + a.W;
     a.F = F.words.p;
     a.D = D.words.p;
-    a.T = T.p;
-    a.df = df.p;
-    a.off = off.p;
-    a.pred = pred.p;
-    a.list = list.p;
-    DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * n, so_hist_k, sgrid(ctx, n), ctx->block_size, 0, (const u64 *)edges.p, n, F.lo, indeg, outdeg);
-    scan_u32_u64_async(ctx, indeg, a.W, off.p, off.p + a.W);
-    DLG_LAUNCH(ctx, DLG_K_MISC, 20.0 * n, so_fill_k, sgrid(ctx, n), ctx->block_size, 0, (const u64 *)edges.p, n, F.lo, (const u64 *)off.p,
-               indeg, pred.p);
-    {
-        DBuf<u64> key(ctx, n ? n : 1), tmp(ctx);
-        DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * n, so_key_k, sgrid(ctx, n), ctx->block_size, 0, (const u64 *)edges.p, n, F.lo, key.p);
-        edges.release();
-        const u32 bounds[4] = {0, (a.W - 1) >> SX_LOG, 0, (a.W << SX_LOG) - 1};
-        radix_sort(ctx, key, n, tmp, 0, bounds);
-        DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * n, so_list_k, sgrid(ctx, n), ctx->block_size, 0, (const u64 *)key.p, n, list.p);
-    }
+    a.T = so.T.p;
+    a.df = so.df.p;
+    a.off = so.off.p;
+    a.pred = so.pred.p;
+    a.list = so.list.p;
     DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * F.nwords, so_base_k,
                (unsigned)std::min<u64>(((u64)a.W * a.nc * SO_L + SN_T - 1) / SN_T, (u64)ctx->num_cus * 8), SN_T, 0, a);
     const unsigned gx = 1 + so_grid((a.W + SX_R - 1) / SX_R, a.nc), gn = so_grid((a.W + SN_R - 1) / SN_R, ng);
