@@ -530,8 +530,9 @@ struct TcRows {
         : csr_off(c), csr_dst(c), deg(c), ell(c), dy(c), ny(c), ax(c), nx(c), alen(c), nlen(c), rcnt(c), abeg(c), nbeg(c),
           aoff(c), noff(c), rbound(c), bpart(c), brange(c), counters(c) {}
 };
-// CSR of the index's rows; Δ0 = unique(E reversed) grouped by source, its
-// bits set in F (F empty).
+// CSR of the index's rows, and their ELL rows when every degree is small.
+void tc_rows_adjacency(dlg_ctx *ctx, const Index &ix, const RowMap &F, TcRows &tr);
+// After it: Δ0 = unique(E reversed) grouped by source, its bits set in F (F empty).
 void tc_rows_setup(dlg_ctx *ctx, const Index &ix, RowMap &F, TcRows &tr);
 // One round: N = (Δ ⋈ E) \ F into F, Δ = N (grouped).  Returns |N|; *raw += |Δ ⋈ E|.
 u64 tc_rows_round(dlg_ctx *ctx, RowMap &F, TcRows &tr, u64 *raw);
@@ -539,6 +540,12 @@ u64 tc_rows_round(dlg_ctx *ctx, RowMap &F, TcRows &tr, u64 *raw);
 // rounds (0: the default) queued ahead of the host; returns the round count,
 // *total += Σ |N|.
 int tc_rows_run(dlg_ctx *ctx, RowMap &F, TcRows &tr, int max_it, int queue, u64 *total, u64 *raw);
+// Every round to the fixpoint (or max_it > 0 rounds) by lists of words
+// (k_tcrings.hip), for edges that are symmetric as a set and whose adjacency it
+// takes; F (empty before) is left complete; returns the round count, |F| to
+// *total, *raw += the join rows.
+bool tc_rings_takes(const TcRows &tr, const RowMap &F);
+int tc_rings_run(dlg_ctx *ctx, const TcRows &tr, RowMap &F, int max_it, u64 *total, u64 *raw);
 // The current Δ as (z, x) tuples.
 void tc_rows_tuples(dlg_ctx *ctx, const TcRows &tr, DBuf<u64> &out);
 // Locality order of the ids 0 .. W-1 of the edges (src[i], dst[i]) (order.cpp):

@@ -338,8 +338,12 @@ void tc_fixpoint(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, Phas
     DBuf<int32_t> reordered(ctx);
     const u64 W = (u64)(ib[1] - ib[0]) + 1;
     bool reorder = !blocks && !hook && o.reorder != 1 && tc_use_rows(o, n, ib, blocks);
-    if (reorder && o.reorder != 2)
-        reorder = W >= ORDER_MIN_W && n <= ORDER_MAX_ROWS && reciprocal_fraction(ctx, ix) >= ORDER_MIN_RECIPROCAL;
+    double reciprocal = 0.0;
+    if (reorder && o.reorder != 2) {
+        reorder = W >= ORDER_MIN_W && n <= ORDER_MAX_ROWS;
+        if (reorder) reciprocal = reciprocal_fraction(ctx, ix);
+        reorder = reorder && reciprocal >= ORDER_MIN_RECIPROCAL;
+    }
     if (reorder) {
         tc_order(ctx, d_rows, n, ib[0], W, sigma, reordered);
         d_rows = reordered.p;
@@ -358,10 +362,30 @@ void tc_fixpoint(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, Phas
         J.release();
         TcRows tr(ctx);
         pc.mark(DLG_PH_DEDUP);
-        tc_rows_setup(ctx, ix, F, tr);                  // Δ0 = F = unique(E reversed)
-        u64 total = tr.nd, raw = 0;
+        tc_rows_adjacency(ctx, ix, F, tr);
+        u64 total = 0, raw = 0;
+        // an exactly symmetric graph, in a locality order: its rounds as lists of words (k_tcrings.hip), if
+        // there is memory for the lists beside F
+        bool rings = reorder && reciprocal == 1.0 && o.join == 0 && o.queue == 0 && tc_rings_takes(tr, F);
+        if (rings) {
+            pc.mark(DLG_PH_JOIN);
+            try {
+                it = tc_rings_run(ctx, tr, F, o.max_it, &total, &raw);
+            } catch (const Error &e) {
+                if (e.status != DLG_OUT_OF_MEMORY) throw;
+                rings = false;
+                fill_u32(ctx, F.words.p, F.nwords, 0u);
+                total = 0;
+                pc.mark(DLG_PH_DEDUP);
+            }
+        }
+        if (!rings) {
+            tc_rows_setup(ctx, ix, F, tr);              // Δ0 = F = unique(E reversed)
+            total = tr.nd;
+        }
         pc.mark(DLG_PH_JOIN);
-        if (!hook) {
+        if (rings) {
+        } else if (!hook) {
             it = tc_rows_run(ctx, F, tr, o.max_it, o.queue, &total, &raw);   // to |F| unchanged (tc.cu:294-300)
         } else {
             while (true) {

@@ -714,7 +714,7 @@ __global__ void tc_rows_unstall_k(u64 *st) {
     if (threadIdx.x == 0 && blockIdx.x == 0) st[TR_ST_STALL] = 0;
 }
 
-void tc_rows_setup(dlg_ctx *ctx, const Index &ix, RowMap &F, TcRows &tr) {
+void tc_rows_adjacency(dlg_ctx *ctx, const Index &ix, const RowMap &F, TcRows &tr) {
     const u64 W = F.W, n = ix.n;
     // CSR of E over the id range (duplicates kept, as the hash index keeps them)
     tr.deg.ensure(W + 1);
@@ -746,6 +746,10 @@ void tc_rows_setup(dlg_ctx *ctx, const Index &ix, RowMap &F, TcRows &tr) {
         DLG_LAUNCH(ctx, DLG_K_MISC, 20.0 * n, ell_fill_k, sgrid(ctx, n), ctx->block_size, 0, (const u64 *)ix.rows.p,
                    n, (const u64 *)tr.csr_off.p, F.lo, tr.ell.p);
     }
+}
+
+void tc_rows_setup(dlg_ctx *ctx, const Index &ix, RowMap &F, TcRows &tr) {
+    const u64 n = ix.n;
     // Δ0 = unique(E reversed), grouped by source; one segment per source, for good
     DBuf<u64> uniq(ctx, n ? n : 1);
     u64 nu = n ? select(ctx, SEL_UNIQUE, ix.rows.p, n, nullptr, 0, uniq.p) : 0;
