@@ -935,7 +935,7 @@ void bitmap_self_join(dlg_ctx *ctx, const u64 *rows, u64 n, const u64 *dense, Bi
 // writes them at the row's place in a candidate array; a scan of the kept
 // counts then places each row in the output.  Rows with more than SJW_CAP
 // candidates are left to the sorted raw join (the host checks the maximum).
-constexpr int SJW_T = 256, SJW_W = SJW_T / WAVE;
+constexpr int SJW_T = 256, SJW_W = SJW_T / WAVE, SJW_RAW = 4;
 
 __device__ __forceinline__ void sjw_sync() {   // LDS written by some lanes of a wave, read by others
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
@@ -952,9 +952,18 @@ __global__ __launch_bounds__(256) void sj_row_raw_k(const u32 *col, const u64 *d
     for (u64 c = (u64)blockIdx.x * blockDim.x + threadIdx.x; c < W; c += stride) {
         u64 t = 0;
         const u64 p0 = dense[c], p1 = dense[c + 1];
-        for (u64 p = p0; p < p1; p++) {
-            const u32 b = col[p];
-            t += dense[b + 1] - dense[b];
+        for (u64 p = p0; p < p1; p += SJW_RAW) {   // SJW_RAW b's in flight; past the run, its last one again (not counted)
+            u32 b[SJW_RAW];
+            u64 d0[SJW_RAW], d1[SJW_RAW];
+#pragma unroll
+            for (int i = 0; i < SJW_RAW; i++) b[i] = col[min(p + i, p1 - 1)];
+#pragma unroll
+            for (int i = 0; i < SJW_RAW; i++) {
+                d0[i] = dense[b[i]];
+                d1[i] = dense[b[i] + 1];
+            }
+#pragma unroll
+            for (int i = 0; i < SJW_RAW; i++) t += p + i < p1 ? d1[i] - d0[i] : 0;
         }
         rraw[c] = t;
         m = t > m ? t : m;
@@ -983,78 +992,133 @@ __global__ __launch_bounds__(256) void sj_row_raw_k(const u32 *col, const u64 *d
     }
 }
 
-// Bitonic sort, ascending, of SJW_REG * WAVE values held as v[r] = element
-// r WAVE + lane: strides below WAVE exchange with lane ^ j by shuffle, larger
-// ones compare registers of the same lane.
-constexpr int SJW_REG = 4;
-template <int R>
-__device__ __forceinline__ void sjw_sort_regs(u32 (&v)[R], int lane) {
-    constexpr u32 P = R * WAVE;
+// y[lane] = v[lane ^ J] without LDS: quad permutes, row rotation and mirrors (DPP)
+// within 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ u32 sjw_dpp(u32 v) {
+    return (u32)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+template <int J>
+__device__ __forceinline__ u32 sjw_xor(u32 v) {
+    static_assert(J == 1 || J == 2 || J == 4 || J == 8, "within a row of 16 lanes");
+    if constexpr (J == 1) return sjw_dpp<0xb1>(v);                      // quad_perm [1, 0, 3, 2]
+    if constexpr (J == 2) return sjw_dpp<0x4e>(v);                      // quad_perm [2, 3, 0, 1]
+    if constexpr (J == 4) return sjw_dpp<0x141>(sjw_dpp<0x1b>(v));      // ^ 3 (quad_perm [3, 2, 1, 0]), ^ 7 (row_half_mirror)
+    return sjw_dpp<0x128>(v);                                           // row_ror: 8
+}
+// The lanes (as a mask, a constant) that have bit k of their element clear in
+// ascending and set in descending blocks: those keep the smaller of a pair.
+constexpr u64 sjw_low_lanes(u32 base, u32 k, u32 j) {
+    u64 m = 0;
+    for (u32 l = 0; l < 64; l++) m |= (u64)((((base + l) & k) == 0) == ((l & j) == 0)) << l;
+    return m;
+}
+// One stage of the network: block size K, distance J < WAVE, element base + lane in v.
+template <u32 BASE, u32 K, u32 J>
+__device__ __forceinline__ void sjw_stage(u32 &v) {
+    constexpr u64 low = sjw_low_lanes(BASE, K, J);
+    u32 x = v, y;
+    if constexpr (J >= 16) {   // both of a pair in both of its lanes
+        const auto p = J == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false) : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        x = p[0];
+        y = p[1];
+    } else {
+        y = sjw_xor<(int)J>(v);
+    }
+    v = __builtin_amdgcn_inverse_ballot_w64(low) ? min(x, y) : max(x, y);
+}
+template <int R, u32 K, u32 J>
+__device__ __forceinline__ void sjw_stages(u32 (&v)[R]) {
+    if constexpr (J >= (u32)WAVE) {   // registers of the same lane
+        constexpr int M = (int)(J / WAVE);
 #pragma unroll
-    for (u32 k = 2; k <= P; k <<= 1) {
-#pragma unroll
-        for (u32 j = k >> 1; j > 0; j >>= 1) {
-            if (j >= (u32)WAVE) {
-                const u32 m = j / WAVE;
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const int q = r ^ (int)m;
-                    if (q > r) {
-                        const u32 e = (u32)r * WAVE + (u32)lane;
-                        const bool asc = (e & k) == 0;
-                        const u32 x = v[r], y = v[q];
-                        if ((x > y) == asc) {
-                            v[r] = y;
-                            v[q] = x;
-                        }
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < R; r++) {
-                    const u32 e = (u32)r * WAVE + (u32)lane;
-                    const bool asc = (e & k) == 0, low = ((u32)lane & j) == 0;
-                    const u32 y = (u32)__shfl_xor((int)v[r], (int)j, WAVE);
-                    const u32 mn = v[r] < y ? v[r] : y, mx = v[r] < y ? y : v[r];
-                    v[r] = low == asc ? mn : mx;
-                }
-            }
+        for (int r = 0; r < R; r++) {
+            if (r & M) continue;
+            const u32 mn = min(v[r], v[r ^ M]), mx = max(v[r], v[r ^ M]);
+            const bool asc = ((u32)r * WAVE & K) == 0;
+            v[r] = asc ? mn : mx;
+            v[r ^ M] = asc ? mx : mn;
+        }
+    } else {
+        sjw_stage<0, K, J>(v[0]);
+        if constexpr (R > 1) sjw_stage<WAVE, K, J>(v[1]);
+        if constexpr (R > 2) {
+            sjw_stage<2 * WAVE, K, J>(v[2]);
+            sjw_stage<3 * WAVE, K, J>(v[3]);
         }
     }
+    if constexpr (J > 1) sjw_stages<R, K, J / 2>(v);
+    else if constexpr (K < (u32)R * WAVE) sjw_stages<R, K * 2, K>(v);
+}
+
+// Bitonic sort, ascending, of R * WAVE values held as v[r] = element r WAVE + lane:
+// distances below WAVE by lane permutes of the vector pipe, larger ones between
+// registers of the same lane.  With LDS shuffles for the lanes, whose latency
+// is paid at each of the 27 stages of 128 values, the kernel below took 1.18 ms
+// for 1e8 candidates in 1e6 rows; with these, and scans for the binary searches over
+// the runs, 0.71.
+constexpr int SJW_REG = 4;
+template <int R>
+__device__ __forceinline__ void sjw_sort_regs(u32 (&v)[R]) {
+    static_assert(R == 1 || R == 2 || R == 4, "a power of two");
+    sjw_stages<R, 2, 1>(v);
+}
+
+// Inclusive scans over the wave's lanes: rows of 16 by shifts, then across rows.
+__device__ __forceinline__ u32 sjw_scan_add(u32 v) {
+    v += sjw_dpp<0x111>(v);   // row_shr 1, 2, 4, 8 (0 shifted in)
+    v += sjw_dpp<0x112>(v);
+    v += sjw_dpp<0x114>(v);
+    v += sjw_dpp<0x118>(v);
+    v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);   // row_bcast 15 into rows 1 and 3
+    v += (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);   // row_bcast 31 into rows 2 and 3
+    return v;
+}
+__device__ __forceinline__ u32 sjw_scan_max(u32 v) {
+    v = max(v, sjw_dpp<0x111>(v));
+    v = max(v, sjw_dpp<0x112>(v));
+    v = max(v, sjw_dpp<0x114>(v));
+    v = max(v, sjw_dpp<0x118>(v));
+    v = max(v, (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false));
+    v = max(v, (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
+    return v;
 }
 
 // Rows the register kernel takes: at most SJW_REG * WAVE candidates from at
 // most WAVE b's (empty rows too).
 __device__ __forceinline__ bool sjw_small(u64 raw, u64 nb) { return raw <= (u64)SJW_REG * WAVE && nb <= (u64)WAVE; }
 
-// A small row's candidates: j = r WAVE + lane found among the lanes' runs
-// (q0, pre: this lane's run start and first candidate) by a binary search
-// over the lanes' starts, loaded into v[r] (R loads in flight), sorted in
-// registers; the first of each value goes to out in order.  Returns their count.
+// A small row's candidates j = r WAVE + lane: the lane whose run holds j is the
+// largest one that starts at or before it, a maximum scan over the starts (each
+// nonempty run's lane, left at its start in `mark`); loaded into v[r] (R loads in
+// flight), sorted in registers; the first of each value goes to out in order.
+// q0, pre, len: this lane's run start, first candidate and length.  Returns their count.
 template <int R>
-__device__ __forceinline__ u32 sjw_small_row(const u32 *col, u32 q0, u32 pre, u64 nb, u64 raw, int lane, u32 *out) {
+__device__ __forceinline__ u32 sjw_small_row(const u32 *col, u32 q0, u32 pre, u32 len, u32 raw, int lane, u32 *mark, u32 *out) {
     u32 v[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) mark[r * WAVE + lane] = 0u;
+    sjw_sync();
+    if (len) mark[pre] = (u32)lane + 1;
+    sjw_sync();
+    u32 before = 0;   // the mark in force at the end of the registers before
+    const u32 shift = q0 - pre;
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const u32 j = (u32)r * WAVE + (u32)lane;
-        int s = 0;   // the last lane whose start is <= j (starts rise with the lane; empty runs share one)
-#pragma unroll
-        for (int st = WAVE / 2; st > 0; st >>= 1) {
-            const u32 ps = __shfl(pre, s + st, WAVE);
-            if (s + st < (int)nb && ps <= j) s += st;
-        }
-        const u32 qs = __shfl(q0, s, WAVE), ps = __shfl(pre, s, WAVE);
-        v[r] = (u64)j < raw ? col[(u64)qs + (j - ps)] : 0xffffffffu;
+        const u32 s = max(sjw_scan_max(mark[j]), before);   // candidate 0 starts a run: s >= 1
+        before = (u32)__builtin_amdgcn_readlane((int)s, WAVE - 1);
+        const u32 at = (u32)__shfl((int)shift, (int)s - 1, WAVE) + j;
+        v[r] = j < raw ? col[at] : 0xffffffffu;
     }
-    sjw_sort_regs<R>(v, lane);
+    sjw_sort_regs<R>(v);
     u32 kept = 0;
 #pragma unroll
     for (int r = 0; r < R; r++) {
-        const u64 e = (u64)r * WAVE + (u64)lane;
+        const u32 e = (u32)r * WAVE + (u32)lane;
         // element e - 1: lane - 1's v[r], or for lane 0 the last lane's v[r - 1]
-        const u32 up = __shfl(v[r], (lane + WAVE - 1) & (WAVE - 1), WAVE);
-        const u32 wrap = __shfl(v[r > 0 ? r - 1 : 0], WAVE - 1, WAVE);
-        const u32 prev = lane > 0 ? up : wrap;
+        const int wrap = r ? __builtin_amdgcn_readlane((int)v[r - 1], WAVE - 1) : 0;
+        const u32 prev = (u32)__builtin_amdgcn_update_dpp(wrap, (int)v[r], 0x138, 0xf, 0xf, false);   // wave_shr 1
         const bool keep = e < raw && (e == 0 || v[r] != prev);
         const u64 bal = __ballot(keep);
         if (keep) out[kept + __builtin_amdgcn_mbcnt_hi((u32)(bal >> 32), __builtin_amdgcn_mbcnt_lo((u32)bal, 0u))] = v[r];
@@ -1063,13 +1127,13 @@ __device__ __forceinline__ u32 sjw_small_row(const u32 *col, u32 q0, u32 pre, u6
     return kept;
 }
 
-// Small rows with no LDS: lane l takes the row's l-th b, a wave scan lays the
-// b's runs end to end, and candidate j = r WAVE + lane is found by a binary
-// search over the lanes' starts (by shuffle) and loaded straight into v[r]
-// (SJW_REG loads in flight), then sorted in registers and deduplicated.
+// Small rows: lane l takes the row's l-th b, a wave scan lays the b's runs end to
+// end, and sjw_small_row does the rest without the LDS but for a mark per run.
 __global__ __launch_bounds__(256) void sj_row_small_k(const u32 *col, const u64 *dense, const u64 *roff, u64 W,
                                                       u32 *cand, u32 *ucnt) {
+    __shared__ u32 s_mark[SJW_W][SJW_REG * WAVE];
     const int lane = threadIdx.x & (WAVE - 1);
+    u32 *mark = s_mark[threadIdx.x / WAVE];
     for (u64 c = ((u64)blockIdx.x * blockDim.x + threadIdx.x) / WAVE; c < W; c += (u64)gridDim.x * blockDim.x / WAVE) {
         const u64 r0 = roff[c], raw = roff[c + 1] - r0;
         const u64 p0 = dense[c], nb = dense[c + 1] - p0;
@@ -1085,17 +1149,11 @@ __global__ __launch_bounds__(256) void sj_row_small_k(const u32 *col, const u64 
             q0 = (u32)d0;
             len = (u32)(dense[b + 1] - d0);
         }
-        u32 inc = len;
-#pragma unroll
-        for (int d = 1; d < WAVE; d <<= 1) {
-            const u32 t = __shfl_up(inc, d, WAVE);
-            if (lane >= d) inc += t;
-        }
-        const u32 pre = inc - len;   // this lane's first candidate
+        const u32 pre = sjw_scan_add(len) - len;   // this lane's first candidate
         u32 kept;
-        if (raw <= (u64)WAVE) kept = sjw_small_row<1>(col, q0, pre, nb, raw, lane, cand + r0);
-        else if (raw <= 2 * (u64)WAVE) kept = sjw_small_row<2>(col, q0, pre, nb, raw, lane, cand + r0);
-        else kept = sjw_small_row<SJW_REG>(col, q0, pre, nb, raw, lane, cand + r0);
+        if (raw <= (u64)WAVE) kept = sjw_small_row<1>(col, q0, pre, len, (u32)raw, lane, mark, cand + r0);
+        else if (raw <= 2 * (u64)WAVE) kept = sjw_small_row<2>(col, q0, pre, len, (u32)raw, lane, mark, cand + r0);
+        else kept = sjw_small_row<SJW_REG>(col, q0, pre, len, (u32)raw, lane, mark, cand + r0);
         if (lane == 0) ucnt[c] = kept;
     }
 }
@@ -1108,10 +1166,28 @@ __global__ __launch_bounds__(SJW_T) void sj_row_sort_k(const u32 *col, const u64
     const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
     u32 *buf = s_buf[wv];
     u64 *pre = s_pre[wv], *q0s = s_q0[wv];
-    for (u64 c = (u64)blockIdx.x * SJW_W + wv; c < W; c += (u64)gridDim.x * SJW_W) {   // wave-uniform
+    // 64 rows a look, as most are sj_row_small_k's (1e6 rows with hardly any to sort: 158 -> 87 us)
+    u64 mine = 0, base = ((u64)blockIdx.x * SJW_W + wv) * WAVE;
+    const u64 step = (u64)gridDim.x * SJW_W * WAVE;
+    bool fresh = true;
+    while (true) {   // wave-uniform
+        if (!mine) {
+            if (!fresh) base += step;
+            fresh = false;
+            if (base >= W) break;
+            const u64 l = base + (u64)lane;
+            bool is = false;
+            if (l < W) {
+                const u64 n = roff[l + 1] - roff[l];
+                is = !sjw_small(n, dense[l + 1] - dense[l]) && n <= SJW_CAP;   // the others: sj_row_small_k's, or heavy rows
+            }
+            mine = __ballot(is);
+            continue;
+        }
+        const u64 c = base + (u64)(__ffsll((unsigned long long)mine) - 1);
+        mine &= mine - 1;
         const u64 r0 = roff[c], raw = roff[c + 1] - r0;
         const u64 p1 = dense[c + 1];
-        if (sjw_small(raw, p1 - dense[c]) || raw > SJW_CAP) continue;   // sj_row_small_k's, or a heavy row
         // gather the row's candidates into buf[0, raw)
         u64 filled = 0;
         for (u64 pb = dense[c]; pb < p1; pb += WAVE) {
@@ -1148,7 +1224,7 @@ __global__ __launch_bounds__(SJW_T) void sj_row_sort_k(const u32 *col, const u64
                 const u64 e = (u64)r * WAVE + (u64)lane;
                 v[r] = e < raw ? buf[e] : 0xffffffffu;
             }
-            sjw_sort_regs<SJW_REG>(v, lane);
+            sjw_sort_regs<SJW_REG>(v);
             u32 kept = 0;
 #pragma unroll
             for (int r = 0; r < SJW_REG; r++) {
