@@ -638,8 +638,9 @@ void unpack_rows(dlg_ctx *ctx, const u64 *t, u64 n, int orient, int32_t *rows);
 // E into out[0, n) and E⁻¹ into out_rev[0, n), row order kept, also returning
 // the count of adjacent input rows out of order and, in cb, the flipped
 // bounds of both columns (min a, max a, min b, max b) -- one read
-// (synchronises).
-u64 pack_sym_rows_scan(dlg_ctx *ctx, const int32_t *rows, u64 n, u64 *out, u64 *out_rev, u32 *cb);
+// (synchronises).  *both: the rows are in strictly ascending order and their
+// own reverse; out is E then, and neither out_rev nor cb is written.
+u64 pack_sym_rows_scan(dlg_ctx *ctx, const int32_t *rows, u64 n, u64 *out, u64 *out_rev, u32 *cb, bool *both);
 void fill_u64(dlg_ctx *ctx, u64 *p, u64 n, u64 v);
 void fill_u32(dlg_ctx *ctx, u32 *p, u64 n, u32 v);
 void copy_u64(dlg_ctx *ctx, u64 *dst, const u64 *src, u64 n);

@@ -699,10 +699,14 @@ void wcc_graph_build(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, 
     // and column bounds taken in the same read
     DBuf<u64> sym(ctx, 2 * n), edge(ctx), tmp(ctx);
     u32 cb[4];
-    const u64 breaks = pack_sym_rows_scan(ctx, d_rows, n, sym.p, sym.p + n, cb);
+    bool both;
+    const u64 breaks = pack_sym_rows_scan(ctx, d_rows, n, sym.p, sym.p + n, cb, &both);
     const bool presorted = n >= WCC_PRESORTED_MIN && breaks == 0;
     pc.mark(DLG_PH_DEDUP);
-    if (presorted) {
+    if (both) {   // E, sorted and without duplicates, is its own reverse
+        edge.swap(sym);
+        g.ne = n;
+    } else if (presorted) {
         // E arrives sorted by (src, dst): E⁻¹ in that order lists each dst's sources in
         // ascending order, so a stable sort by its key alone sorts it by (dst, src) --
         // the key's passes only -- and one merge keeping one copy of each edge gives
