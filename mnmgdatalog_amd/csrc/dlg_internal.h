@@ -219,6 +219,16 @@ __device__ __forceinline__ u32 fmix32(u32 h) {
 }
 __device__ __forceinline__ u32 tkey(u64 t) { return (u32)(t >> 32); }
 __device__ __forceinline__ u32 tval(u64 t) { return (u32)t; }
+// The group of a key in an index's slots; all ones: none.
+__device__ __forceinline__ u32 ix_find(const u64 *slots, u64 mask, u32 key) {
+    u64 p = fmix32(key) & mask;
+    while (true) {
+        u64 s = slots[p];
+        if (s == EMPTY_SLOT) return 0xffffffffu;
+        if (tkey(s) == key) return tval(s);
+        p = (p + 1) & mask;
+    }
+}
 __device__ __forceinline__ u64 tmake(u32 k, u32 v) { return ((u64)k << 32) | v; }
 __device__ __forceinline__ u64 lanemask_lt() {
     return (1ull << (threadIdx.x & (WAVE - 1))) - 1ull;
@@ -628,6 +638,10 @@ u64 hashrel_insert_list(dlg_ctx *ctx, HashRel &r, const u64 *x, u64 n);
 // tuples [off, off + n)); nodiag drops rows with key == value.  *raw += |probe ⋈ index|.
 u64 hashrel_insert_join(dlg_ctx *ctx, HashRel &r, const Index &ix, const u64 *probe, u64 off, u64 n, int proj,
                         bool nodiag, JoinScratch &js, u64 *raw);
+// TC's rounds N = Δ ⋈ index (tuples (index value, probe value)) \ F until a
+// round finds nothing new or `max_it` (> 0) have run: Δ is the relation's tuples
+// [off, off + n) at first, then those that the round before appended.  Returns their number.
+int hashrel_rounds(dlg_ctx *ctx, HashRel &r, const Index &ix, u64 off, u64 n, int max_it, JoinScratch &js, u64 *raw);
 // Merge of sorted a, b into out (a first on ties).
 void merge(dlg_ctx *ctx, const u64 *a, u64 na, const u64 *b, u64 nb, u64 *out);
 // The merge with one copy of each value kept (inputs sorted, duplicates

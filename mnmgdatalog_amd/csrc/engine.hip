@@ -423,12 +423,17 @@ void tc_fixpoint(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, Phas
         u64 beg = 0, nd = hashrel_insert_list(ctx, F, J.p, n);   // F = Δ0
         J.release();
         pc.mark(DLG_PH_JOIN);
-        while (true) {
+        if (!hook) {
+            u64 raw = 0;
+            it = hashrel_rounds(ctx, F, ix, beg, nd, o.max_it, js, &raw);   // (z, x)
+            out.raw += (i64)raw;
+        }
+        while (hook) {
             u64 raw = 0;
             const u64 nn = hashrel_insert_join(ctx, F, ix, nullptr, beg, nd, DLG_PROJ_HV_PV, false, js, &raw);   // (z, x)
             out.raw += (i64)raw;
             it++;
-            if (hook) hook->on_round(ctx, F.all.p + beg + nd, nn, it, false);
+            hook->on_round(ctx, F.all.p + beg + nd, nn, it, false);
             if (nn == 0) break;                         // |F| unchanged (tc.cu:294-300)
             beg += nd;
             nd = nn;

@@ -29,16 +29,6 @@
 
 namespace dlg {
 
-__device__ __forceinline__ u32 ix_find(const u64 *slots, u64 mask, u32 key) {
-    u64 p = fmix32(key) & mask;
-    while (true) {
-        u64 s = slots[p];
-        if (s == EMPTY_SLOT) return 0xffffffffu;
-        if (tkey(s) == key) return tval(s);
-        p = (p + 1) & mask;
-    }
-}
-
 __global__ void set_last_k(u32 *gstart, u64 g, u32 n) {
     if (threadIdx.x == 0 && blockIdx.x == 0) gstart[g] = n;
 }

@@ -59,3 +59,36 @@ def test_large_rounds(ctx):
     got, want = ctx.run("tc", rows), ctx.run("tc", rows, strategy=2)
     same(got, want)
     assert got["raw_join_rows"] == want["raw_join_rows"]
+
+
+# rounds queued ahead: tiles of 256 probes and their remainders, many rounds, a hub whose rows one tile does not take,
+# far more join rows than the set has room for, and a stop after k rounds
+@pytest.mark.parametrize("shape", ["path 255", "path 300", "path 1000", "hub", "cliques"])
+@pytest.mark.parametrize("k", [0, 1, 3, 4])
+def test_queued_rounds(ctx, orc, shape, k):
+    rng = np.random.default_rng(len(shape))
+    if shape.startswith("path"):
+        n = int(shape.split()[1])
+        rows = np.stack([np.arange(n), np.arange(1, n + 1)], 1)
+        rows = np.concatenate([rows, rng.integers(0, n, (n // 8, 2))]) if n == 300 else rows
+    elif shape == "hub":   # 300 paths of 2 into a hub of 400 ends, another of 17,000
+        rows = np.concatenate([np.stack([np.arange(300) + 10, np.full(300, 1)], 1), np.stack([np.full(400, 1), np.arange(400) + 1000], 1),
+                               np.stack([np.full(17_000, 2), np.arange(17_000) + 2000], 1), [[1000, 2], [5, 10]]])
+    else:
+        rows = np.concatenate([np.stack(np.nonzero(~np.eye(40, dtype=bool)), 1) + 50 * i for i in range(6)] + [[[3, 55], [60, 110]]])
+    rows = (rows * 101).astype(np.int32)
+    kw = {"max_iterations": k} if k else {}
+    got = ctx.run("tc", rows, strategy=3, **kw)
+    same(got, orc.tc(rows, **kw))
+    assert got["raw_join_rows"] == ctx.run("tc", rows, strategy=2, **kw)["raw_join_rows"]
+
+
+def test_tight_budget(orc):
+    """A request under a memory budget that has room for its rounds one by one, but not for several at once."""
+    rows = (np.random.default_rng(4).integers(0, 3000, size=(2900, 2)) * 4096).astype(np.int32)
+    want = orc.tc(rows)
+    for mb in (256, 320, 512):
+        with dlg.Server(0, workers=1, hbm_budget=mb << 20, retain_bytes=1, strategy=3) as srv:
+            got = srv.wait(srv.submit("tc", rows))
+        assert got["status"] == 0
+        same(got, want)
