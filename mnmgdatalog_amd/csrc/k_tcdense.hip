@@ -25,7 +25,8 @@
 // Bound by the latency of dependent reads (list, flag, row) at small sizes
 // and by the cache's bandwidth at large ones.
 // Measured against the row kernel with its compaction and index build (whole
-// call): 437 ids, 700 edges 1.13 -> 0.31 ms (a round 4.7 us; it was 14);
+// call): 437 ids, 700 edges 1.13 -> 0.31 ms (a round 4.7 us; it was 14; one workgroup
+// below takes it now);
 // 3,000 ids, 7,000 power-law edges with 6.3M rows to the host 4.6 -> 1.6 ms (a
 // round 5.6 us, the rest the copy; one wave per source had the hubs' rows to
 // itself, up to 0.3 ms a round); 512 instances of 1,000 to 23,911 edges in
@@ -335,6 +336,180 @@ __global__ void td_wgblk_k(const TdBlock *blk, u32 nblk, u32 nwg, u32 *wgblk) {
     wgblk[i] = a;
 }
 
+// ---------------------------------------------------------- one workgroup's closure
+// The whole run of a small range by one workgroup: F and D in LDS, the
+// predecessors taken from the edges' own bits (row z of the first D holds z's predecessors),
+// every round two barriers instead of a launch.  A thread keeps its words of N in
+// registers while D is still read.  Takes what fits: 2 W wpr words, the out-degrees,
+// the lists (2 bytes an edge): about 700 ids, less with many edges.
+// Bound by the LDS reads of a round's predecessors and its two barriers.
+constexpr int TS_T = 1024, TS_I = 5;              // threads, items (uint4s of the map) a thread at most
+constexpr u32 TS_LONG = 128, TS_NLONG = 8;        // predecessors above which all threads share a row; such rows at most
+constexpr u32 TS_LDS = 40000;                     // words: one workgroup's LDS but for 3.8 KB
+constexpr u64 TS_MAX_ROWS = 8192;                 // edges, read by one workgroup
+
+static u64 ts_words(u64 n, u64 W, u64 wpr) { return (2 * W + TS_NLONG) * wpr + 2 * W + 1 + (n + 1) / 2; }
+static bool ts_takes(u64 n, u64 W, u64 wpr) {
+    return n <= TS_MAX_ROWS && W <= (u64)TS_T && ts_words(n, W, wpr) <= TS_LDS && W * (wpr / 4) <= (u64)TS_T * TS_I;
+}
+
+__device__ __forceinline__ u64 ts_sum(u64 v, u64 *s_w) {   // every thread calls it; valid in thread 0
+#pragma unroll
+    for (int d = WAVE / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, WAVE);
+    if (threadIdx.x % WAVE == 0) s_w[threadIdx.x / WAVE] = v;
+    __syncthreads();
+    v = 0;
+    if (threadIdx.x == 0)
+        for (int w = 0; w < TS_T / WAVE; w++) v += s_w[w];
+    __syncthreads();
+    return v;
+}
+
+__global__ __launch_bounds__(TS_T) void td_small_k(const int2 *rows, u32 n, u32 lo, u32 W, u32 wpr, int max_it, u32 *out,
+                                                   u32 out_words, u64 *host, u64 seq) {
+    __shared__ __align__(16) u32 pool[TS_LDS];
+    __shared__ u64 s_w[TS_T / WAVE + 1];
+    __shared__ u32 s_long[TS_NLONG], s_nlong;
+    const u32 mw = W * wpr, wq = wpr / 4, items = W * wq;
+    u32 *D = pool, *F = pool + mw, *sums = F + mw, *outdeg = sums + TS_NLONG * wpr, *first = outdeg + W;   // first: W + 1 list starts
+    unsigned short *adj = (unsigned short *)(first + W + 1);
+    for (u32 i = threadIdx.x; i < mw; i += TS_T) D[i] = 0;
+    if (threadIdx.x < W) outdeg[threadIdx.x] = 0;
+    if (threadIdx.x == 0) s_nlong = 0;
+    __syncthreads();
+    for (u32 i = threadIdx.x; i < n; i += TS_T) {
+        const int2 e = rows[i];
+        const u32 x = td_key(e.x, lo), z = td_key(e.y, lo);
+        atomicOr(D + z * wpr + (x >> 5), 1u << (x & 31));
+        atomicAdd(outdeg + x, 1u);
+    }
+    __syncthreads();
+    // the predecessors of row threadIdx.x, without duplicates; F = D
+    u64 c = 0, w = 0;   // this thread's new tuples so far; the join rows that the last round's make
+    {
+        const u32 *row = D + threadIdx.x * wpr;
+        u32 k = 0;
+        if (threadIdx.x < W)
+            for (u32 i = 0; i < wpr; i++) k += (u32)__popc(row[i]);
+        u64 tot;
+        u32 at = (u32)block_exclusive_scan<u64>((u64)k, s_w, &tot);
+        if (threadIdx.x < W) {
+            first[threadIdx.x] = at;
+            if (threadIdx.x == W - 1) first[W] = (u32)tot;   // at most n
+            for (u32 i = 0; i < wpr; i++)
+                for (u32 b = row[i]; b; b &= b - 1) adj[at++] = (unsigned short)(i * 32 + (u32)__ffs(b) - 1);
+            if (k > TS_LONG) {
+                const u32 j = atomicAdd(&s_nlong, 1u);
+                if (j < TS_NLONG) s_long[j] = threadIdx.x;
+            }
+            c = k;
+            w = (u64)k * outdeg[threadIdx.x];
+        }
+    }
+    uint4 *D4 = (uint4 *)D, *F4 = (uint4 *)F, *S4 = (uint4 *)sums;
+    for (u32 i = threadIdx.x; i < items; i += TS_T) F4[i] = D4[i];
+    u32 from[TS_I], to[TS_I], col[TS_I], deg[TS_I];
+    __syncthreads();
+    if (s_nlong > TS_NLONG) {   // block-uniform
+        if (threadIdx.x == 0) {
+            host[2] = 0;
+            __threadfence_system();
+            *(volatile u64 *)(host + dlg_ctx::MAPPED_SEQ) = seq;
+            __threadfence_system();
+        }
+        return;
+    }
+#pragma unroll
+    for (int q = 0; q < TS_I; q++) {
+        const u32 i = threadIdx.x + (u32)q * TS_T, r = i < items ? i / wq : 0u;
+        col[q] = i - r * wq;
+        from[q] = i < items ? first[r] : 0u;
+        to[q] = i < items ? first[r + 1] : 0u;   // past the end: an empty list
+        deg[q] = outdeg[r];
+        if (to[q] - from[q] > TS_LONG) to[q] = from[q];
+    }
+    const u32 nlong = s_nlong, part = TS_T / wq, slot = threadIdx.x / wq, scol = threadIdx.x % wq;
+    int it = 0;
+    u64 raw = 0;
+    while (max_it <= 0 || it < max_it) {   // block-uniform; a round that finds nothing is the last, as F can only grow
+        raw += w;
+        w = 0;
+        uint4 nw[TS_I];
+        bool some = false;
+        // the words of `a` that item i of F does not have, into F
+        auto update = [&](uint4 a, u32 i, u32 dg) {
+            const uint4 f = F4[i];
+            a = make_uint4(a.x & ~f.x, a.y & ~f.y, a.z & ~f.z, a.w & ~f.w);
+            if (td_any(a)) {
+                F4[i] = make_uint4(f.x | a.x, f.y | a.y, f.z | a.z, f.w | a.w);
+                const u32 k = (u32)(__popc(a.x) + __popc(a.y) + __popc(a.z) + __popc(a.w));
+                c += k;
+                w += (u64)k * dg;
+                some = true;
+            }
+            return a;
+        };
+        if (nlong) {   // block-uniform
+            for (u32 i = threadIdx.x; i < nlong * wq; i += TS_T) S4[i] = make_uint4(0u, 0u, 0u, 0u);
+            __syncthreads();
+            for (u32 j = 0; j < nlong; j++) {
+                const u32 p1 = first[s_long[j] + 1];
+                uint4 a = make_uint4(0u, 0u, 0u, 0u);
+                if (slot < part)
+                    for (u32 p = first[s_long[j]] + slot; p < p1; p += part) {
+                        const uint4 v = D4[(u32)adj[p] * wq + scol];
+                        a = make_uint4(a.x | v.x, a.y | v.y, a.z | v.z, a.w | v.w);
+                    }
+                u32 *sum = sums + (j * wq + scol) * 4;
+                if (a.x) atomicOr(sum, a.x);
+                if (a.y) atomicOr(sum + 1, a.y);
+                if (a.z) atomicOr(sum + 2, a.z);
+                if (a.w) atomicOr(sum + 3, a.w);
+            }
+            __syncthreads();
+            for (u32 i = threadIdx.x; i < nlong * wq; i += TS_T) {
+                const u32 r = s_long[i / wq];
+                S4[i] = update(S4[i], r * wq + i % wq, outdeg[r]);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < TS_I; q++) {
+            uint4 a = make_uint4(0u, 0u, 0u, 0u);
+            for (u32 p = from[q]; p < to[q]; p += 4) {   // past the end the last one again
+                uint4 v[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[k] = D4[(u32)adj[min(p + k, to[q] - 1)] * wq + col[q]];
+#pragma unroll
+                for (int k = 0; k < 4; k++) a = make_uint4(a.x | v[k].x, a.y | v[k].y, a.z | v[k].z, a.w | v[k].w);
+            }
+            if (td_any(a)) a = update(a, threadIdx.x + (u32)q * TS_T, deg[q]);
+            nw[q] = a;
+        }
+        it++;
+        const bool any = __syncthreads_or(some);   // D is read no more
+        if (!any) break;
+#pragma unroll
+        for (int q = 0; q < TS_I; q++)
+            if (threadIdx.x + (u32)q * TS_T < items) D4[threadIdx.x + (u32)q * TS_T] = nw[q];
+        if (nlong) {
+            __syncthreads();   // over the empty words that the rows' own threads have for them
+            for (u32 i = threadIdx.x; i < nlong * wq; i += TS_T) D4[s_long[i / wq] * wq + i % wq] = S4[i];
+        }
+        __syncthreads();
+    }
+    for (u32 i = threadIdx.x; i < out_words / 4; i += TS_T) ((uint4 *)out)[i] = i < items ? F4[i] : make_uint4(0u, 0u, 0u, 0u);
+    c = ts_sum(c, s_w);
+    raw = ts_sum(raw, s_w);
+    if (threadIdx.x == 0) {
+        host[0] = c;
+        host[1] = raw;
+        host[2] = (u64)it;
+        __threadfence_system();
+        *(volatile u64 *)(host + dlg_ctx::MAPPED_SEQ) = seq;
+        __threadfence_system();
+    }
+}
+
 int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, const std::vector<u32> *starts, int max_it,
                  DBuf<u64> &out, u64 *total, u64 *raw, std::vector<int> *iters) {
     // the id ranges that hold rows, as in rowmap_init
@@ -363,6 +538,22 @@ int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, con
         hb.push_back(k);
         owner.push_back((int)i);
         maps.push_back({(u32)b0, k.W, k.wpr, k.base});
+    }
+    if (!starts && ts_takes(n, W, hb[0].wpr)) {
+        DBuf<u32> F(ctx, words);
+        const u64 seq = ++ctx->mapped_seq;
+        DLG_LAUNCH(ctx, DLG_K_BITMAP_INSERT, 8.0 * n + 4.0 * words, td_small_k, 1, TS_T, 0, (const int2 *)d_rows, (u32)n, lo,
+                   (u32)W, hb[0].wpr, max_it, F.p, (u32)words, ctx->mapped_dev(seq), seq);
+        ctx->wait_mapped(seq);
+        const volatile u64 *m = ctx->mapped_host(seq);
+        const int it = (int)m[2];
+        if (it > 0) {   // 0: too many rows with long lists
+            *total = m[0];
+            *raw += m[1];
+            bitmap_emit_tiled(ctx, F.p, maps, words, out, *total);
+            if (iters) iters->assign(1, it);
+            return it;
+        }
     }
     const u32 nblk = (u32)hb.size();
     // four tasks per sub-group once that still leaves every CU eight workgroups

@@ -100,3 +100,40 @@ def test_batch_digest_segments(ctx, prog):
         p = ctx.run(prog, rows, keep_output=False, check_output=1)
         assert (r["output_size"], r["output_sum"]) == (p["output_size"], p["output_sum"])
         assert r["output_order_breaks"] == p["output_order_breaks"] == 0
+
+
+# one workgroup's closure: the widest ranges it takes and the first it does not (by the map, by the edges' lists, by
+# their number), many rounds, a hub, duplicates, and stops after k rounds
+@pytest.mark.parametrize("width,edges", [(128, 8185), (129, 8186), (384, 400), (385, 400), (512, 600), (640, 700), (640, 8000), (697, 1200),
+                                         (704, 2500), (720, 900), (735, 750), (768, 800), (769, 800), (1024, 1100)])
+@pytest.mark.parametrize("k", [0, 3])
+def test_one_workgroup(ctx, orc, width, edges, k):
+    rows = graph(width, edges, width + edges, hub=width // 3)
+    rows = rows[:8192] if edges == 8185 else rows
+    kw = {"max_iterations": k} if k else {}
+    got = ctx.run("tc", rows, **kw)
+    same(got, orc.tc(rows, **kw))
+    assert got["raw_join_rows"] == ctx.run("tc", rows, queue=1, **kw)["raw_join_rows"]
+
+
+@pytest.mark.parametrize("n", [1, 300, 700])
+@pytest.mark.parametrize("k", [0, 1, 2, 5])
+def test_one_workgroup_paths(ctx, orc, n, k):
+    rows = np.stack([np.arange(n), np.arange(1, n + 1)], 1)
+    rows = np.concatenate([rows, rows[:7], rows[:7]]).astype(np.int32) - 2**31 // 2
+    kw = {"max_iterations": k} if k else {}
+    got = ctx.run("tc", rows, **kw)
+    same(got, orc.tc(rows, **kw))
+    assert got["raw_join_rows"] == ctx.run("tc", rows, queue=1, **kw)["raw_join_rows"]
+
+
+@pytest.mark.parametrize("hubs", [1, 7, 8, 9, 20])
+@pytest.mark.parametrize("k", [0, 2])
+def test_one_workgroup_hubs(ctx, orc, hubs, k):
+    """Rows of 128 to 130 predecessors and more: those that one workgroup shares, and more of them than it takes."""
+    r = [np.stack([np.arange(128 + h % 3 + 9 * (h == 4)), np.full(128 + h % 3 + 9 * (h == 4), 200 + h)], 1) for h in range(hubs)]
+    rows = np.concatenate(r + [np.stack([np.arange(300, 420), np.arange(301, 421)], 1), [[200, 300], [200 + hubs - 1, 5], [420, 7]]]).astype(np.int32)
+    kw = {"max_iterations": k} if k else {}
+    got = ctx.run("tc", rows, **kw)
+    same(got, orc.tc(rows, **kw))
+    assert got["raw_join_rows"] == ctx.run("tc", rows, queue=1, **kw)["raw_join_rows"]
