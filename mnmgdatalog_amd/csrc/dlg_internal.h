@@ -653,8 +653,10 @@ void unpack_rows(dlg_ctx *ctx, const u64 *t, u64 n, int orient, int32_t *rows);
 // the count of adjacent input rows out of order and, in cb, the flipped
 // bounds of both columns (min a, max a, min b, max b) -- one read
 // (synchronises).  *both: the rows are in strictly ascending order and their
-// own reverse; out is E then, and neither out_rev nor cb is written.
-u64 pack_sym_rows_scan(dlg_ctx *ctx, const int32_t *rows, u64 n, u64 *out, u64 *out_rev, u32 *cb, bool *both);
+// own reverse; out is E then, heads has a bit per row that begins a key's run, and
+// neither out_rev nor cb is written.
+u64 pack_sym_rows_scan(dlg_ctx *ctx, const int32_t *rows, u64 n, u64 *out, u64 *out_rev, u32 *cb, bool *both,
+                       DBuf<u64> &heads);
 void fill_u64(dlg_ctx *ctx, u64 *p, u64 n, u64 v);
 void fill_u32(dlg_ctx *ctx, u32 *p, u64 n, u32 v);
 void copy_u64(dlg_ctx *ctx, u64 *dst, const u64 *src, u64 n);
@@ -673,8 +675,11 @@ struct Index {
 };
 // Build from a device relation (copied); `presorted` skips the sort;
 // `sorted_lookup` builds no hash slots (probes binary-search the rows).
+// `heads`: the rows' key heads, where the caller has them (a bit per row).
 void index_build(dlg_ctx *ctx, Index &ix, const u64 *rel, u64 n, double load_factor,
-                 bool presorted, bool sorted_lookup = false);
+                 bool presorted, bool sorted_lookup = false, const u64 *heads = nullptr);
+// The positions of the set bits among n flags, their number returned (synchronises).
+u64 select_flagged(dlg_ctx *ctx, const u64 *flags, u64 n, u32 *out);
 // Dense row offsets by key over [lo, lo + W) (index_build drops them); the
 // hash-index count phase then reads an offset pair per probe instead of
 // probing the slots.

@@ -702,10 +702,10 @@ void wcc_graph_build(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, 
     pc.mark(DLG_PH_INIT);
     // E then E⁻¹ in one buffer (wcc.cu:140-160), with the input's order breaks
     // and column bounds taken in the same read
-    DBuf<u64> sym(ctx, 2 * n), edge(ctx), tmp(ctx);
+    DBuf<u64> sym(ctx, 2 * n), edge(ctx), tmp(ctx), heads(ctx);
     u32 cb[4];
     bool both;
-    const u64 breaks = pack_sym_rows_scan(ctx, d_rows, n, sym.p, sym.p + n, cb, &both);
+    const u64 breaks = pack_sym_rows_scan(ctx, d_rows, n, sym.p, sym.p + n, cb, &both, heads);
     const bool presorted = n >= WCC_PRESORTED_MIN && breaks == 0;
     pc.mark(DLG_PH_DEDUP);
     if (both) {   // E, sorted and without duplicates, is its own reverse
@@ -736,7 +736,7 @@ void wcc_graph_build(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, 
     tmp.release();
     pc.mark(DLG_PH_HASHTABLE);
     g.ix.rows.swap(edge);   // the index keeps the sorted edges in place
-    index_build(ctx, g.ix, g.ix.rows.p, g.ne, o.lf, true, true);
+    index_build(ctx, g.ix, g.ix.rows.p, g.ne, o.lf, true, true, both ? heads.p : nullptr);
     // the rounds read the groups' runs; the neighbour lookup takes the rank
     // directory when it applies, else hash probes (slots built only then)
     if (o.join != 1) {

@@ -51,7 +51,7 @@ __global__ void hash_insert_k(const u64 *rows, const u32 *gstart, u64 G, u64 *sl
 }
 
 void index_build(dlg_ctx *ctx, Index &ix, const u64 *rel, u64 n, double lf, bool presorted,
-                 bool sorted_lookup) {
+                 bool sorted_lookup, const u64 *heads) {
     ix.n = n;
     ix.groups = 0;
     ix.nslots = 0;
@@ -74,7 +74,7 @@ void index_build(dlg_ctx *ctx, Index &ix, const u64 *rel, u64 n, double lf, bool
             ix.rows.ensure(n);
             if (rel != ix.rows.p) copy_u64(ctx, ix.rows.p, rel, n);
         }
-        G = select(ctx, SEL_KEY_HEAD, ix.rows.p, n, nullptr, 0, ix.gstart.p);
+        G = heads ? select_flagged(ctx, heads, n, ix.gstart.p) : select(ctx, SEL_KEY_HEAD, ix.rows.p, n, nullptr, 0, ix.gstart.p);
     }
     DLG_LAUNCH(ctx, DLG_K_MISC, 4.0, set_last_k, 1, 64, 0, ix.gstart.p, G, (u32)n);
     ix.groups = G;

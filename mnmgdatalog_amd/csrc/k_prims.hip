@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256) void pack_sym_scan_k(const int2 *rows, u64 n, 
 // ------------------------------------------- relations that are their own reverse
 // A WCC input often lists both directions of every edge, sorted.  It is then its own
 // E u E⁻¹, and the reversed copy, its sort and the merge are for nothing (R-MAT-23,
-// 2.6e8 rows: 13.2 -> 5.4 ms for the whole call).  Whether it is, in one read: the rows are in strictly
+// 2.6e8 rows: 13.2 -> 4.8 ms for the whole call).  Whether it is, in one read: the rows are in strictly
 // ascending order, and {(a, b) : a < b} and {(b, a) : a > b} are the same set, which
 // two products over the rows tell,
 //     prod (r - min(a, b) - s max(a, b))  mod p = 2^61 - 1,  once over a < b, once over a > b.
@@ -162,13 +162,13 @@ __global__ __launch_bounds__(FP_WAVES * WAVE) void reverse_probe_k(const int2 *r
     if (lane == 0 && (lo == n || row_key(rows[lo]) != want)) *miss = 1u;
 }
 
-// Rows packed as (a, b), with the bounds of the first column, the count of rows not
-// below their successor, and the workgroup's products, unless the look before missed.
-// Bound by the products beside the copy (FP_I rows in flight a thread): 2.6e8 rows 0.93
-// ms, 4.5 TB/s; the scan that writes both directions takes 1.43.
+// Rows packed as (a, b), with a bit per row that begins a key's run, the count of rows
+// not above the one before, and the workgroup's products, unless the look before missed.
+// Bound by the products beside the copy (FP_I rows in flight a thread): 2.6e8 rows 1.0
+// ms, 4.2 TB/s; the scan that writes both directions takes 1.43.
 constexpr int FP_T = 256, FP_I = 4;
-__global__ __launch_bounds__(FP_T) void pack_both_scan_k(const int2 *rows, u64 n, u64 *out, FpPoint at, const u32 *miss,
-                                                        u64 *part, unsigned long long *breaks) {
+__global__ __launch_bounds__(FP_T) void pack_both_scan_k(const int2 *rows, u64 n, u64 *out, u64 *heads, FpPoint at,
+                                                        const u32 *miss, u64 *part, unsigned long long *breaks) {
     if (*miss) return;   // set by an earlier launch: the same for all
     u64 up[FP_POINTS], down[FP_POINTS];
 #pragma unroll
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(FP_T) void pack_both_scan_k(const int2 *rows, u64 n
         for (int j = 0; j < FP_I; j++) {
             const u64 i = base + (u64)j * FP_T;
             v[j] = rows[i < n ? i : n - 1];
-            q[j] = rows[i + 1 < n ? i + 1 : n - 1];
+            q[j] = rows[i < n && i > 0 ? i - 1 : 0];
         }
 #pragma unroll
         for (int j = 0; j < FP_I; j++) {
@@ -190,7 +190,9 @@ __global__ __launch_bounds__(FP_T) void pack_both_scan_k(const int2 *rows, u64 n
             const u32 a = (u32)v[j].x ^ 0x80000000u, b = (u32)v[j].y ^ 0x80000000u;
             const u64 x = min(a, b), y = max(a, b);
             if (i < n) out[i] = tmake(a, b);
-            dc += i + 1 < n && tmake(a, b) >= row_key(q[j]);
+            dc += i < n && i > 0 && row_key(q[j]) >= tmake(a, b);
+            const u64 hm = __ballot(i < n && (i == 0 || q[j].x != v[j].x));   // i: a multiple of 64 in lane 0
+            if (threadIdx.x % WAVE == 0 && i < n) heads[i / WAVE] = hm;
             const bool asc = a < b, use = i < n && a != b;
 #pragma unroll
             for (int k = 0; k < FP_POINTS; k++) {
@@ -266,7 +268,8 @@ __global__ void pack_scan_init_k(u64 *w) {
     if (threadIdx.x < 4) mm[threadIdx.x] = threadIdx.x & 1 ? 0u : 0xffffffffu;
     else if (threadIdx.x < 2 + PS_WORDS) w[threadIdx.x - 2] = 0ull;   // words 2 .. PS_WORDS - 1
 }
-u64 pack_sym_rows_scan(dlg_ctx *ctx, const int32_t *rows, u64 n, u64 *out, u64 *out_rev, u32 *cb, bool *both) {
+u64 pack_sym_rows_scan(dlg_ctx *ctx, const int32_t *rows, u64 n, u64 *out, u64 *out_rev, u32 *cb, bool *both,
+                       DBuf<u64> &heads) {
     cb[0] = cb[1] = cb[2] = cb[3] = 0u;
     *both = false;
     if (!n) return 0;
@@ -275,6 +278,7 @@ u64 pack_sym_rows_scan(dlg_ctx *ctx, const int32_t *rows, u64 n, u64 *out, u64 *
     const unsigned g = (unsigned)std::min<u64>((n + 255) / 256, (u64)ctx->num_cus * 8);
     FpPoint at;
     bool look = n >= FP_MIN && getentropy(&at, sizeof(at)) == 0;
+    if (look) heads.ensure((n + WAVE - 1) / WAVE);
     while (true) {
         u32 *miss = look ? (u32 *)(w.p + PS_MISS) : nullptr;
         DLG_LAUNCH(ctx, DLG_K_MISC, 0.0, pack_scan_init_k, 1, 64, 0, w.p);
@@ -286,7 +290,7 @@ u64 pack_sym_rows_scan(dlg_ctx *ctx, const int32_t *rows, u64 n, u64 *out, u64 *
             const unsigned gb = (unsigned)std::min<u64>((n + FP_T * FP_I - 1) / (FP_T * FP_I), (u64)ctx->num_cus * 8);
             DBuf<u64> part(ctx, (u64)gb * 2 * FP_POINTS);
             DLG_LAUNCH(ctx, DLG_K_MISC, 0.0, reverse_probe_k, FP_SAMPLES / FP_WAVES, FP_WAVES * WAVE, 0, r, n, miss);
-            DLG_LAUNCH(ctx, DLG_K_PACK, 16.0 * n, pack_both_scan_k, gb, FP_T, 0, r, n, out, at, (const u32 *)miss, part.p,
+            DLG_LAUNCH(ctx, DLG_K_PACK, 16.0 * n, pack_both_scan_k, gb, FP_T, 0, r, n, out, heads.p, at, (const u32 *)miss, part.p,
                        (unsigned long long *)(w.p + PS_BREAKS));
             DLG_LAUNCH(ctx, DLG_K_MISC, 0.0, fp_fold_k, 1, 2 * FP_POINTS * WAVE, 0, (const u64 *)part.p, (u32)gb,
                        (const u32 *)miss, w.p + PS_BREAKS);
@@ -1577,6 +1581,38 @@ static u64 select_small(dlg_ctx *ctx, const u64 *in, u64 n, const u64 *other, u6
     return ((const volatile u64 *)ctx->mapped_host(seq))[0];
 }
 
+// The positions of the set bits among `n` flags: a thread takes a word, as few are
+// set (select_scatter_k has a thread a row: 2.6e8 rows with 4.9M heads 252 us, most of it
+// its 128,000 workgroups; 20 here).  bpre: the bits before each workgroup's words.
+constexpr u64 HW_ROWS = (u64)SEL_T * WAVE;   // rows a workgroup
+constexpr u64 HW_SPARSE = 8;                 // rows a head from which on
+__global__ __launch_bounds__(SEL_T) void heads_sum_k(const u64 *flags, u64 words, u64 *bsum) {
+    __shared__ u64 sc[SEL_T / WAVE + 1];
+    const u64 w = (u64)blockIdx.x * SEL_T + threadIdx.x;
+    u64 tot;
+    block_exclusive_scan<u64>(w < words ? (u64)__popcll(flags[w]) : 0ull, sc, &tot);
+    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
+}
+__global__ __launch_bounds__(SEL_T) void heads_scatter_k(const u64 *flags, u64 words, const u64 *bpre, u64 step, u32 *out) {
+    __shared__ u64 sc[SEL_T / WAVE + 1];
+    const u64 w = (u64)blockIdx.x * SEL_T + threadIdx.x;
+    const u64 f = w < words ? flags[w] : 0ull;
+    u64 at = block_exclusive_scan<u64>((u64)__popcll(f), sc, nullptr) + bpre[blockIdx.x * step];
+    for (u64 b = f; b; b &= b - 1) out[at++] = (u32)(w * WAVE + (u64)__ffsll((unsigned long long)b) - 1);
+}
+u64 select_flagged(dlg_ctx *ctx, const u64 *flags, u64 n, u32 *out) {
+    if (n == 0) return 0;
+    const u64 words = (n + WAVE - 1) / WAVE, nb = (n + HW_ROWS - 1) / HW_ROWS;
+    DBuf<u64> bsum(ctx, nb), tot(ctx, 1);
+    DLG_LAUNCH(ctx, DLG_K_SELECT, 8.0 * words, heads_sum_k, (unsigned)nb, SEL_T, 0, flags, words, bsum.p);
+    scan_blocks(ctx, bsum.p, nb, tot.p);
+    u64 total = 0;
+    ctx->read_scalars(tot.p, 1, &total);
+    DLG_LAUNCH(ctx, DLG_K_SELECT, 8.0 * words + 4.0 * total, heads_scatter_k, (unsigned)nb, SEL_T, 0, flags, words,
+               (const u64 *)bsum.p, 1ull, out);
+    return total;
+}
+
 u64 select(dlg_ctx *ctx, int mode, const u64 *in, u64 n, const u64 *other, u64 n_other,
            void *out) {
     if (n == 0) return 0;
@@ -1627,7 +1663,10 @@ u64 select(dlg_ctx *ctx, int mode, const u64 *in, u64 n, const u64 *other, u64 n
     u64 total = 0;
     ctx->read_scalars(tot.p, 1, &total);
     if (total == 0) return 0;
-    if (mode == SEL_KEY_HEAD)
+    if (mode == SEL_KEY_HEAD && total <= n / HW_SPARSE)
+        DLG_LAUNCH(ctx, DLG_K_SELECT, 8.0 * ((n + 63) / 64) + 4.0 * total, heads_scatter_k, (unsigned)((n + HW_ROWS - 1) / HW_ROWS),
+                   SEL_T, 0, (const u64 *)flags.p, (n + WAVE - 1) / WAVE, (const u64 *)bsum.p, HW_ROWS / SEL_TILE, (u32 *)out);
+    else if (mode == SEL_KEY_HEAD)
         DLG_LAUNCH(ctx, DLG_K_SELECT, 8.0 * ((n + 63) / 64) + 12.0 * total,
                    select_scatter_k<true>, (unsigned)nb, SEL_T, 0, in, n, flags.p, bsum.p, out);
     else
