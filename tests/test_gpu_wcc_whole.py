@@ -64,3 +64,26 @@ def test_batch_stops_each_by_its_own_rule(ctx, limit):
             continue
         same(r, want)
         assert r["nodes"] == want["nodes"]
+
+
+# one workgroup's rounds: the largest it takes and the first it does not (by edges, by nodes), stars, and stops after k rounds
+@pytest.mark.parametrize("kind,n", [("path", 15), ("path", 1023), ("path", 1025), ("path", 8192), ("path", 8193), ("star", 1), ("star", 4000),
+                                    ("star", 8192), ("star", 8194), ("random", 500), ("random", 8191), ("random", 8192), ("random", 8193),
+                                    ("loops", 500), ("loops", 16_384), ("loops", 16_385)])
+@pytest.mark.parametrize("k", [1, 2, 6])
+def test_one_workgroup(ctx, orc, kind, n, k):
+    rng = np.random.default_rng(n)
+    if kind == "path":
+        rows = np.stack([np.arange(n), np.arange(1, n + 1)], 1)
+    elif kind == "star":
+        rows = np.stack([np.full(n, n // 2), np.arange(n)], 1)
+    elif kind == "random":   # n undirected edges, each once
+        a, b = np.triu_indices(1500, 1)
+        pick = rng.choice(len(a), n, replace=False)
+        rows = np.stack([a[pick], b[pick]], 1)
+    else:
+        rows = np.stack([np.arange(n), np.arange(n)], 1)
+    rows = (rng.permutation(rows.max() + 1)[rows] if kind != "path" else rows).astype(np.int32) - 700
+    same(ctx.run("wcc", rows, max_iterations=k), ctx.run("wcc", rows, max_iterations=k, strategy=2))
+    if k == 6 and (kind != "path" or n < 2000):
+        same(ctx.run("wcc", rows), orc.wcc(rows))
