@@ -1178,7 +1178,44 @@ u64 sort_heads_small(dlg_ctx *ctx, const u64 *in, u64 n, u64 *out, u32 *heads) {
     return sort_small(ctx, in, n, out, SS_HEADS, false, heads);
 }
 
+// The bounds of a few tuples, one launch that publishes them (a fold by workgroups, one of their
+// partials and a read-back otherwise).
+__global__ __launch_bounds__(SS_T) void minmax_small_k(const u64 *data, u32 n, u64 *host, u64 seq) {
+    u32 b[4] = {0xffffffffu, 0u, 0xffffffffu, 0u};
+    for (u32 i = threadIdx.x; i < n; i += SS_T) {
+        const u64 x = data[i];
+        b[0] = min(b[0], tkey(x)); b[1] = max(b[1], tkey(x));
+        b[2] = min(b[2], tval(x)); b[3] = max(b[3], tval(x));
+    }
+    __shared__ u32 sm[4][SS_T / WAVE];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+#pragma unroll
+        for (int d = WAVE / 2; d > 0; d >>= 1) {
+            const u32 o = (u32)__shfl_xor((int)b[q], d, WAVE);
+            b[q] = q & 1 ? max(b[q], o) : min(b[q], o);
+        }
+        if (threadIdx.x % WAVE == 0) sm[q][threadIdx.x / WAVE] = b[q];
+    }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int w = 1; w < SS_T / WAVE; w++)
+        for (int q = 0; q < 4; q++) b[q] = q & 1 ? max(b[q], sm[q][w]) : min(b[q], sm[q][w]);
+    host[0] = (u64)b[1] << 32 | b[0];
+    host[1] = (u64)b[3] << 32 | b[2];
+    __threadfence_system();
+    *(volatile u64 *)(host + dlg_ctx::MAPPED_SEQ) = seq;
+    __threadfence_system();
+}
+
 void tuple_bounds(dlg_ctx *ctx, const u64 *data, u64 n, u32 *h) {
+    if (n <= SORT_SMALL_MAX) {
+        const u64 seq = ++ctx->mapped_seq;
+        DLG_LAUNCH(ctx, DLG_K_SORT_HIST, 8.0 * n, minmax_small_k, 1, SS_T, 0, data, (u32)n, ctx->mapped_dev(seq), seq);
+        ctx->wait_mapped(seq);
+        std::memcpy(h, (const void *)ctx->mapped_host(seq), 16);
+        return;
+    }
     const unsigned g = n ? (unsigned)std::min<u64>((n + 255) / 256, (u64)ctx->num_cus * 8) : 0u;
     DBuf<u32> mm(ctx, 4 + 4 * (u64)g);   // the bounds, then the workgroups' partials
     if (g) DLG_LAUNCH(ctx, DLG_K_SORT_HIST, 8.0 * n, minmax_k, g, 256, 0, data, n, mm.p + 4);
