@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstdlib>
+#include <cstring>
 
 namespace dlg {
 
@@ -156,7 +157,8 @@ struct Layout {
     int exhausted = 0;                // first instance that starts past the last id (B: none)
 };
 
-static Layout make_layout(int B, const int32_t *const *rows, const int64_t *n) {
+// mm: the instances' bounds (flipped ids: least, greatest), or null: their rows are read here.
+static Layout make_layout(int B, const int32_t *const *rows, const int64_t *n, const u32 *mm) {
     Layout L;
     L.B = B;
     L.lo.resize(B);
@@ -168,7 +170,11 @@ static Layout make_layout(int B, const int32_t *const *rows, const int64_t *n) {
         if (n[i] < 0 || (n[i] > 0 && !rows[i])) fail(DLG_INVALID_INPUT, "bad instance rows");
         if (base > (int64_t)INT32_MAX && L.exhausted == B) L.exhausted = i;
         int64_t lo = INT64_MAX, hi = INT64_MIN;
-        for (int64_t r = 0; r < 2 * n[i]; r++) {
+        if (mm && n[i]) {
+            lo = (int32_t)(mm[2 * i] ^ 0x80000000u);
+            hi = (int32_t)(mm[2 * i + 1] ^ 0x80000000u);
+        }
+        for (int64_t r = 0; !mm && r < 2 * n[i]; r++) {
             lo = std::min<int64_t>(lo, rows[i][r]);
             hi = std::max<int64_t>(hi, rows[i][r]);
         }
@@ -183,6 +189,115 @@ static Layout make_layout(int B, const int32_t *const *rows, const int64_t *n) {
     }
     L.ub[B] = base - 1 >= INT32_MAX ? 0xffffffffu : (u32)((uint64_t)(base + 2147483648LL));
     return L;
+}
+
+// The instances' rows on the device, one after the other as given, with their
+// bounds found and their ids shifted there.  The host only copies them into a page-locked
+// block, a chunk of which is on its way while the next is copied; reading 3.7M rows twice
+// more on the host for bounds and shifts, and copying from pageable memory, left the
+// device idle for 9 of a batch's 31 ms.  Fewer rows than BU_MIN don't pay for the two
+// launches and the wait; more than BU_MAX would lock 1 GiB.
+constexpr int64_t BU_MIN = 1 << 16, BU_MAX = 1ll << 27;
+constexpr int64_t BU_CHUNK = 1 << 18;   // rows
+constexpr u64 BU_SEG = 4096;            // rows a workgroup
+
+// f(instance, its first row in the segment, one past its last) for the workgroup's rows.
+template <typename F>
+__device__ __forceinline__ void bu_segments(const u64 *off, u32 B, u64 n, F f) {
+    const u64 s0 = (u64)blockIdx.x * BU_SEG, s1 = s0 + BU_SEG < n ? s0 + BU_SEG : n;
+    u32 j = 0, hi = B;   // the last instance starting at or before s0 (block-uniform)
+    while (hi - j > 1) {
+        const u32 mid = (j + hi) >> 1;
+        if (off[mid] <= s0) j = mid; else hi = mid;
+    }
+    for (; j < B && off[j] < s1; j++) {
+        const u64 i0 = off[j] > s0 ? off[j] : s0, i1 = off[j + 1] < s1 ? off[j + 1] : s1;
+        if (i0 < i1) f(j, i0, i1);
+    }
+}
+__global__ __launch_bounds__(256) void inst_bounds_k(const int2 *rows, u64 n, const u64 *off, u32 B, u32 *mm) {
+    bu_segments(off, B, n, [&](u32 j, u64 i0, u64 i1) {
+        u32 lo = 0xffffffffu, hi = 0u;
+        for (u64 i = i0 + threadIdx.x; i < i1; i += 256) {
+            const int2 r = rows[i];
+            const u32 a = (u32)r.x ^ 0x80000000u, b = (u32)r.y ^ 0x80000000u;
+            lo = min(lo, min(a, b));
+            hi = max(hi, max(a, b));
+        }
+#pragma unroll
+        for (int d = WAVE / 2; d > 0; d >>= 1) {
+            lo = min(lo, (u32)__shfl_xor((int)lo, d, WAVE));
+            hi = max(hi, (u32)__shfl_xor((int)hi, d, WAVE));
+        }
+        if (threadIdx.x % WAVE == 0 && lo <= hi) {   // a wave with rows
+            atomicMin(&mm[2 * j], lo);
+            atomicMax(&mm[2 * j + 1], hi);
+        }
+    });
+}
+__global__ __launch_bounds__(256) void inst_shift_k(int2 *rows, u64 n, const u64 *off, u32 B, const u32 *shift) {
+    bu_segments(off, B, n, [&](u32 j, u64 i0, u64 i1) {
+        const u32 s = shift[j];
+        for (u64 i = i0 + threadIdx.x; i < i1; i += 256) {
+            const int2 r = rows[i];
+            rows[i] = make_int2((int)((u32)r.x + s), (int)((u32)r.y + s));
+        }
+    });
+}
+
+struct StagingBlock {   // given back once nothing copies from it
+    dlg_ctx *ctx;
+    void *p;
+    ~StagingBlock() {
+        (void)hipStreamSynchronize(ctx->stream);
+        host_block_free(p);
+    }
+};
+
+// False: too few, too many or bad rows (the caller's own reading reports those).
+static bool upload_union(dlg_ctx *ctx, int B, const int32_t *const *rows, const int64_t *n, DBuf<int32_t> &d, DBuf<u64> &off,
+                         std::vector<u32> &mm) {
+    std::vector<u64> ho(B + 1, 0);
+    for (int i = 0; i < B; i++) {
+        if (n[i] < 0 || n[i] > BU_MAX || (n[i] > 0 && !rows[i])) return false;
+        ho[i + 1] = ho[i] + (u64)n[i];
+        if (ho[i + 1] > (u64)BU_MAX) return false;
+    }
+    const u64 N = ho[B];
+    if (N < (u64)BU_MIN) return false;
+    StagingBlock stage{ctx, host_block_alloc(8 * N)};
+    if (!stage.p) return false;
+    d.ensure(2 * N);
+    off.ensure(B + 1);
+    DBuf<u32> m(ctx, 2 * (size_t)B);
+    mm.resize(2 * (size_t)B);
+    for (int i = 0; i < B; i++) {
+        mm[2 * i] = 0xffffffffu;
+        mm[2 * i + 1] = 0u;
+    }
+    HIPCHK(hipMemcpyAsync(off.p, ho.data(), 8 * (size_t)(B + 1), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(hipMemcpyAsync(m.p, mm.data(), 8 * (size_t)B, hipMemcpyHostToDevice, ctx->stream));
+    char *h = (char *)stage.p;
+    u64 have = 0, sent = 0;   // rows
+    auto send = [&]() {
+        if (have > sent)
+            HIPCHK(hipMemcpyAsync(d.p + 2 * sent, h + 8 * sent, 8 * (have - sent), hipMemcpyHostToDevice, ctx->stream));
+        sent = have;
+    };
+    for (int i = 0; i < B; i++)
+        for (int64_t r = 0; r < n[i];) {
+            const int64_t take = std::min(n[i] - r, BU_CHUNK - (int64_t)(have - sent));
+            std::memcpy(h + 8 * have, rows[i] + 2 * r, 8 * (size_t)take);
+            have += (u64)take;
+            r += take;
+            if (have - sent == (u64)BU_CHUNK) send();
+        }
+    send();
+    DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * N, inst_bounds_k, grid_for(N, BU_SEG), 256, 0, (const int2 *)d.p, N, (const u64 *)off.p,
+               (u32)B, m.p);
+    HIPCHK(hipMemcpyAsync(mm.data(), m.p, 8 * (size_t)B, hipMemcpyDeviceToHost, ctx->stream));
+    ctx->sync();
+    return true;
 }
 
 // Boundary positions of the instance key ranges in a sorted relation.
@@ -507,8 +622,14 @@ static void wcc_batch_rounds(dlg_ctx *ctx, WccState &s, const WccGraph &g, const
 
 void batch_run(dlg_ctx *ctx, int prog, int B, const int32_t *const *rows, const int64_t *n,
                       const Opts &o, dlg_result *res, dlg_batch_stats *st) {
-    Layout L = make_layout(B, rows, n);
+    auto t0 = Clock::now();
+    DBuf<int32_t> d_rows(ctx);
+    DBuf<u64> roff(ctx);
+    std::vector<u32> mm, shift;
+    const bool up = upload_union(ctx, B, rows, n, d_rows, roff, mm);
+    Layout L = make_layout(B, rows, n, up ? mm.data() : nullptr);
     if (L.exhausted < B) {
+        d_rows.release();
         // The instances from L.exhausted on start where the ids are used up, so
         // they are empty (a wider one overflows above); their range start would
         // be the last id of the instance before them, whose tuples the range
@@ -525,8 +646,9 @@ void batch_run(dlg_ctx *ctx, int prog, int B, const int32_t *const *rows, const 
         return;
     }
     if (L.total_rows >= 0x7fffffffLL) fail(DLG_OVERFLOW, "batch has more than 2^31-2 rows");
-    std::vector<int32_t> un((size_t)(2 * L.total_rows + 2));
-    {
+    std::vector<int32_t> un;
+    if (!up) {
+        un.resize((size_t)(2 * L.total_rows + 2));
         size_t k = 0;
         for (int i = 0; i < B; i++)
             for (int64_t r = 0; r < 2 * n[i]; r++) un[k++] = (int32_t)((int64_t)rows[i][r] + L.shift[i]);
@@ -536,10 +658,19 @@ void batch_run(dlg_ctx *ctx, int prog, int B, const int32_t *const *rows, const 
         res[i].input_rows = n[i];
         res[i].raw_join_rows = -1;
     }
-    auto t0 = Clock::now();
     u64 N = (u64)L.total_rows;
-    DBuf<int32_t> d_rows(ctx, 2 * (N ? N : 1));
-    if (N)
+    if (up) {
+        shift.resize(B);
+        for (int i = 0; i < B; i++) shift[i] = (u32)L.shift[i];
+        DBuf<u32> dsh(ctx, B);
+        HIPCHK(hipMemcpyAsync(dsh.p, shift.data(), 4 * (size_t)B, hipMemcpyHostToDevice, ctx->stream));
+        DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * N, inst_shift_k, grid_for(N, BU_SEG), 256, 0, (int2 *)d_rows.p, N,
+                   (const u64 *)roff.p, (u32)B, (const u32 *)dsh.p);
+    } else {
+        t0 = Clock::now();
+        d_rows.ensure(2 * (N ? N : 1));
+    }
+    if (N && !up)
         HIPCHK(hipMemcpyAsync(d_rows.p, un.data(), sizeof(int32_t) * 2 * N, hipMemcpyHostToDevice,
                               ctx->stream));
     DBuf<u32> ub(ctx, B + 1);
