@@ -550,16 +550,27 @@ static void split_rows(dlg_ctx *ctx, const u64 *d, const std::vector<u64> &b, co
                    (const u64 *)bnd.p, (const u32 *)dsh.p, (u32)L.B, orient, both ? 1 : 0, rows.p);
         ctx->sync();   // the host vectors go out of scope
     }
+    // Every block before the first copy: where one cannot be had, nothing is on its way
+    // into those that the caller gives back (a block given back goes to the next that asks
+    // for one, another thread's too).
     for (int i = 0; i < L.B; i++) {
         const u64 cnt = b[i + 1] - b[i];
         res[i].n_rows = (int64_t)cnt;
         res[i].rows = (int32_t *)host_block_alloc(sizeof(int32_t) * 2 * (cnt ? cnt : 1));
         if (!res[i].rows) fail(DLG_OUT_OF_MEMORY, "host allocation of batch rows");
-        if (cnt)
-            HIPCHK(hipMemcpyAsync(res[i].rows, rows.p + 2 * b[i], sizeof(int32_t) * 2 * cnt, hipMemcpyDeviceToHost,
-                                  ctx->stream));
     }
-    ctx->sync();
+    try {
+        for (int i = 0; i < L.B; i++) {
+            const u64 cnt = b[i + 1] - b[i];
+            if (cnt)
+                HIPCHK(hipMemcpyAsync(res[i].rows, rows.p + 2 * b[i], sizeof(int32_t) * 2 * cnt, hipMemcpyDeviceToHost,
+                                      ctx->stream));
+        }
+        ctx->sync();
+    } catch (...) {
+        (void)hipStreamSynchronize(ctx->stream);
+        throw;
+    }
 }
 
 // The rounds of a batch's WCC union, pushed from the frontier: per round the

@@ -124,6 +124,7 @@ std::unordered_map<void *, size_t> pinned_blocks;   // handed out: size class
 std::map<size_t, std::vector<void *>> pinned_free;
 size_t pinned_total = 0, pinned_kept = 0;           // total: handed out and kept
 int contexts = 0;
+std::atomic<int64_t> blocks_until_failure{-1};      // for tests: < 0 none
 
 // Takes kept blocks out of the books, largest first, until at most `keep` bytes
 // remain; the caller frees them without the lock.
@@ -155,6 +156,7 @@ void host_contexts(int change) {
 }
 
 void *host_block_alloc(size_t bytes) {
+    if (blocks_until_failure.load(std::memory_order_relaxed) >= 0 && blocks_until_failure.fetch_sub(1) == 0) return nullptr;
     const size_t sz = Pool::round_size(bytes);
     if (bytes <= PINNED_BLOCK_MAX) {
         std::vector<void *> gone;
@@ -369,6 +371,10 @@ void dlg_ctx_destroy(dlg_ctx *c) {
 const char *dlg_last_error(const dlg_ctx *c) { return c ? c->last_error.c_str() : "null context"; }
 
 void dlg_host_free(void *p) { host_block_free(p); }
+
+// For tests: of the host blocks that the library allocates from now on, the one after the
+// next n fails, once.  (Not in the header.)
+void dlg_test_fail_host_block(int64_t n) { blocks_until_failure.store(n); }
 
 dlg_status dlg_ctx_sync(dlg_ctx *c) {
     if (!c) return DLG_INVALID_INPUT;

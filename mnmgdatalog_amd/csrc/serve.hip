@@ -225,14 +225,19 @@ void run_unit(dlg_server *s, dlg_ctx *ctx, std::vector<Request *> &batch, dlg_st
             int B = (int)batch.size();
             std::vector<const int32_t *> ptrs(B);
             std::vector<int64_t> ns(B);
-            std::vector<dlg_result> out(B);
+            std::vector<dlg_result> out(B);   // cleared: freed below if the batch fails
             for (int i = 0; i < B; i++) {
                 ptrs[i] = batch[i]->rows.data();
                 ns[i] = batch[i]->n;
             }
             dlg_batch_stats bst;
             std::memset(&bst, 0, sizeof(bst));
-            batch_run(ctx, r0->prog, B, ptrs.data(), ns.data(), s->opts, out.data(), &bst);
+            try {
+                batch_run(ctx, r0->prog, B, ptrs.data(), ns.data(), s->opts, out.data(), &bst);
+            } catch (...) {
+                for (dlg_result &r : out) dlg_result_free(&r);
+                throw;
+            }
             for (int i = 0; i < B; i++) {
                 batch[i]->res = out[i];
                 batch[i]->res.device_seconds = bst.device_seconds;
