@@ -781,6 +781,8 @@ extern "C" dlg_status dlg_batch_run(dlg_ctx *ctx, int prog, int32_t count, const
                                     dlg_batch_stats *stats) {
     if (!ctx || count < 0 || (count && (!h_rows || !n || !results)) || !stats) return DLG_INVALID_INPUT;
     std::memset(stats, 0, sizeof(*stats));
+    // freed below whatever fails, and read by a caller who looks at the rows first
+    for (int i = 0; i < count; i++) std::memset(&results[i], 0, sizeof(dlg_result));
     if (count == 0) return DLG_OK;
     API_BEGIN(ctx)
     Opts op = read_opts(ctx, o);

@@ -1,7 +1,7 @@
 """A batch that fails while its rows go to the host: its blocks, which the next call may be given, are not written
 any more once the call has returned."""
 import time
-from ctypes import c_int64
+from ctypes import byref, c_int64, c_void_p, memset, sizeof
 
 import numpy as np
 import pytest
@@ -56,3 +56,17 @@ def test_served_batch_fails():
     assert all(g["status"] == 0 for g in got)
     for i, g in enumerate(got[1:]):
         assert np.array_equal(g["rows"], closure(40 + i))
+
+
+@pytest.mark.parametrize("total", [10, 70_000])
+def test_results_given_uncleared(total):
+    """Results that hold what the caller left in them, and a batch refused before any is filled in: ids that do not fit."""
+    inst = [np.array([[-2**31, 2**31 - 1]] * total, np.int32), np.array([[0, 1]], np.int32)]
+    with dlg.Ctx(0) as ctx:
+        ptrs = (c_void_p * 2)(*[a.ctypes.data for a in inst])
+        ns = (c_int64 * 2)(*[len(a) for a in inst])
+        res, st, o = (dlg.Result * 2)(), dlg.BatchStats(), dlg.Opts()
+        memset(byref(res), 0x5a, sizeof(res))
+        s = ctx.L.dlg_batch_run(ctx.h, dlg.PROGS["tc"], 2, ptrs, ns, byref(o), res, byref(st))
+        assert s == dlg.DLG_OVERFLOW
+        assert all(not r.rows and r.n_rows == 0 for r in res)
