@@ -934,61 +934,78 @@ void bitmap_self_join(dlg_ctx *ctx, const u64 *rows, u64 n, const u64 *dense, Bi
 // wave scan), sorts them there (bitonic), keeps the first of each value and
 // writes them at the row's place in a candidate array; a scan of the kept
 // counts then places each row in the output.  Rows with more than SJW_CAP
-// candidates are left to the sorted raw join (the host checks the maximum).
-constexpr int SJW_T = 256, SJW_W = SJW_T / WAVE, SJW_RAW = 4;
+// candidates are materialised and sorted together (the host checks the maximum).
+constexpr int SJW_T = 256, SJW_W = SJW_T / WAVE, SJW_RAW = 4, SJW_REG = 4;
 
 __device__ __forceinline__ void sjw_sync() {   // LDS written by some lanes of a wave, read by others
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     __builtin_amdgcn_wave_barrier();
 }
 
+// Rows the register kernel takes: at most SJW_REG * WAVE candidates from at
+// most WAVE b's (empty rows too).
+__device__ __forceinline__ bool sjw_small(u64 raw, u64 nb) { return raw <= (u64)SJW_REG * WAVE && nb <= (u64)WAVE; }
+
 // rraw[c] = c's candidates: the sum over c's run of the run lengths of its b's;
-// the largest to mx[0], the longest run of b's to mx[1].
-__global__ __launch_bounds__(256) void sj_row_raw_k(const u32 *col, const u64 *dense, u64 W, u64 *rraw,
+// the largest to mx[0].  The rows that sj_row_sort_k takes are listed, in no
+// order, their number in mx[1]: one atomic a workgroup, not a wave.
+__global__ __launch_bounds__(256) void sj_row_raw_k(const u32 *col, const u64 *dense, u64 W, u64 *rraw, u32 *list,
                                                     unsigned long long *mx) {
-    __shared__ u64 s_m[2][256 / WAVE];
-    u64 m = 0, mb = 0;
-    const u64 stride = (u64)gridDim.x * blockDim.x;
-    for (u64 c = (u64)blockIdx.x * blockDim.x + threadIdx.x; c < W; c += stride) {
+    __shared__ u64 s_m[256 / WAVE], s_at;
+    __shared__ u32 s_n[256 / WAVE];
+    const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
+    u64 m = 0;
+    const u64 stride = (u64)gridDim.x * 256;
+    for (u64 base = (u64)blockIdx.x * 256; base < W; base += stride) {   // block-uniform
+        const u64 c = base + threadIdx.x;
         u64 t = 0;
-        const u64 p0 = dense[c], p1 = dense[c + 1];
-        for (u64 p = p0; p < p1; p += SJW_RAW) {   // SJW_RAW b's in flight; past the run, its last one again (not counted)
-            u32 b[SJW_RAW];
-            u64 d0[SJW_RAW], d1[SJW_RAW];
+        bool sort = false;
+        if (c < W) {
+            const u64 p0 = dense[c], p1 = dense[c + 1];
+            for (u64 p = p0; p < p1; p += SJW_RAW) {   // SJW_RAW b's in flight; past the run, its last one again (not counted)
+                u32 b[SJW_RAW];
+                u64 d0[SJW_RAW], d1[SJW_RAW];
 #pragma unroll
-            for (int i = 0; i < SJW_RAW; i++) b[i] = col[min(p + i, p1 - 1)];
+                for (int i = 0; i < SJW_RAW; i++) b[i] = col[min(p + i, p1 - 1)];
 #pragma unroll
-            for (int i = 0; i < SJW_RAW; i++) {
-                d0[i] = dense[b[i]];
-                d1[i] = dense[b[i] + 1];
+                for (int i = 0; i < SJW_RAW; i++) {
+                    d0[i] = dense[b[i]];
+                    d1[i] = dense[b[i] + 1];
+                }
+#pragma unroll
+                for (int i = 0; i < SJW_RAW; i++) t += p + i < p1 ? d1[i] - d0[i] : 0;
             }
-#pragma unroll
-            for (int i = 0; i < SJW_RAW; i++) t += p + i < p1 ? d1[i] - d0[i] : 0;
+            rraw[c] = t;
+            m = t > m ? t : m;
+            sort = !sjw_small(t, p1 - p0) && t <= SJW_CAP;
         }
-        rraw[c] = t;
-        m = t > m ? t : m;
-        mb = p1 - p0 > mb ? p1 - p0 : mb;
+        const u64 bal = __ballot(sort);
+        if (lane == 0) s_n[wv] = (u32)__popcll(bal);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            u32 n = 0;
+            for (int w = 0; w < 256 / WAVE; w++) n += s_n[w];
+            if (n) s_at = atomicAdd(mx + 1, (unsigned long long)n);
+        }
+        __syncthreads();
+        if (sort) {
+            u64 at = s_at + (u64)__popcll(bal & lanemask_lt());
+            for (int w = 0; w < wv; w++) at += s_n[w];
+            list[at] = (u32)c;
+        }
+        __syncthreads();   // s_n and s_at are rewritten
     }
 #pragma unroll
     for (int o = WAVE / 2; o > 0; o >>= 1) {
-        const u64 x = __shfl_xor(m, o, WAVE), y = __shfl_xor(mb, o, WAVE);
+        const u64 x = __shfl_xor(m, o, WAVE);
         m = x > m ? x : m;
-        mb = y > mb ? y : mb;
     }
-    if ((threadIdx.x & (WAVE - 1)) == 0) {
-        s_m[0][threadIdx.x / WAVE] = m;
-        s_m[1][threadIdx.x / WAVE] = mb;
-    }
+    if (lane == 0) s_m[wv] = m;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < 256 / WAVE; w++) {
-            m = s_m[0][w] > m ? s_m[0][w] : m;
-            mb = s_m[1][w] > mb ? s_m[1][w] : mb;
-        }
+        for (int w = 1; w < 256 / WAVE; w++) m = s_m[w] > m ? s_m[w] : m;
         // an atomic only where it can still raise the maximum (a stale read only costs an atomic)
         if (m > __hip_atomic_load(mx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(mx, (unsigned long long)m);
-        if (mb > __hip_atomic_load(mx + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            atomicMax(mx + 1, (unsigned long long)mb);
     }
 }
 
@@ -1057,7 +1074,6 @@ __device__ __forceinline__ void sjw_stages(u32 (&v)[R]) {
 // is paid at each of the 27 stages of 128 values, the kernel below took 1.18 ms
 // for 1e8 candidates in 1e6 rows; with these, and scans for the binary searches over
 // the runs, 0.71.
-constexpr int SJW_REG = 4;
 template <int R>
 __device__ __forceinline__ void sjw_sort_regs(u32 (&v)[R]) {
     static_assert(R == 1 || R == 2 || R == 4, "a power of two");
@@ -1083,10 +1099,6 @@ __device__ __forceinline__ u32 sjw_scan_max(u32 v) {
     v = max(v, (u32)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false));
     return v;
 }
-
-// Rows the register kernel takes: at most SJW_REG * WAVE candidates from at
-// most WAVE b's (empty rows too).
-__device__ __forceinline__ bool sjw_small(u64 raw, u64 nb) { return raw <= (u64)SJW_REG * WAVE && nb <= (u64)WAVE; }
 
 // A small row's candidates j = r WAVE + lane: the lane whose run holds j is the
 // largest one that starts at or before it, a maximum scan over the starts (each
@@ -1158,34 +1170,22 @@ __global__ __launch_bounds__(256) void sj_row_small_k(const u32 *col, const u64 
     }
 }
 
-__global__ __launch_bounds__(SJW_T) void sj_row_sort_k(const u32 *col, const u64 *dense, const u64 *roff, u64 W,
-                                                       u32 *cand, u32 *ucnt) {
+// The listed rows, one to a wave: those of more candidates or b's than sj_row_small_k
+// takes, up to SJW_CAP candidates.  Bound by LDS (the network's steps), so the rows are
+// spread over every wave that fits, wherever in the range they lie.  Whole joins, with a
+// wave looking through 64 rows in turn for those to sort, with a row of any kind to a wave, and
+// with the list: 600,000 rows over 30,000 ids 3.87, 1.09, 1.01 ms; 3M over 100,000 10.3, 5.5,
+// 5.4; 6M over 400,000 3.64, 3.91, 2.84; 10M over 1M (hardly any to sort) 2.01, 2.79, 2.00.
+__global__ __launch_bounds__(SJW_T) void sj_row_sort_k(const u32 *col, const u64 *dense, const u64 *roff, const u32 *list,
+                                                       u64 n, u32 *cand, u32 *ucnt) {
     __shared__ u32 s_buf[SJW_W][SJW_CAP];
     __shared__ u64 s_pre[SJW_W][WAVE + 1];
     __shared__ u64 s_q0[SJW_W][WAVE];
     const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
     u32 *buf = s_buf[wv];
     u64 *pre = s_pre[wv], *q0s = s_q0[wv];
-    // 64 rows a look, as most are sj_row_small_k's (1e6 rows with hardly any to sort: 158 -> 87 us)
-    u64 mine = 0, base = ((u64)blockIdx.x * SJW_W + wv) * WAVE;
-    const u64 step = (u64)gridDim.x * SJW_W * WAVE;
-    bool fresh = true;
-    while (true) {   // wave-uniform
-        if (!mine) {
-            if (!fresh) base += step;
-            fresh = false;
-            if (base >= W) break;
-            const u64 l = base + (u64)lane;
-            bool is = false;
-            if (l < W) {
-                const u64 n = roff[l + 1] - roff[l];
-                is = !sjw_small(n, dense[l + 1] - dense[l]) && n <= SJW_CAP;   // the others: sj_row_small_k's, or heavy rows
-            }
-            mine = __ballot(is);
-            continue;
-        }
-        const u64 c = base + (u64)(__ffsll((unsigned long long)mine) - 1);
-        mine &= mine - 1;
+    for (u64 k = (u64)blockIdx.x * SJW_W + wv; k < n; k += (u64)gridDim.x * SJW_W) {   // wave-uniform
+        const u64 c = list[k];
         const u64 r0 = roff[c], raw = roff[c + 1] - r0;
         const u64 p1 = dense[c + 1];
         // gather the row's candidates into buf[0, raw)
@@ -1415,13 +1415,13 @@ bool self_join_rows(dlg_ctx *ctx, const u64 *rows, u64 n, const u64 *dense, u32 
     DBuf<u32> col(ctx, n);
     DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * n, sj_col_k, sgrid(ctx, n), ctx->block_size, 0, rows, n, lo, col.p);
     DBuf<u64> roff(ctx, W + 1), mx(ctx, 2);
+    DBuf<u32> list(ctx, W);
     fill_u64(ctx, mx.p, 2, 0ull);
     DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * W + 12.0 * n, sj_row_raw_k, sgrid(ctx, W), 256, 0, (const u32 *)col.p, dense,
-               W, roff.p, (unsigned long long *)mx.p);
+               W, roff.p, list.p, (unsigned long long *)mx.p);
     u64 hm[2];
     ctx->read_scalars(mx.p, 2, hm);
-    const u64 m = hm[0];
-    const bool big_b = hm[1] > (u64)WAVE;   // a row with more b's than the register kernel takes
+    const u64 m = hm[0], nsort = hm[1];
     scan_u64_async(ctx, roff.p, W, roff.p, roff.p + W);   // roff[W] = all candidates
     u64 total = 0;
     ctx->read_scalars(roff.p + W, 1, &total);
@@ -1431,9 +1431,11 @@ bool self_join_rows(dlg_ctx *ctx, const u64 *rows, u64 n, const u64 *dense, u32 
     const unsigned g = (unsigned)std::min<u64>((W + SJW_W - 1) / SJW_W, (u64)ctx->num_cus * 8);
     DLG_LAUNCH(ctx, DLG_K_BITMAP_INSERT, 8.0 * total + 8.0 * n + 16.0 * W, sj_row_small_k, g, 256, 0,
                (const u32 *)col.p, dense, (const u64 *)roff.p, W, cand.p, ucnt.p);
-    if (m > (u64)SJW_REG * WAVE || big_b)
-        DLG_LAUNCH(ctx, DLG_K_BITMAP_INSERT, 16.0 * W, sj_row_sort_k, g, SJW_T, 0, (const u32 *)col.p, dense,
-                   (const u64 *)roff.p, W, cand.p, ucnt.p);
+    if (nsort)
+        DLG_LAUNCH(ctx, DLG_K_BITMAP_INSERT, 20.0 * nsort, sj_row_sort_k,
+                   (unsigned)std::min<u64>((nsort + SJW_W - 1) / SJW_W, (u64)ctx->num_cus * 8), SJW_T, 0, (const u32 *)col.p,
+                   dense, (const u64 *)roff.p, (const u32 *)list.p, nsort, cand.p, ucnt.p);
+    list.release();   // what is queued reads it first: a block of the stream's own pool
     if (m > SJW_CAP) {   // heavy rows: their candidates materialised, sorted and deduplicated
         DBuf<u64> hoff(ctx, W + 1);
         DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * W, sj_heavy_raw_k, sgrid(ctx, W), ctx->block_size, 0, (const u64 *)roff.p,

@@ -32,3 +32,23 @@ def test_counts(ctx, orc, runs, count):
     got, want = ctx.run("single_join", rows, strategy=2), orc.single_join(rows)
     assert got["output_size"] == want["output_size"]
     assert np.array_equal(got["rows"], want["rows"])
+
+
+@pytest.mark.parametrize("every", [1, 2, 63, 65, 4000])
+@pytest.mark.parametrize("n", [1, 3, 255, 256, 257, 5000])
+def test_rows_to_sort(ctx, orc, n, every):
+    """`n` output rows, every `every`-th of them (and the first) of 300 candidates, which go through LDS, the others of
+    two: listed rows at the edges of workgroups, all, few and one of them; one row too long for LDS beside them."""
+    rng = np.random.default_rng(7 * n + every)
+    c = np.arange(n)
+    many = c % every == 0
+    a = 10_000 + np.arange(3000)
+    b = 20_000 + np.where(many, 0, 1 + c % 50)                     # row c: one b, shared by the rows of many
+    parts = [np.stack([b, c], 1), np.stack([rng.choice(a, 300, replace=False), np.full(300, 20_000)], 1)]
+    for k in range(50):
+        parts.append(np.stack([rng.choice(a, 2, replace=False), np.full(2, 20_001 + k)], 1))
+    parts += [[[30_000, n + 1]], np.stack([a, np.full(3000, 30_000)], 1), [[399_999, 399_998]]]
+    rows = np.concatenate(parts).astype(np.int32)
+    got, want = ctx.run("single_join", rows, strategy=2), orc.single_join(rows)
+    assert got["output_size"] == want["output_size"]
+    assert np.array_equal(got["rows"], want["rows"])
