@@ -357,6 +357,12 @@ u64 hashrel_insert_join(dlg_ctx *ctx, HashRel &r, const Index &ix, const u64 *pr
 // 27 -> 12.6 us) 82 -> 38; 3,000 power-law ids in a wide range 3.9 -> 3.5.
 constexpr int HR_DEPTH = 3, HR_SETS = 4;
 constexpr u64 HR_ROWS = 1ull << 14;
+// Room that rounds queued ahead may ask for beyond the relation: what the largest of them
+// take when every row is new, or a quarter of the relation.  The room is counted in join rows,
+// as a tile cannot know which of its own are new; a round of many more rows than new tuples
+// (cliques) runs by itself, which asks for room as its tuples come: 700 ids with 40,000 edges
+// held 840 MB for 490,000 tuples, and hold 82 so (2.0 -> 2.2 ms).
+constexpr u64 HR_ROOM = 2 * (HR_DEPTH + 1) * HJ_BIG_MIN;
 static_assert(HR_DEPTH + 2 <= dlg_ctx::MAPPED_SLOTS, "every queued round has a mapped slot of its own");
 
 struct HrState {
@@ -462,12 +468,13 @@ int hashrel_rounds(dlg_ctx *ctx, HashRel &r, const Index &ix, u64 off, u64 n, in
         return n != 0 && !(max_it > 0 && it >= max_it);
     };
     while (true) {
-        if (plain || n >= HJ_BIG_MIN) {   // large rounds have threads of several rows each
+        const u64 ahead = 2 * (HR_DEPTH + 1) * per;
+        if (plain || n >= HJ_BIG_MIN || ahead > std::max(HR_ROOM, r.n / 4)) {   // large rounds have threads of several rows each
             if (!alone(r.n)) return it;
             continue;
         }
         try {
-            hs_grow(ctx, r, 2 * (HR_DEPTH + 1) * per);
+            hs_grow(ctx, r, ahead);
         } catch (const Error &e) {   // no memory for so many rounds at once
             if (e.status != DLG_OUT_OF_MEMORY) throw;
             plain = true;

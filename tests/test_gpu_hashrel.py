@@ -1,5 +1,7 @@
 """TC and SG over wide id ranges: join rows inserted into the hash set as they are formed, against the
 oracle and the sorted-run layout (strategy 2)."""
+from ctypes import CDLL, byref, c_size_t
+
 import numpy as np
 import pytest
 
@@ -92,3 +94,23 @@ def test_tight_budget(orc):
             got = srv.wait(srv.submit("tc", rows))
         assert got["status"] == 0
         same(got, want)
+
+
+def free_bytes():
+    free, total = c_size_t(), c_size_t()
+    assert CDLL("libamdhip64.so").hipMemGetInfo(byref(free), byref(total)) == 0   # the library that libdlg.so has loaded
+    return free.value
+
+
+def test_room_by_new_tuples():
+    """Rounds of 7 and more times as many join rows as new tuples: the set takes room for its tuples, not for the rows."""
+    rows = (np.random.default_rng(6).integers(0, 700, size=(40_000, 2)) * 4096).astype(np.int32)
+    with dlg.Ctx(0) as c:
+        c.run("tc", rows[:100], keep_output=False, strategy=3)
+        free = free_bytes()
+        got = c.run("tc", rows, keep_output=False, strategy=3, check_output=1)
+        used = free - free_bytes()
+        want = c.run("tc", rows, keep_output=False, strategy=2, check_output=1)
+    assert got["output_size"] == 490_000 and got["output_sum"] == want["output_sum"]
+    assert (got["iterations"], got["raw_join_rows"]) == (want["iterations"], want["raw_join_rows"])
+    assert used < 256 << 20
