@@ -630,6 +630,7 @@ struct HashRel {
     HashSet hs;
     u64 n = 0, limit = 0;
     double lf;
+    bool tight = false;   // there was no memory for the room asked for
     HashRel(dlg_ctx *c, double load_factor) : all(c), count(c), hs(c), lf(load_factor) {}
 };
 // The tuples of x (any order, duplicates allowed) that are absent, appended.  Returns their number.

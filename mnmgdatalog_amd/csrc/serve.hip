@@ -83,8 +83,9 @@ double now_s(const dlg_server *s) { return secs(s->t0, Clock::now()); }
 // W * ceil(W / 32) words each (SG: F, the round's maps D and R; TC by row ORs
 // has three maps, at most 32 MiB more, which the slack covers), plus the
 // sorted output and the round buffers, about 32 B per output tuple, plus
-// the edge index.  Wider ranges keep F as sorted tuples with a hash set and
-// a final sort: about 48 B per output tuple.  The output is |TC| by SCC
+// the edge index.  Wider ranges keep F as an array of tuples with a hash set and
+// a final sort: 48 B per output tuple, which the set keeps to where its usual growth would
+// take more (k_hashset.hip).  The output is |TC| by SCC
 // condensation (dlg_predict_tc_size, estimates padded by a quarter), or the
 // bound nodes^2 (SG; TC when even the bound fits or the request has more than
 // PREDICT_MAX_ROWS rows), with nodes bounded by the id range and twice the rows.

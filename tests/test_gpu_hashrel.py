@@ -114,3 +114,14 @@ def test_room_by_new_tuples():
     assert got["output_size"] == 490_000 and got["output_sum"] == want["output_sum"]
     assert (got["iterations"], got["raw_join_rows"]) == (want["iterations"], want["raw_join_rows"])
     assert used < 256 << 20
+
+
+@pytest.mark.parametrize("n,m,seed", [(1159, 2643, 6), (6599, 10_613, 42), (7046, 13_037, 56), (1199, 2767, 69)])
+def test_served_within_its_reservation(ctx, n, m, seed):
+    """Served closures over a wide id range keep within the memory reserved for them: none is run a second time."""
+    ids = np.sort(np.random.default_rng(5).choice(2**31 - 1, n, replace=False)).astype(np.int32)
+    rows = ids[np.random.default_rng(seed).integers(0, n, (m, 2))]
+    with dlg.Server(0, workers=2, hbm_budget=40 << 30, retain_bytes=1) as srv:
+        got = srv.wait(srv.submit("tc", rows))
+    assert got["status"] == 0 and got["attempts"] == 1
+    same(got, ctx.run("tc", rows, strategy=2))
