@@ -308,16 +308,29 @@ void tc_fixpoint(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, Phas
     if (tc_use_dense(o, n, ib, blocks)) {
         edge.release();
         J.release();
+        delta.release();
         pc.mark(DLG_PH_JOIN);
         u64 total = 0, raw = 0;
         std::vector<int> first_empty;
-        out.iterations = tc_dense_run(ctx, d_rows, n, ib[0], ib[1], blocks, o.max_it, out.full, &total, &raw,
-                                      hook ? &first_empty : nullptr);
-        if (hook) hook->on_finished(first_empty);
-        pc.mark(DLG_PH_FINAL);
-        out.raw += (i64)raw;
-        out.nfull = total;
-        return;
+        bool done = true;
+        try {
+            out.iterations = tc_dense_run(ctx, d_rows, n, ib[0], ib[1], blocks, o.max_it, out.full, &total, &raw,
+                                          hook ? &first_empty : nullptr);
+        } catch (const Error &e) {   // three maps; the row kernel has one beside its lists
+            if (e.status != DLG_OUT_OF_MEMORY) throw;
+            done = false;
+        }
+        if (done) {
+            if (hook) hook->on_finished(first_empty);
+            pc.mark(DLG_PH_FINAL);
+            out.raw += (i64)raw;
+            out.nfull = total;
+            return;
+        }
+        out.full.release();
+        edge.ensure(n);
+        J.ensure(n);
+        pack_rows(ctx, d_rows, n, DLG_ORIENT_KV, edge.p);
     }
     pc.mark(DLG_PH_HASHTABLE);
     Index ix(ctx);

@@ -275,6 +275,15 @@ __device__ __forceinline__ u32 td_block_of(const TdBlock *blk, u32 nblk, u32 row
     return a;
 }
 
+// zero[0, zn), F[0, mn) and D[0, mn) cleared.
+__global__ void td_clear_k(u64 *zero, u64 zn, u64 *F, u64 *D, u64 mn) {
+    const u64 stride = (u64)gridDim.x * blockDim.x;
+    for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < zn || i < mn; i += stride) {
+        if (i < zn) zero[i] = 0;
+        if (i < mn) F[i] = D[i] = 0;
+    }
+}
+
 // The predecessor lists (indeg counts down to each list's next free place),
 // the edges' bits in F and D with their tasks' flags, their distinct count and next join rows (slot
 // of round 0), and the rows with long lists.
@@ -583,20 +592,20 @@ int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, con
     a.done = nlong + 1;
     a.nlong = nlong;
     a.outdeg = outdeg;
-    DBuf<u32> map(ctx, 3 * words);   // F, then D twice (a round reads one and writes the other)
+    DBuf<u32> F(ctx, words), D2(ctx, 2 * words);   // D twice: a round reads one and writes the other
     DBuf<u64> flags2(ctx, fw ? fw : 1), off(ctx, W + 1), tab(ctx, sizeof(TdBlock) / 8 * nblk);
     DBuf<u32> adj(ctx, n), wgblk(ctx);
     DBuf<uint2> longs(ctx, n / TD_LONG + 1);
-    a.F = map.p;
-    u32 *D[2] = {map.p + words, map.p + 2 * words};
+    a.F = F.p;
+    u32 *D[2] = {D2.p, D2.p + words};
     unsigned char *fl[2] = {flags, (unsigned char *)flags2.p};
     a.blk = (const TdBlock *)tab.p;
     a.off = off.p;
     a.adj = adj.p;
     a.longs = longs.p;
     HIPCHK(hipMemcpyAsync(tab.p, hb.data(), sizeof(TdBlock) * nblk, hipMemcpyHostToDevice, ctx->stream));
-    fill_u64(ctx, zero.p, zw, 0ull);
-    fill_u64(ctx, (u64 *)map.p, words, 0ull);   // F and the first D: 2 * words u32s
+    DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * (zw + words), td_clear_k, sgrid(ctx, std::max(zw, words / 2)), ctx->block_size, 0, zero.p, zw,
+               (u64 *)F.p, (u64 *)D[0], words / 2);
     a.wgblk = nullptr;
     if (nblk > 1) {
         wgblk.ensure(nwg);
@@ -605,7 +614,6 @@ int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, con
     }
     DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * n, td_hist_k, sgrid(ctx, n), ctx->block_size, 0, (const int2 *)d_rows, n, lo,
                indeg, outdeg);
-    DBuf<u64> tot(ctx, 1);
     scan_u32_u64_async(ctx, indeg, W, off.p, off.p + W);
     const unsigned fg = (unsigned)std::min<u64>((std::max(n, W) + TD_T - 1) / TD_T, (u64)ctx->num_cus * 8);
     DLG_LAUNCH(ctx, DLG_K_MISC, 40.0 * n, td_fill_k, fg, TD_T, 0, (const int2 *)d_rows, n, lo, W, a, indeg, adj.p, D[0],
@@ -654,6 +662,7 @@ int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, con
         iters->assign(st.size() - 1, 1);   // a range without rows finds nothing in round one
         for (u32 b = 0; b < nblk; b++) (*iters)[owner[b]] = nblk > 1 && h[b] ? (int)h[b] : it;
     }
+    D2.release();   // before the relation itself is allocated
     bitmap_emit_tiled(ctx, a.F, maps, words, out, *total);
     return it;
 }

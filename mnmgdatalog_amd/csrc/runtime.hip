@@ -375,6 +375,12 @@ void dlg_host_free(void *p) { host_block_free(p); }
 // For tests: of the host blocks that the library allocates from now on, the one after the
 // next n fails, once.  (Not in the header.)
 void dlg_test_fail_host_block(int64_t n) { blocks_until_failure.store(n); }
+// For tests: the device memory that the context may hold from now on (0: any), its kept
+// blocks given back first.  (Not in the header.)
+void dlg_test_budget(dlg_ctx *c, uint64_t bytes) {
+    c->pool->trim();
+    c->pool->set_budget(bytes);
+}
 
 dlg_status dlg_ctx_sync(dlg_ctx *c) {
     if (!c) return DLG_INVALID_INPUT;

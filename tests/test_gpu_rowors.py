@@ -1,5 +1,7 @@
 """TC by row ORs (id ranges up to 2^14 ids): the relation, round count and join rows at the edges of its
 words, chunks, tasks and long-list rows, against the oracle and the row kernel (which `queue` selects)."""
+from ctypes import c_uint64
+
 import numpy as np
 import pytest
 
@@ -137,3 +139,32 @@ def test_one_workgroup_hubs(ctx, orc, hubs, k):
     got = ctx.run("tc", rows, **kw)
     same(got, orc.tc(rows, **kw))
     assert got["raw_join_rows"] == ctx.run("tc", rows, queue=1, **kw)["raw_join_rows"]
+
+
+def budget(ctx, mb):
+    ctx.L.dlg_test_budget(ctx.h, c_uint64(int(mb * (1 << 20))))
+
+
+# 16,384 ids: maps of 32 MB, the row ORs' three in 96; the row kernel's one and its copy for the read-out in 64.  With
+# small ranges beside it a map is a little larger, in blocks of 40 MB (the pool's size class): 120 and 80.
+@pytest.mark.parametrize("batch", [False, True])
+@pytest.mark.parametrize("mb", [1, 8, 31, 33, 50, 65, 80, 95, 97, 99, 128])
+def test_short_of_memory(ctx, orc, batch, mb):
+    inst = [graph(16384, 9000, 1)] if not batch else [graph(16384, 9000, 1), graph(300, 400, 2), graph(20, 9, 3)]
+
+    def run():
+        return ctx.batch_run("tc", inst)[0] if batch else [ctx.run("tc", inst[0])]
+
+    budget(ctx, mb)
+    try:
+        got = run()
+    except dlg.DlgError as e:
+        assert e.status == dlg.DLG_OUT_OF_MEMORY and mb < (95 if batch else 80)
+        got = None
+    finally:
+        budget(ctx, 0)
+    for g in (got, run()):   # and what follows it
+        for r, rows in zip(g or [], inst):
+            same(r, orc.tc(rows))
+            if not batch:
+                assert r["raw_join_rows"] == ctx.run("tc", rows, queue=1)["raw_join_rows"]
