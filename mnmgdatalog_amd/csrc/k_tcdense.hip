@@ -276,12 +276,10 @@ __device__ __forceinline__ u32 td_block_of(const TdBlock *blk, u32 nblk, u32 row
 }
 
 // zero[0, zn), F[0, mn) and D[0, mn) cleared.
-__global__ void td_clear_k(u64 *zero, u64 zn, u64 *F, u64 *D, u64 mn) {
-    const u64 stride = (u64)gridDim.x * blockDim.x;
-    for (u64 i = (u64)blockIdx.x * blockDim.x + threadIdx.x; i < zn || i < mn; i += stride) {
-        if (i < zn) zero[i] = 0;
-        if (i < mn) F[i] = D[i] = 0;
-    }
+__global__ void td_clear_k(u64 *zero, u64 zn, uint4 *F, uint4 *D, u64 mn) {
+    const u64 i0 = (u64)blockIdx.x * blockDim.x + threadIdx.x, stride = (u64)gridDim.x * blockDim.x;
+    for (u64 i = i0; i < mn; i += stride) F[i] = D[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (u64 i = i0; i < zn; i += stride) zero[i] = 0;
 }
 
 // The predecessor lists (indeg counts down to each list's next free place),
@@ -604,8 +602,8 @@ int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, con
     a.adj = adj.p;
     a.longs = longs.p;
     HIPCHK(hipMemcpyAsync(tab.p, hb.data(), sizeof(TdBlock) * nblk, hipMemcpyHostToDevice, ctx->stream));
-    DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * (zw + words), td_clear_k, sgrid(ctx, std::max(zw, words / 2)), ctx->block_size, 0, zero.p, zw,
-               (u64 *)F.p, (u64 *)D[0], words / 2);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * (zw + words), td_clear_k, sgrid(ctx, std::max(zw, words / 4)), ctx->block_size, 0, zero.p, zw,
+               (uint4 *)F.p, (uint4 *)D[0], words / 4);
     a.wgblk = nullptr;
     if (nblk > 1) {
         wgblk.ensure(nwg);
