@@ -475,12 +475,13 @@ struct MapRef {
 u64 bitmap_emit_maps(dlg_ctx *ctx, const u32 *words, const std::vector<MapRef> &maps, bool transposed, u64 *out,
                      u64 expect);
 // The same for row-major maps that each start at a whole emission tile of
-// `words` (emit_tile_words(rows * wpr) words each, the padding clear, nwords
+// `words` (emit_tile_words(rows * wpr, small) words each, the padding clear, nwords
 // in all): read out as they lie.  `out` is resized; the count is checked
 // against `expect` before anything is written (synchronises).
-u64 emit_tile_words(u64 nwords);
+// small: tiles of an eighth of the words, for maps that a tile would mostly pad.
+u64 emit_tile_words(u64 nwords, bool small);
 void bitmap_emit_tiled(dlg_ctx *ctx, u32 *words, const std::vector<MapRef> &maps, u64 nwords, DBuf<u64> &out,
-                       u64 expect);
+                       u64 expect, bool small);
 // A W-row block of a map, emitted in tuple order at out through a padded
 // scratch copy (transposed back when `transposed`).  Returns its set bits.
 u64 bitmap_emit_block(dlg_ctx *ctx, const u32 *words, u32 lo, u64 W, u64 wpr, bool transposed, DBuf<u32> &scratch,

@@ -1547,7 +1547,10 @@ u64 bitmap_emit_maps(dlg_ctx *ctx, const u32 *words, const std::vector<MapRef> &
     return total;
 }
 
-u64 emit_tile_words(u64 nwords) { return (nwords + BE_TILE - 1) / BE_TILE * BE_TILE; }
+u64 emit_tile_words(u64 nwords, bool small) {
+    const u64 t = small ? BE_T : BE_TILE;
+    return (nwords + t - 1) / t * t;
+}
 
 // Maps too small to give every CU a tile of BE_TILE words go by tiles of BE_T
 // words: TC of 437 ids (3 large tiles) 31 us of emission by large tiles.
@@ -1587,10 +1590,10 @@ static void emit_tiled(dlg_ctx *ctx, u32 *words, const std::vector<MapRef> &maps
 }
 
 void bitmap_emit_tiled(dlg_ctx *ctx, u32 *words, const std::vector<MapRef> &maps, u64 nwords, DBuf<u64> &out,
-                       u64 expect) {
+                       u64 expect, bool small) {
     out.ensure(expect ? expect : 1);
     if (nwords == 0) return;
-    if (nwords < (u64)ctx->num_cus * BE_TILE) emit_tiled<1>(ctx, words, maps, nwords, out.p, expect);
+    if (small || nwords < (u64)ctx->num_cus * BE_TILE) emit_tiled<1>(ctx, words, maps, nwords, out.p, expect);
     else emit_tiled<BE_W>(ctx, words, maps, nwords, out.p, expect);
 }
 

@@ -528,7 +528,15 @@ int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, con
     std::vector<TdBlock> hb;
     std::vector<int> owner;   // the range each block is
     std::vector<MapRef> maps;
-    u64 words = 0, tasks = 0;
+    // Tiles of 256 words where those of 2,048 would mostly pad (many instances of a few ids:
+    // 100,000 of 10 took 2.4 GB of maps, and take 0.3): each map is there three times.
+    u64 words = 0, tasks = 0, pad_big = 0, pad_small = 0;
+    for (size_t i = 0; i + 1 < st.size(); i++) {
+        const u64 b0 = std::max<u64>(st[i], lo), b1 = std::min<u64>(st[i + 1], (u64)hi + 1), w = b1 > b0 ? b1 - b0 : 0;
+        pad_big += emit_tile_words(w * ((w + 127) / 128 * 4), false);
+        pad_small += emit_tile_words(w * ((w + 127) / 128 * 4), true);
+    }
+    const bool small = 2 * pad_small <= pad_big;
     for (size_t i = 0; i + 1 < st.size(); i++) {
         const u64 b0 = std::max<u64>(st[i], lo), b1 = std::min<u64>(st[i + 1], (u64)hi + 1);
         if (b1 <= b0) continue;
@@ -540,7 +548,7 @@ int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, con
         k.base = words;
         k.task0 = tasks;
         k.wg0 = k.pad = 0;
-        words += emit_tile_words((u64)k.W * k.wpr);
+        words += emit_tile_words((u64)k.W * k.wpr, small);
         tasks += (u64)k.W * k.nc;
         hb.push_back(k);
         owner.push_back((int)i);
@@ -557,7 +565,7 @@ int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, con
         if (it > 0) {   // 0: too many rows with long lists
             *total = m[0];
             *raw += m[1];
-            bitmap_emit_tiled(ctx, F.p, maps, words, out, *total);
+            bitmap_emit_tiled(ctx, F.p, maps, words, out, *total, small);
             if (iters) iters->assign(1, it);
             return it;
         }
@@ -661,7 +669,7 @@ int tc_dense_run(dlg_ctx *ctx, const int32_t *d_rows, u64 n, u32 lo, u32 hi, con
         for (u32 b = 0; b < nblk; b++) (*iters)[owner[b]] = nblk > 1 && h[b] ? (int)h[b] : it;
     }
     D2.release();   // before the relation itself is allocated
-    bitmap_emit_tiled(ctx, a.F, maps, words, out, *total);
+    bitmap_emit_tiled(ctx, a.F, maps, words, out, *total, small);
     return it;
 }
 

@@ -168,3 +168,31 @@ def test_short_of_memory(ctx, orc, batch, mb):
             same(r, orc.tc(rows))
             if not batch:
                 assert r["raw_join_rows"] == ctx.run("tc", rows, queue=1)["raw_join_rows"]
+
+
+# many small instances: maps in tiles of 256 words where those of 2,048 would mostly pad, in fewer and in more tiles than
+# CUs take (256 x 2,048 words), one map of several tiles among them
+@pytest.mark.parametrize("count,ids", [(1, 10), (5, 64), (300, 30), (3000, 12), (3000, 70), (40, 200)])
+def test_many_small_instances(ctx, orc, count, ids):
+    rng = np.random.default_rng(count + ids)
+    inst = [rng.integers(-ids, ids, size=(ids // 2, 2)).astype(np.int32) // 2 for _ in range(count)]
+    inst.append(graph(150, 170, 9))
+    res, _ = ctx.batch_run("tc", inst, check_output=1)
+    for r, rows in zip(res, inst):
+        want = orc.tc(rows)
+        same(r, want)
+        assert r["output_order_breaks"] == 0
+
+
+def test_tiny_instances_memory(ctx):
+    """20,000 instances of up to 10 ids in 256 MB (the maps in tiles of 2,048 words: three of 160)."""
+    rng = np.random.default_rng(2)
+    inst = [rng.integers(0, 10, size=(8, 2)).astype(np.int32) for _ in range(20_000)]
+    want, _ = ctx.batch_run("tc", inst, keep_output=False, check_output=1)
+    row_kernel, _ = ctx.batch_run("tc", inst, keep_output=False, check_output=1, queue=1)
+    assert want == row_kernel
+    budget(ctx, 256)
+    try:
+        assert ctx.batch_run("tc", inst, keep_output=False, check_output=1)[0] == want
+    finally:
+        budget(ctx, 0)
