@@ -192,11 +192,12 @@ static Layout make_layout(int B, const int32_t *const *rows, const int64_t *n, c
 }
 
 // The instances' rows on the device, one after the other as given, with their
-// bounds found and their ids shifted there.  The host only copies them into a page-locked
-// block, a chunk of which is on its way while the next is copied; reading 3.7M rows twice
+// bounds found and their ids shifted there.  The host only copies them into two page-locked
+// chunks in turn, one of which is on its way while the other is filled; reading 3.7M rows twice
 // more on the host for bounds and shifts, and copying from pageable memory, left the
-// device idle for 9 of a batch's 31 ms.  Fewer rows than BU_MIN don't pay for the two
-// launches and the wait; more than BU_MAX would lock 1 GiB.
+// device idle for 9 of a batch's 31 ms.  (With the whole union page-locked the first batch of a
+// size paid for locking it: 16M rows 80 ms, 61 from pageable memory, 39 so.)  Fewer rows than BU_MIN
+// don't pay for the two launches and the wait.
 constexpr int64_t BU_MIN = 1 << 16, BU_MAX = 1ll << 27;
 constexpr int64_t BU_CHUNK = 1 << 18;   // rows
 constexpr u64 BU_SEG = 4096;            // rows a workgroup
@@ -245,12 +246,33 @@ __global__ __launch_bounds__(256) void inst_shift_k(int2 *rows, u64 n, const u64
     });
 }
 
-struct StagingBlock {   // given back once nothing copies from it
+// Two chunks of `rows` rows, copied from in turn; given back once nothing copies from them.
+struct Staging {
     dlg_ctx *ctx;
-    void *p;
-    ~StagingBlock() {
+    int64_t rows;
+    int32_t *p;
+    hipEvent_t left[2] = {nullptr, nullptr};   // the chunk's last copy is over
+    bool used[2] = {false, false};
+    int cur = 0;
+    int64_t have = 0;                          // rows in the chunk at hand
+    Staging(dlg_ctx *c, int64_t n) : ctx(c), rows(n), p((int32_t *)host_block_alloc(16 * (size_t)n)) {}
+    Staging(const Staging &) = delete;
+    ~Staging() {
         (void)hipStreamSynchronize(ctx->stream);
+        for (hipEvent_t e : left)
+            if (e) (void)hipEventDestroy(e);
         host_block_free(p);
+    }
+    int32_t *at() { return p + 2 * (cur * rows + have); }
+    void send(int32_t *d) {   // the chunk's rows, to d
+        if (!have) return;
+        HIPCHK(hipMemcpyAsync(d, p + 2 * cur * rows, 8 * (size_t)have, hipMemcpyHostToDevice, ctx->stream));
+        if (!left[cur]) HIPCHK(hipEventCreateWithFlags(&left[cur], hipEventDisableTiming));
+        HIPCHK(hipEventRecord(left[cur], ctx->stream));
+        used[cur] = true;
+        cur ^= 1;
+        have = 0;
+        if (used[cur]) HIPCHK(hipEventSynchronize(left[cur]));
     }
 };
 
@@ -265,7 +287,7 @@ static bool upload_union(dlg_ctx *ctx, int B, const int32_t *const *rows, const 
     }
     const u64 N = ho[B];
     if (N < (u64)BU_MIN) return false;
-    StagingBlock stage{ctx, host_block_alloc(8 * N)};
+    Staging stage(ctx, std::min<int64_t>(BU_CHUNK, ((int64_t)N + 1) / 2));
     if (!stage.p) return false;
     d.ensure(2 * N);
     off.ensure(B + 1);
@@ -277,20 +299,19 @@ static bool upload_union(dlg_ctx *ctx, int B, const int32_t *const *rows, const 
     }
     HIPCHK(hipMemcpyAsync(off.p, ho.data(), 8 * (size_t)(B + 1), hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(hipMemcpyAsync(m.p, mm.data(), 8 * (size_t)B, hipMemcpyHostToDevice, ctx->stream));
-    char *h = (char *)stage.p;
-    u64 have = 0, sent = 0;   // rows
+    u64 sent = 0;   // rows
     auto send = [&]() {
-        if (have > sent)
-            HIPCHK(hipMemcpyAsync(d.p + 2 * sent, h + 8 * sent, 8 * (have - sent), hipMemcpyHostToDevice, ctx->stream));
-        sent = have;
+        const int64_t k = stage.have;
+        stage.send(d.p + 2 * sent);
+        sent += (u64)k;
     };
     for (int i = 0; i < B; i++)
         for (int64_t r = 0; r < n[i];) {
-            const int64_t take = std::min(n[i] - r, BU_CHUNK - (int64_t)(have - sent));
-            std::memcpy(h + 8 * have, rows[i] + 2 * r, 8 * (size_t)take);
-            have += (u64)take;
+            const int64_t take = std::min(n[i] - r, stage.rows - stage.have);
+            std::memcpy(stage.at(), rows[i] + 2 * r, 8 * (size_t)take);
+            stage.have += take;
             r += take;
-            if (have - sent == (u64)BU_CHUNK) send();
+            if (stage.have == stage.rows) send();
         }
     send();
     DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * N, inst_bounds_k, grid_for(N, BU_SEG), 256, 0, (const int2 *)d.p, N, (const u64 *)off.p,

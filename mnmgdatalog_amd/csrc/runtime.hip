@@ -375,6 +375,11 @@ void dlg_host_free(void *p) { host_block_free(p); }
 // For tests: of the host blocks that the library allocates from now on, the one after the
 // next n fails, once.  (Not in the header.)
 void dlg_test_fail_host_block(int64_t n) { blocks_until_failure.store(n); }
+// For tests: the page-locked bytes that the library holds, handed out and kept.  (Not in the header.)
+uint64_t dlg_test_pinned_bytes(void) {
+    std::lock_guard<std::mutex> lk(pinned_mu);
+    return pinned_total;
+}
 // For tests: the device memory that the context may hold from now on (0: any), its kept
 // blocks given back first.  (Not in the header.)
 void dlg_test_budget(dlg_ctx *c, uint64_t bytes) {

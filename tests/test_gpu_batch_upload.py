@@ -1,5 +1,7 @@
 """Batches whose rows are bounded and shifted on the device: totals around the first that is (65,536 rows), empty
 instances, instances over several chunks of the upload (262,144 rows) and segments (4,096), ids at both ends of their range."""
+from ctypes import c_uint64
+
 import numpy as np
 import pytest
 
@@ -45,3 +47,17 @@ def test_chunks_and_ends(ctx, prog):
     inst = [empty, rows(262_143, 60_000, -2**31, 1), empty, rows(1, 1, 2**31 - 1, 2), rows(262_145, 70_000, 2**31 - 70_000, 3),
             rows(4097, 900, 0, 4), rows(40_000, 5000, -7, 5), empty]
     check(ctx, prog, inst)
+
+
+@pytest.mark.parametrize("total", [100_000, 524_287, 524_289, 4_000_000])
+def test_page_locked(ctx, total):
+    """The rows go up by two chunks of 2 MB at most, however many they are."""
+    pinned = ctx.L.dlg_test_pinned_bytes
+    pinned.restype = c_uint64
+    inst = [rows(total // 4, 30_000, 0, k) for k in range(4)]
+    before = pinned()
+    res, _ = ctx.batch_run("wcc", inst, keep_output=False)
+    assert pinned() - before <= 4 << 20
+    want = [ctx.run("wcc", i, keep_output=False) for i in inst]
+    assert [(r["iterations"], r["output_size"], r["secondary"]) for r in res] == [
+        (w["iterations"], w["output_size"], w["secondary"]) for w in want]
