@@ -302,7 +302,8 @@ void dlg_result_free(dlg_result *res);
  * instance's own digest (its rows in its own ids), equal to its plain run's. */
 typedef enum dlg_prog { DLG_PROG_TC = 0, DLG_PROG_SG = 1, DLG_PROG_WCC = 2, DLG_PROG_SJ = 3 } dlg_prog;
 typedef struct dlg_batch_stats {
-    double device_seconds;   /* upload-to-resident wall time of the whole batch      */
+    double device_seconds;   /* wall time from the first row's upload to the resident
+                                results of the whole batch                            */
     int32_t rounds;          /* fixpoint rounds run (max over instances)             */
     int64_t total_output;    /* sum of output_size                                    */
     int64_t union_rows;      /* input rows of the union                               */

@@ -276,9 +276,10 @@ struct Staging {
     }
 };
 
-// False: too few, too many or bad rows (the caller's own reading reports those).
+// False: too few, too many or bad rows (the caller's own reading reports those).  t0: when the
+// first chunk is sent.
 static bool upload_union(dlg_ctx *ctx, int B, const int32_t *const *rows, const int64_t *n, DBuf<int32_t> &d, DBuf<u64> &off,
-                         std::vector<u32> &mm) {
+                         std::vector<u32> &mm, Clock::time_point &t0) {
     std::vector<u64> ho(B + 1, 0);
     for (int i = 0; i < B; i++) {
         if (n[i] < 0 || n[i] > BU_MAX || (n[i] > 0 && !rows[i])) return false;
@@ -302,6 +303,7 @@ static bool upload_union(dlg_ctx *ctx, int B, const int32_t *const *rows, const 
     u64 sent = 0;   // rows
     auto send = [&]() {
         const int64_t k = stage.have;
+        if (!sent) t0 = Clock::now();
         stage.send(d.p + 2 * sent);
         sent += (u64)k;
     };
@@ -654,11 +656,11 @@ static void wcc_batch_rounds(dlg_ctx *ctx, WccState &s, const WccGraph &g, const
 
 void batch_run(dlg_ctx *ctx, int prog, int B, const int32_t *const *rows, const int64_t *n,
                       const Opts &o, dlg_result *res, dlg_batch_stats *st) {
-    auto t0 = Clock::now();
+    Clock::time_point t0;
     DBuf<int32_t> d_rows(ctx);
     DBuf<u64> roff(ctx);
     std::vector<u32> mm, shift;
-    const bool up = upload_union(ctx, B, rows, n, d_rows, roff, mm);
+    const bool up = upload_union(ctx, B, rows, n, d_rows, roff, mm, t0);
     Layout L = make_layout(B, rows, n, up ? mm.data() : nullptr);
     if (L.exhausted < B) {
         d_rows.release();
