@@ -598,12 +598,13 @@ static void split_rows(dlg_ctx *ctx, const u64 *d, const std::vector<u64> &b, co
 
 // The rounds of a batch's WCC union, pushed from the frontier: per round the
 // frontier is counted by instance, and an instance whose rule fires drops out
-// of it.  (Graphs too large for whole-graph pulls, and the other round forms.)
+// of it.  (Graphs too large for whole-graph pulls, what those leave, and the other round forms.)
 static void wcc_batch_rounds(dlg_ctx *ctx, WccState &s, const WccGraph &g, const Opts &o, PhaseClock &pc,
-                             const u32 *vstart, const std::vector<u32> &hv, std::vector<int> &iters, int &rounds) {
+                             const u32 *vstart, const std::vector<u32> &hv, const WccRest &rest, std::vector<int> &iters,
+                             int &rounds) {
     const u64 V = g.V;
     const int B = (int)hv.size() - 1;
-    wcc_setup(ctx, s, V);
+    if (!rest.left) wcc_setup(ctx, s, V);
     DBuf<u32> cnt(ctx, B), live(ctx, B);
     std::vector<i64> prev(B), cur(B);
     std::vector<char> done(B, 0);
@@ -611,6 +612,16 @@ static void wcc_batch_rounds(dlg_ctx *ctx, WccState &s, const WccGraph &g, const
     for (int i = 0; i < B; i++) prev[i] = (i64)(hv[i + 1] - hv[i]);   // wcc.cu:236-242
     int live_n = B;
     u64 nf = V;
+    if (rest.left) {
+        nf = rest.nf;
+        for (int i = 0; i < B; i++) {
+            prev[i] = (i64)rest.prev[i];
+            if (!rest.done[i]) continue;
+            done[i] = 1;
+            hlive[i] = 0;
+            live_n--;
+        }
+    }
     DBuf<u32> tnode(ctx, V ? V : 1), tlabel(ctx, V ? V : 1);
     std::vector<u32> hc(B);
     while (live_n > 0) {
@@ -745,14 +756,14 @@ void batch_run(dlg_ctx *ctx, int prog, int B, const int32_t *const *rows, const 
         WccState s(ctx);
         std::vector<int> iters(B, 0);
         const bool whole = o.strategy == 0 && o.relax == WCC_AUTO && g.ne <= WD_MAX_EDGES;
+        WccRest rest;
         if (whole) {
             pc.mark(DLG_PH_JOIN);
             std::vector<u32> hit;
-            rounds = wcc_rounds_whole(ctx, s, V, g.ix, g.nbr.p, o.max_it, vstart.p, (u32)B, &hit);
+            rounds = wcc_rounds_whole(ctx, s, V, g.ix, g.nbr.p, o.max_it, vstart.p, (u32)B, &hit, &rest);
             for (int i = 0; i < B; i++) iters[i] = (int)hit[i];
-        } else {
-            wcc_batch_rounds(ctx, s, g, o, pc, vstart.p, hv, iters, rounds);
         }
+        if (!whole || rest.left) wcc_batch_rounds(ctx, s, g, o, pc, vstart.p, hv, rest, iters, rounds);
         // components per instance
         pc.mark(DLG_PH_FINAL);
         DBuf<u32> ccount(ctx, V ? V : 1), flags(ctx, V ? V : 1);

@@ -742,8 +742,16 @@ u64 wcc_finalize(dlg_ctx *ctx, WccState &s, const Index &ix, DBuf<u64> &out, i64
 constexpr u64 WD_MAX_EDGES = 1ull << 25;
 // With vstart (device, B + 1 entries: instance i holds the nodes [vstart[i],
 // vstart[i + 1])), each instance stops by its own rule, its round count in iters.
+// Where few nodes are left to lower, one graph goes on by captured push rounds; a batch's
+// rounds are left to the caller (`rest`: nf nodes in s.fnode and s.flabel, the instances'
+// last counts and which have stopped).
+struct WccRest {
+    bool left = false;
+    u64 nf = 0;
+    std::vector<u32> prev, done;
+};
 int wcc_rounds_whole(dlg_ctx *ctx, WccState &s, u64 V, const Index &ix, const u32 *nbr, int max_it,
-                     const u32 *vstart = nullptr, u32 B = 0, std::vector<u32> *iters = nullptr);
+                     const u32 *vstart = nullptr, u32 B = 0, std::vector<u32> *iters = nullptr, WccRest *rest = nullptr);
 // All rounds through replays of a captured graph of `kr` rounds; returns the
 // iteration count (labels in s.L).  `ne` = edges of the index.
 int wcc_rounds_graph(dlg_ctx *ctx, WccState &s, const Index &ix, const u32 *nbr, u64 ne, int max_it,

@@ -32,7 +32,9 @@
 #include "dlg_internal.h"
 
 #include <algorithm>
+#include <chrono>
 #include <deque>
+#include <memory>
 
 namespace dlg {
 
@@ -513,6 +515,15 @@ void wcc_setup(dlg_ctx *ctx, WccState &s, u64 V) {
                    s.flabel.p, s.mark.p, V);
 }
 
+// Frontier lists and marks, the labels left as they are.
+static void wcc_lists(dlg_ctx *ctx, WccState &s, u64 V) {
+    s.mark.ensure(V);
+    s.fnode.ensure(V);
+    s.flabel.ensure(V);
+    s.nnode.ensure(V);
+    fill_u32(ctx, s.mark.p, V, 0u);
+}
+
 // Components: returns #distinct labels, *largest, and the (label, 0) tuples in `out`.
 u64 wcc_finalize(dlg_ctx *ctx, WccState &s, const Index &ix, DBuf<u64> &out, i64 *largest) {
     u64 V = s.V;
@@ -554,8 +565,8 @@ u64 wcc_finalize(dlg_ctx *ctx, WccState &s, const Index &ix, DBuf<u64> &out, i64
 // 160,000 nodes, 355,000 edges, ~500 rounds 15.4 -> 2.0 ms (a round 4.6 us
 // instead of 41); 12.4M nodes, 28.8M edges, 4,303 rounds 2,693 -> 344 ms;
 // R-MAT 2^17 to 2^20 nodes 1.36 -> 0.82 and 4.3 -> 4.1 ms; a star of 200,000
-// 1.0 -> 0.56 ms (1.1 with its hub in one workgroup).  Never slower up to
-// WD_MAX_EDGES, the range the captured rounds were taken for.
+// 1.0 -> 0.56 ms (1.1 with its hub in one workgroup).  Where they cost more than the captured
+// rounds (many rounds of few nodes), those take over: see wcc_rounds_whole.
 // Batches: 400 instances 2.8 -> 1.6 ms on the device.
 namespace dlg {
 
@@ -648,28 +659,35 @@ __device__ __forceinline__ void wd_count(WdState *st, const WdInst &in, u32 roun
 }
 
 // Publishes round `round` - 1: the stop rule (wcc.cu:366-383) on its count, or
-// on each instance's; host[1] = nothing is left to run.
+// on each instance's; host[0] = the nodes it lowered (of the instances left),
+// host[1] = nothing is left to run.
 template <bool MULTI>
 __device__ __forceinline__ void wd_publish(WdState *st, const WdInst &in, u32 round, u64 *host, u64 seq) {
-    __shared__ u32 s_live;
+    __shared__ u32 s_live, s_low;
     if (MULTI) {
-        if (threadIdx.x == 0) s_live = 0;
+        if (threadIdx.x == 0) s_live = s_low = 0;
         __syncthreads();
         const u32 *cur = in.cnt + (u64)((round - 1) % WD_SETS) * in.B;
         u32 *next = in.cnt + (u64)((round + 1) % WD_SETS) * in.B;
-        u32 live = 0;
+        u32 live = 0, low = 0;
         for (u32 i = threadIdx.x; i < in.B; i += WD_T) {
             next[i] = 0;
             if (in.done[i]) continue;
             in.iters[i] = round - 1;
-            if (cur[i] == in.prev[i]) in.done[i] = 1;
-            else live++;
+            if (cur[i] == in.prev[i]) {
+                in.done[i] = 1;
+            } else {
+                live++;
+                low += cur[i];
+            }
             in.prev[i] = cur[i];
         }
         if (live) atomicAdd(&s_live, live);
+        if (low) atomicAdd(&s_low, low);
         __syncthreads();
         if (threadIdx.x == 0) {
             if (s_live == 0 && !st->done) st->done = round;
+            host[0] = s_low;
             host[1] = st->done != 0;
         }
     } else if (threadIdx.x < WAVE) {   // WD_SLOTS == WAVE: a slice per lane
@@ -679,6 +697,7 @@ __device__ __forceinline__ void wd_publish(WdState *st, const WdInst &in, u32 ro
         for (int d = WAVE / 2; d > 0; d >>= 1) c += __shfl_xor(c, d, WAVE);
         if (threadIdx.x == 0) {
             if (c == st->prev && !st->done) st->done = round;
+            host[0] = c;
             host[1] = st->done != 0;
             st->prev = c;
         }
@@ -795,6 +814,45 @@ __global__ void wd_inst_k(const u32 *vstart, WdInst in, u64 V, u32 *of) {
         in.done[i] = in.iters[i] = 0;
     }
 }
+// Rounds from labels L whose last round lowered `prev` nodes: both arrays hold them.
+__global__ void wd_again_k(WdState *st, const u32 *L, u32 *Ln, u64 V, u64 prev) {
+    const u64 i0 = (u64)blockIdx.x * blockDim.x + threadIdx.x, stride = (u64)gridDim.x * blockDim.x;
+    for (u64 i = i0; i < V; i += stride) Ln[i] = L[i];
+    for (u64 i = i0; i < (u64)WD_SETS * WD_SLOTS * WD_LINE; i += stride) (&st->cnt[0][0][0])[i] = 0;
+    if (i0 == 0) {
+        st->prev = prev;
+        st->done = 0;
+    }
+}
+// The instances' labels after `rounds` rounds to L (those of its last round where the rule has fired),
+// and the nodes that the last round lowered in the others.
+__global__ __launch_bounds__(WA_T) void wd_export_k(u32 *L, const u32 *Ln, u64 V, WdInst in, u32 rounds, u32 *node, u32 *label,
+                                                    u32 *count) {
+    __shared__ u32 s_cnt[WA_I * WA_T / WAVE + 1];
+    const u64 base = (u64)blockIdx.x * WA_TILE;
+    bool app[WA_I];
+    u32 l[WA_I], slot[WA_I];
+#pragma unroll
+    for (int r = 0; r < WA_I; r++) {
+        const u64 i = base + (u64)r * WA_T + threadIdx.x;
+        app[r] = false;
+        l[r] = 0;
+        if (i < V) {
+            const u32 inst = in.of[i], a = L[i], b = Ln[i];
+            const bool fin = in.done[inst] != 0, odd = ((fin ? in.iters[inst] : rounds) & 1u) != 0;
+            l[r] = odd ? b : a;
+            app[r] = !fin && l[r] < (odd ? a : b);
+            L[i] = l[r];
+        }
+    }
+    block_append<WA_T, WA_I>(app, count, s_cnt, slot);
+#pragma unroll
+    for (int r = 0; r < WA_I; r++)
+        if (app[r]) {
+            node[slot[r]] = (u32)(base + (u64)r * WA_T + threadIdx.x);
+            label[slot[r]] = l[r];
+        }
+}
 // The labels of each node's instance's last round.
 __global__ void wd_pick_k(u32 *L, const u32 *Ln, u64 V, WdInst in) {
     const u64 stride = (u64)gridDim.x * blockDim.x;
@@ -895,84 +953,6 @@ __global__ __launch_bounds__(WO_T) void wo_rounds_k(const u32 *gstart, const u32
         *(volatile u64 *)(host + dlg_ctx::MAPPED_SEQ) = seq;
         __threadfence_system();
     }
-}
-
-int wcc_rounds_whole(dlg_ctx *ctx, WccState &s, u64 V, const Index &ix, const u32 *nbr, int max_it, const u32 *vstart,
-                     u32 B, std::vector<u32> *iters) {
-    s.V = V;
-    if (iters) iters->assign(B, 1);
-    if (V == 0) return 1;   // empty graph: the first round already sees 0 == 0
-    s.L.ensure(V);
-    s.counter.ensure(4);
-    if (!vstart && wo_takes(V, ix.n)) {
-        const u64 seq = ++ctx->mapped_seq;
-        DLG_LAUNCH(ctx, DLG_K_WCC_RELAX, 8.0 * ix.n + 16.0 * V, wo_rounds_k, 1, WO_T, 0, (const u32 *)ix.gstart.p, nbr, (u32)V,
-                   (u32)ix.n, max_it, s.L.p, ctx->mapped_dev(seq), seq);
-        ctx->wait_mapped(seq);
-        return (int)ctx->mapped_host(seq)[0];
-    }
-    static_assert(WD_SLOTS == WAVE, "the publisher's wave sums a slice per lane");
-    DBuf<u64> stbuf(ctx, (sizeof(WdState) + 7) / 8);
-    WdState *st = (WdState *)stbuf.p;
-    s.Ln.ensure(V);
-    u32 *buf[2] = {s.L.p, s.Ln.p};   // round r leaves its labels in buf[r & 1]
-    DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * V, wd_init_k, sgrid(ctx, V), ctx->block_size, 0, st, buf[0], buf[1], V);
-    DBuf<u32> mid(ctx, ix.n / WD_THREAD + 1);
-    DBuf<uint2> hub(ctx, ix.n / WD_WAVE + ix.n / WD_SEG + 1);
-    DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * V, wd_lists_k, (unsigned)std::min<u64>((V + WD_T - 1) / WD_T, (u64)ctx->num_cus * 8),
-               WD_T, 0, (const u32 *)ix.gstart.p, V, mid.p, hub.p, st);
-    WdInst in{nullptr, B, nullptr, nullptr, nullptr, nullptr};
-    DBuf<u32> of(ctx), ist(ctx);
-    if (vstart) {
-        of.ensure(V);
-        ist.ensure((u64)(WD_SETS + 3) * B);
-        in.of = of.p;
-        in.cnt = ist.p;
-        in.prev = ist.p + (u64)WD_SETS * B;
-        in.done = in.prev + B;
-        in.iters = in.done + B;
-        DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * V, wd_inst_k, sgrid(ctx, V), ctx->block_size, 0, vstart, in, V, of.p);
-    }
-    u64 seq = ++ctx->mapped_seq;
-    DLG_LAUNCH(ctx, DLG_K_MISC, 0.0, wd_sizes_k, 1, 64, 0, (const WdState *)st, ctx->mapped_dev(seq), seq);
-    ctx->wait_mapped(seq);
-    const u32 nmid = (u32)ctx->mapped_host(seq)[0], nhub = (u32)ctx->mapped_host(seq)[1];
-    const unsigned g = 1u + (unsigned)((V + WD_T - 1) / WD_T) + (nmid + WD_T / WAVE - 1) / (WD_T / WAVE) + nhub;
-    std::deque<u64> q;   // sequence numbers of the rounds not read yet
-    int launched = 0, it = 0;
-    auto launch = [&](bool publish_only) {
-        const u32 r = (u32)launched + 1;
-        seq = r > 1 ? ++ctx->mapped_seq : 0;   // round 1 has no round before it
-        auto go = [&](auto kern) {
-            // 4 B neighbour + 4 B label per edge; a start and two labels per node
-            DLG_LAUNCH(ctx, DLG_K_WCC_RELAX, publish_only ? 0.0 : 8.0 * ix.n + 16.0 * V, kern, publish_only ? 1u : g, WD_T,
-                       0, (const u32 *)ix.gstart.p, nbr, V, (const u32 *)buf[(r - 1) & 1], buf[r & 1],
-                       (const u32 *)mid.p, nmid, (const uint2 *)hub.p, st, in, r, publish_only ? 1 : 0,
-                       ctx->mapped_dev(seq), seq);
-        };
-        if (vstart) go(wd_round_k<true>);
-        else go(wd_round_k<false>);
-        if (r > 1) q.push_back(seq);
-        if (!publish_only) launched++;
-    };
-    while (true) {
-        while (launched < it + 1 + WD_DEPTH && (max_it <= 0 || launched < max_it)) launch(false);
-        if (q.empty()) launch(true);   // the last round asked for
-        ctx->wait_mapped(q.front());
-        const bool done = ctx->mapped_host(q.front())[1] != 0;
-        q.pop_front();
-        it++;
-        if (done || (max_it > 0 && it >= max_it)) break;
-    }
-    if (vstart) {
-        DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * V, wd_pick_k, sgrid(ctx, V), ctx->block_size, 0, s.L.p, (const u32 *)s.Ln.p, V,
-                   in);
-        HIPCHK(hipMemcpyAsync(iters->data(), in.iters, 4 * (size_t)B, hipMemcpyDeviceToHost, ctx->stream));
-        ctx->sync();
-    } else if (it & 1) {
-        s.L.swap(s.Ln);
-    }
-    return it;
 }
 
 }  // namespace dlg
@@ -1132,66 +1112,246 @@ static void gw_capture_round(dlg_ctx *ctx, WccState &s, const Index &ix, const u
     hipLaunchKernelGGL(gw_end_k, dim3(1), dim3(64), 0, ctx->stream, st);
 }
 
+__global__ void gw_start_k(WccDev *st, WccDev h) {
+    if (threadIdx.x == 0 && blockIdx.x == 0) *st = h;
+}
+
+typedef std::chrono::steady_clock WallClock;
+static double wall_us(WallClock::time_point t0) { return std::chrono::duration<double, std::micro>(WallClock::now() - t0).count(); }
+
+// A captured graph of `kr` rounds (even) on the labels in L, replayed until `go` says no.
+struct GwRounds {
+    dlg_ctx *ctx;
+    u32 *L;
+    DBuf<u32> nlabel;
+    DBuf<u64> bsum, stbuf;
+    WccDev *st;
+    hipGraph_t graph = nullptr;
+    hipGraphExec_t exec = nullptr;
+
+    // s: fnode, flabel, nnode and mark are there (wcc_setup, wcc_lists)
+    GwRounds(dlg_ctx *c, WccState &s, const Index &ix, const u32 *nbr, u64 ne, int kr)
+        : ctx(c), L(s.L.p), nlabel(c, s.V), bsum(c, (s.V + GW_TILE - 1) / GW_TILE + 1), stbuf(c, (sizeof(WccDev) + 7) / 8) {
+        const u64 V = s.V;
+        s.cnt.ensure(V);
+        s.pstart.ensure(V);
+        s.offs.ensure(V + 1);
+        st = (WccDev *)stbuf.p;
+        if (kr < 2) kr = 2;
+        kr &= ~1;
+        const bool prof = ctx->prof;
+        ctx->prof = false;
+        HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+        for (int r = 0; r < kr; r++) {
+            if (r % 2 == 0)
+                gw_capture_round(ctx, s, ix, nbr, V, ne, st, s.fnode.p, s.flabel.p, s.nnode.p, bsum.p);
+            else
+                gw_capture_round(ctx, s, ix, nbr, V, ne, st, s.nnode.p, nlabel.p, s.fnode.p, bsum.p);
+        }
+        const hipError_t ce = hipStreamEndCapture(ctx->stream, &graph);
+        ctx->prof = prof;
+        HIPCHK(ce);
+        const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        if (ie != hipSuccess) {
+            (void)hipGraphDestroy(graph);
+            HIPCHK(ie);
+        }
+    }
+    GwRounds(const GwRounds &) = delete;
+    ~GwRounds() {
+        (void)hipGraphExecDestroy(exec);
+        (void)hipGraphDestroy(graph);
+    }
+    // From the nf nodes in fnode, lowered by round `it`, which follow a round that lowered `prev`.
+    // go: whether to replay again, given what a round of the last replay took (us).
+    template <typename F>
+    WccDev run(u64 nf, u64 prev, int it, int max_it, F go) {
+        WccDev h;
+        std::memset(&h, 0, sizeof(h));
+        h.nf = nf;
+        h.prev = prev;
+        h.it = (u32)it;
+        h.max_it = (u32)(max_it > 0 ? max_it : 0);
+        DLG_LAUNCH(ctx, DLG_K_MISC, 0.0, gw_start_k, 1, 64, 0, st, h);
+        while (true) {
+            const auto t0 = WallClock::now();
+            const u32 before = h.it;
+            if (ctx->prof) ctx->prof_begin();
+            HIPCHK(hipGraphLaunch(exec, ctx->stream));
+            if (ctx->prof) ctx->prof_end(DLG_K_WCC_RELAX, 0.0);
+            static_assert(sizeof(WccDev) <= 8 * dlg_ctx::MAPPED_SEQ, "the state fits a mapped slot");
+            ctx->read_words((const u32 *)st, (int)(sizeof(WccDev) / 4), &h);
+            if (h.done || !go(wall_us(t0) / (double)(h.it - before))) return h;
+        }
+    }
+};
+
 // Runs the rounds of wcc_solve with captured graphs of `kr` rounds (even).
 // Returns the iteration count; the labels are left in s.L.
 int wcc_rounds_graph(dlg_ctx *ctx, WccState &s, const Index &ix, const u32 *nbr, u64 ne, int max_it,
                      int kr) {
     const u64 V = s.V;
     if (V == 0) return 1;   // empty graph: the first round already sees 0 == 0
-    if (kr < 2) kr = 2;
-    kr &= ~1;
-    s.cnt.ensure(V);
-    s.pstart.ensure(V);
-    s.offs.ensure(V + 1);
-    DBuf<u32> nlabel(ctx, V);
-    DBuf<u64> bsum(ctx, (V + GW_TILE - 1) / GW_TILE + 1);
-    DBuf<u64> stbuf(ctx, (sizeof(WccDev) + 7) / 8);
-    WccDev *st = (WccDev *)stbuf.p;
-    WccDev h;
-    std::memset(&h, 0, sizeof(h));
-    h.nf = V;
-    h.prev = V;
-    h.max_it = (u32)(max_it > 0 ? max_it : 0);
-    HIPCHK(hipMemcpyAsync(st, &h, sizeof(h), hipMemcpyHostToDevice, ctx->stream));
-    ctx->sync();
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    bool prof = ctx->prof;
-    ctx->prof = false;
-    HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-    for (int r = 0; r < kr; r++) {
-        if (r % 2 == 0)
-            gw_capture_round(ctx, s, ix, nbr, V, ne, st, s.fnode.p, s.flabel.p, s.nnode.p, bsum.p);
-        else
-            gw_capture_round(ctx, s, ix, nbr, V, ne, st, s.nnode.p, nlabel.p, s.fnode.p, bsum.p);
+    GwRounds g(ctx, s, ix, nbr, ne, kr);
+    return (int)g.run(V, V, 0, max_it, [](double) { return true; }).it;
+}
+
+// ------------------------------------------------------ whole-graph rounds, run
+// A pull of the whole graph costs what the graph costs, however few nodes a round lowers:
+// a core with a long tail (R-MAT of 2^20 nodes and a path of 3,000 behind it) took 146, 292
+// and 448 ms with 8, 17 and 31 million edges, by captured push rounds 82, 85 and 85.  So the
+// pulls are left for those once they have cost WD_LEAVE_US more than those would have (81, 80
+// and 83 ms), and taken up again where the pushes turn out to take longer.
+// A pull's time is taken from the rounds themselves, and from the edges where they say more
+// (something else may hold them up): at random 18, 46, 97 and 149 us at 2.1, 6.3, 16.8 and 31
+// million, in grids half of that.  A push round's comes from the nodes lowered: 15 us up to a hundred,
+// 27 at 1,500, 36 at 13,000, 40 at 130,000, 95 at 1,000,000 of one edge on and one back.
+constexpr double WD_LEAVE_US = 250.0;   // a few pulls; the switch and the pulls queued cost as much again
+static double wd_pull_us(u64 ne) { return 5.0 + (double)ne / 190e3; }
+static double gw_push_us(u64 nodes) { return 15.0 + std::min((double)nodes / 256.0, 25.0) + (double)nodes / 16384.0; }
+// A round that wcc_batch_rounds launches by itself: 77 us at least.
+static double wd_batch_push_us(u64 nodes, u32 B) { return 80.0 + 0.003 * (double)B + (double)nodes / 8192.0; }
+
+int wcc_rounds_whole(dlg_ctx *ctx, WccState &s, u64 V, const Index &ix, const u32 *nbr, int max_it, const u32 *vstart,
+                     u32 B, std::vector<u32> *iters, WccRest *rest) {
+    s.V = V;
+    if (iters) iters->assign(B, 1);
+    if (V == 0) return 1;   // empty graph: the first round already sees 0 == 0
+    s.L.ensure(V);
+    s.counter.ensure(4);
+    if (!vstart && wo_takes(V, ix.n)) {
+        const u64 seq = ++ctx->mapped_seq;
+        DLG_LAUNCH(ctx, DLG_K_WCC_RELAX, 8.0 * ix.n + 16.0 * V, wo_rounds_k, 1, WO_T, 0, (const u32 *)ix.gstart.p, nbr, (u32)V,
+                   (u32)ix.n, max_it, s.L.p, ctx->mapped_dev(seq), seq);
+        ctx->wait_mapped(seq);
+        return (int)ctx->mapped_host(seq)[0];
     }
-    hipError_t ce = hipStreamEndCapture(ctx->stream, &graph);
-    ctx->prof = prof;
-    HIPCHK(ce);
-    hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-    if (ie != hipSuccess) {
-        (void)hipGraphDestroy(graph);
-        HIPCHK(ie);
+    static_assert(WD_SLOTS == WAVE, "the publisher's wave sums a slice per lane");
+    DBuf<u64> stbuf(ctx, (sizeof(WdState) + 7) / 8);
+    WdState *st = (WdState *)stbuf.p;
+    s.Ln.ensure(V);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * V, wd_init_k, sgrid(ctx, V), ctx->block_size, 0, st, s.L.p, s.Ln.p, V);
+    DBuf<u32> mid(ctx, ix.n / WD_THREAD + 1);
+    DBuf<uint2> hub(ctx, ix.n / WD_WAVE + ix.n / WD_SEG + 1);
+    DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * V, wd_lists_k, (unsigned)std::min<u64>((V + WD_T - 1) / WD_T, (u64)ctx->num_cus * 8),
+               WD_T, 0, (const u32 *)ix.gstart.p, V, mid.p, hub.p, st);
+    WdInst in{nullptr, B, nullptr, nullptr, nullptr, nullptr};
+    DBuf<u32> of(ctx), ist(ctx);
+    if (vstart) {
+        of.ensure(V);
+        ist.ensure((u64)(WD_SETS + 3) * B);
+        in.of = of.p;
+        in.cnt = ist.p;
+        in.prev = ist.p + (u64)WD_SETS * B;
+        in.done = in.prev + B;
+        in.iters = in.done + B;
+        DLG_LAUNCH(ctx, DLG_K_MISC, 4.0 * V, wd_inst_k, sgrid(ctx, V), ctx->block_size, 0, vstart, in, V, of.p);
     }
-    int it = 0;
-    try {
+    u64 seq = ++ctx->mapped_seq;
+    DLG_LAUNCH(ctx, DLG_K_MISC, 0.0, wd_sizes_k, 1, 64, 0, (const WdState *)st, ctx->mapped_dev(seq), seq);
+    ctx->wait_mapped(seq);
+    const u32 nmid = (u32)ctx->mapped_host(seq)[0], nhub = (u32)ctx->mapped_host(seq)[1];
+    const unsigned g = 1u + (unsigned)((V + WD_T - 1) / WD_T) + (nmid + WD_T / WAVE - 1) / (WD_T / WAVE) + nhub;
+    std::deque<u64> q;   // sequence numbers of the rounds not read yet
+    u32 *buf[2];         // a stretch's round r leaves its labels in buf[r & 1]
+    int launched = 0;    // rounds of the stretch
+    auto launch = [&](bool publish_only) {
+        const u32 r = (u32)launched + 1;
+        seq = r > 1 ? ++ctx->mapped_seq : 0;   // round 1 has no round before it
+        auto go = [&](auto kern) {
+            // 4 B neighbour + 4 B label per edge; a start and two labels per node
+            DLG_LAUNCH(ctx, DLG_K_WCC_RELAX, publish_only ? 0.0 : 8.0 * ix.n + 16.0 * V, kern, publish_only ? 1u : g, WD_T,
+                       0, (const u32 *)ix.gstart.p, nbr, V, (const u32 *)buf[(r - 1) & 1], buf[r & 1],
+                       (const u32 *)mid.p, nmid, (const uint2 *)hub.p, st, in, r, publish_only ? 1 : 0,
+                       ctx->mapped_dev(seq), seq);
+        };
+        if (vstart) go(wd_round_k<true>);
+        else go(wd_round_k<false>);
+        if (r > 1) q.push_back(seq);
+        if (!publish_only) launched++;
+    };
+    const double pull_most = 1.5 * wd_pull_us(ix.n);
+    double pull_us = pull_most, leave_us = WD_LEAVE_US;
+    bool may_leave = !vstart || rest;
+    std::unique_ptr<GwRounds> push;
+    int it = 0;   // rounds before the stretch
+    while (true) {
+        buf[0] = s.L.p;
+        buf[1] = s.Ln.p;
+        launched = 0;
+        int seen = 0;
+        u64 low = 0;
+        double lost = 0.0;
+        bool fin = false, closing = false;
+        auto t0 = WallClock::now();   // of the last round seen
         while (true) {
-            if (ctx->prof) ctx->prof_begin();
-            HIPCHK(hipGraphLaunch(exec, ctx->stream));
-            if (ctx->prof) ctx->prof_end(DLG_K_WCC_RELAX, 0.0);
-            WccDev cur;
-            static_assert(sizeof(WccDev) <= 8 * dlg_ctx::MAPPED_SEQ, "the state fits a mapped slot");
-            ctx->read_words((const u32 *)st, (int)(sizeof(WccDev) / 4), &cur);
-            it = (int)cur.it;
-            if (cur.done) break;
+            while (!closing && launched < seen + 1 + WD_DEPTH && (max_it <= 0 || it + launched < max_it)) launch(false);
+            if (q.empty()) launch(true);   // nothing behind the last round publishes it
+            ctx->wait_mapped(q.front());
+            const volatile u64 *m = ctx->mapped_host(q.front());
+            low = m[0];
+            fin = m[1] != 0;
+            q.pop_front();
+            seen++;
+            fin = fin || (max_it > 0 && it + seen >= max_it);
+            if (fin || (closing && seen == launched)) break;
+            if (seen > 1) pull_us = 0.75 * pull_us + 0.25 * std::min(wall_us(t0), pull_most);   // the rounds are queued: one's time
+            t0 = WallClock::now();
+            lost = std::max(0.0, lost + pull_us - (vstart ? wd_batch_push_us(low, B) : gw_push_us(low)));
+            closing = closing || (may_leave && lost >= leave_us);
         }
-    } catch (...) {
-        (void)hipGraphExecDestroy(exec);
-        (void)hipGraphDestroy(graph);
-        throw;
+        it += seen;
+        if (vstart) {
+            if (fin) {
+                DLG_LAUNCH(ctx, DLG_K_MISC, 12.0 * V, wd_pick_k, sgrid(ctx, V), ctx->block_size, 0, s.L.p, (const u32 *)s.Ln.p,
+                           V, in);
+            } else {
+                wcc_lists(ctx, s, V);
+                fill_u32(ctx, s.counter.p, 1, 0u);
+                DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * V, wd_export_k, grid_for(V, WA_TILE), WA_T, 0, s.L.p, (const u32 *)s.Ln.p, V,
+                           in, (u32)it, s.fnode.p, s.flabel.p, s.counter.p);
+                rest->left = true;
+                rest->nf = low;
+                rest->prev.resize(B);
+                rest->done.resize(B);
+                HIPCHK(hipMemcpyAsync(rest->prev.data(), in.prev, 4 * (size_t)B, hipMemcpyDeviceToHost, ctx->stream));
+                HIPCHK(hipMemcpyAsync(rest->done.data(), in.done, 4 * (size_t)B, hipMemcpyDeviceToHost, ctx->stream));
+                s.Ln.release();   // read by what is queued; the pool is the stream's own
+            }
+            HIPCHK(hipMemcpyAsync(iters->data(), in.iters, 4 * (size_t)B, hipMemcpyDeviceToHost, ctx->stream));
+            ctx->sync();
+            return it;
+        }
+        if (seen & 1) s.L.swap(s.Ln);   // the last round's labels in L, the one before's in Ln
+        if (fin) break;
+        if (!push) {
+            try {
+                wcc_lists(ctx, s, V);
+                push.reset(new GwRounds(ctx, s, ix, nbr, ix.n, 16));
+            } catch (const Error &e) {   // pulls need less
+                if (e.status != DLG_OUT_OF_MEMORY) throw;
+                may_leave = false;
+            }
+        }
+        if (push) {
+            fill_u32(ctx, s.counter.p, 1, 0u);
+            DLG_LAUNCH(ctx, DLG_K_MISC, 16.0 * V, wcc_changed_k, grid_for(V, WA_TILE), WA_T, 0, s.Ln.p, (const u32 *)s.L.p, V,
+                       s.fnode.p, s.flabel.p, s.counter.p);   // both arrays hold the last labels now
+            int replays = 0;
+            const WccDev h = push->run(low, low, it, max_it, [&](double us) { return replays++ == 0 || us <= pull_us; });   // the first one sets up
+            it = (int)h.it;
+            if (s.L.p != push->L) s.L.swap(s.Ln);
+            if (h.done) break;
+            low = h.prev;
+            leave_us *= 8.0;   // rounds that grew again: the next time costs as much
+        }
+        DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * V, wd_again_k, sgrid(ctx, V), ctx->block_size, 0, st, (const u32 *)s.L.p, s.Ln.p, V, low);
     }
-    (void)hipGraphExecDestroy(exec);
-    (void)hipGraphDestroy(graph);
+    if (push) {   // as much for the components as there was before
+        push.reset();
+        for (DBuf<u32> *b : {&s.mark, &s.fnode, &s.flabel, &s.nnode, &s.cnt, &s.pstart}) b->release();
+        s.offs.release();
+    }
     return it;
 }
 

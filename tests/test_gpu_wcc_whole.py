@@ -87,3 +87,55 @@ def test_one_workgroup(ctx, orc, kind, n, k):
     same(ctx.run("wcc", rows, max_iterations=k), ctx.run("wcc", rows, max_iterations=k, strategy=2))
     if k == 6 and (kind != "path" or n < 2000):
         same(ctx.run("wcc", rows), orc.wcc(rows))
+
+
+# Few nodes lowered for many rounds in a graph whose pulls cost more than that: the rounds go on by pushes; and back
+# to pulls where many nodes are lowered again.
+def tail(core, n):
+    v = int(core.max()) + 1
+    k = np.arange(n)
+    return np.concatenate([core, np.stack([np.where(k == 0, core.min(), v + k - 1), v + k], 1)]).astype(np.int32)
+
+
+def comb(chains, length, gap, feeder):
+    """`chains` chains at a hub, which settle in `length` rounds; `gap` rounds after the first the hub sees a lower label
+    in each of `feeder` rounds, and so does every chain.  A path beside them has a node fewer to lower in every round, so
+    that no two rounds lower as many."""
+    hub, g0 = feeder, feeder + 1 + chains * length                       # ids: the feeder, the hub, the chains, the gap
+    k = np.arange(chains * length)
+    up = np.where(k % length == 0, hub, hub + k)
+    path = np.concatenate([np.arange(feeder), g0 + np.arange(gap), [hub]])
+    beside = g0 + gap + np.arange(gap + 2 * feeder)
+    return np.concatenate([np.stack([path[:-1], path[1:]], 1), np.stack([up, hub + 1 + k], 1),
+                           np.stack([beside[:-1], beside[1:]], 1)]).astype(np.int32)
+
+
+@pytest.fixture(scope="module")
+def long_graphs():
+    return {"tail": tail(dlg.gen_rmat(17, 2 << 20, 0.57, 0.19, 0.19, 5), 300), "comb": comb(200_000, 40, 200, 100)}
+
+
+@pytest.mark.parametrize("shape", ["tail", "comb"])
+@pytest.mark.parametrize("k", [0, 5, 48, 50, 53, 57, 64, 70, 100, 205, 240, 250, 299])
+def test_few_nodes_left(ctx, long_graphs, shape, k):
+    rows = long_graphs[shape]
+    kw = {"max_iterations": k} if k else {}
+    got = ctx.run("wcc", rows, **kw)
+    same(got, ctx.run("wcc", rows, strategy=2, **kw))
+    if not k:
+        same(got, ctx.run("wcc", rows, strategy=1))
+
+
+@pytest.mark.parametrize("k", [0, 3, 20, 21, 25, 200])
+def test_few_nodes_left_batch(ctx, k):
+    """A batch of 20M edges, which a pull takes longer for than a pushed round of few nodes: instances that stop before,
+    at, and long after the change."""
+    rng = np.random.default_rng(1)
+    inst = [tail(dlg.gen_rmat(20, 10 << 20, 0.57, 0.19, 0.19, 5), 150), np.array([[5, 4]], np.int32),
+            np.stack([np.arange(400), np.arange(1, 401)], 1).astype(np.int32), np.zeros((0, 2), np.int32),
+            rng.integers(0, 1000, (1500, 2)).astype(np.int32), tail(dlg.gen_grid(30, 0.55, 0.01, 20, 3), 40)]
+    kw = {"max_iterations": k} if k else {}
+    res, st = ctx.batch_run("wcc", inst, **kw)
+    for r, rows in zip(res, inst):
+        if len(rows):
+            same(r, ctx.run("wcc", rows, strategy=2, **kw))
