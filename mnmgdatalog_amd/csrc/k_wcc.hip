@@ -1274,6 +1274,11 @@ int wcc_rounds_whole(dlg_ctx *ctx, WccState &s, u64 V, const Index &ix, const u3
     double pull_us = pull_most, leave_us = WD_LEAVE_US;
     bool may_leave = !vstart || rest;
     std::unique_ptr<GwRounds> push;
+    auto end_push = [&]() {   // as much memory for what follows as without it
+        push.reset();
+        for (DBuf<u32> *b : {&s.mark, &s.fnode, &s.flabel, &s.nnode, &s.cnt, &s.pstart}) b->release();
+        s.offs.release();
+    };
     int it = 0;   // rounds before the stretch
     while (true) {
         buf[0] = s.L.p;
@@ -1331,6 +1336,7 @@ int wcc_rounds_whole(dlg_ctx *ctx, WccState &s, u64 V, const Index &ix, const u3
             } catch (const Error &e) {   // pulls need less
                 if (e.status != DLG_OUT_OF_MEMORY) throw;
                 may_leave = false;
+                end_push();
             }
         }
         if (push) {
@@ -1347,11 +1353,7 @@ int wcc_rounds_whole(dlg_ctx *ctx, WccState &s, u64 V, const Index &ix, const u3
         }
         DLG_LAUNCH(ctx, DLG_K_MISC, 8.0 * V, wd_again_k, sgrid(ctx, V), ctx->block_size, 0, st, (const u32 *)s.L.p, s.Ln.p, V, low);
     }
-    if (push) {   // as much for the components as there was before
-        push.reset();
-        for (DBuf<u32> *b : {&s.mark, &s.fnode, &s.flabel, &s.nnode, &s.cnt, &s.pstart}) b->release();
-        s.offs.release();
-    }
+    if (push) end_push();
     return it;
 }
 

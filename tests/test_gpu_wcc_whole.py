@@ -1,5 +1,7 @@
 """WCC by whole-graph pulls: nodes at the edges of the thread, wave and workgroup classes, round limits,
 and batches whose instances stop by their own rule, against the oracle and the pushed rounds."""
+from ctypes import c_uint64
+
 import numpy as np
 import pytest
 
@@ -139,3 +141,24 @@ def test_few_nodes_left_batch(ctx, k):
     for r, rows in zip(res, inst):
         if len(rows):
             same(r, ctx.run("wcc", rows, strategy=2, **kw))
+
+
+def test_pushes_short_of_memory():
+    """A resident graph of many nodes to an edge, whose query has memory for pulls but not for the pushed rounds' lists."""
+    rows = comb(200_000, 40, 200, 100)
+    with dlg.Server(0, workers=1, hbm_budget=8 << 30, retain_bytes=1) as srv:
+        g = srv.add_graph(rows)
+        free = srv.wait(srv.submit("wcc", graph=g))
+    with dlg.Ctx(0) as ctx:
+        want = ctx.run("wcc", rows, strategy=2)
+        d = ctx.upload(rows)
+        for mb in range(900, 2000, 50):   # the graph's build takes most; each is out of memory, or right
+            ctx.L.dlg_test_budget(ctx.h, c_uint64(mb << 20))
+            try:
+                same(ctx.run("wcc", None, device_rows=d, n=len(rows)), want)
+            except dlg.DlgError as e:
+                assert e.status == dlg.DLG_OUT_OF_MEMORY
+        ctx.L.dlg_test_budget(ctx.h, c_uint64(0))
+        ctx.free(d)
+    assert free["status"] == 0 and free["attempts"] == 1
+    same(free, want)
