@@ -815,16 +815,15 @@ static void run_sj(dlg_ctx *ctx, const int32_t *d_rows, u64 n, const Opts &o, dl
 void wcc_solve(dlg_ctx *ctx, const WccGraph &g, const Opts &o, PhaseClock &pc, dlg_result *res) {
     pc.mark(DLG_PH_INIT);
     WccState s(ctx);
-    int it = -1;
+    int it = 0;
     pc.mark(DLG_PH_JOIN);
-    if (o.strategy == 0 && o.relax == WCC_AUTO && g.ne <= WD_MAX_EDGES)
+    if (o.strategy == 0 && o.relax == WCC_AUTO && g.ne <= WD_MAX_EDGES) {
         it = wcc_rounds_whole(ctx, s, g.V, g.ix, g.nbr.p, o.max_it);
-    const bool graph = o.strategy == 2 || (o.strategy == 0 && o.relax == WCC_AUTO && g.ne <= (1ull << 25));
-    if (it < 0) wcc_setup(ctx, s, g.V);
-    if (it < 0 && graph) {
+    } else if (o.strategy == 2) {
+        wcc_setup(ctx, s, g.V);
         it = wcc_rounds_graph(ctx, s, g.ix, g.nbr.p, g.ne, o.max_it, 16);
-    } else if (it < 0) {
-        it = 0;
+    } else {
+        wcc_setup(ctx, s, g.V);
         u64 nf = g.V;
         u64 prev = g.V;                                    // wcc.cu:236-242
         while (true) {

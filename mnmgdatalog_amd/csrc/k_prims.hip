@@ -134,7 +134,8 @@ constexpr u64 FP_MIN = 1ull << 16;
 struct FpPoint {
     u64 r[FP_POINTS], s[FP_POINTS];   // in [0, p)
 };
-// a b mod p, for a < 2^62 and b < 2^63; below 2^61 + 8, not always below p
+// a b mod p, for a b < 2^124 (its two halves' sum fits in 64 bits); below 2^61 + 8, not always
+// below p.  The terms multiplied up are below 2^62 + 2^61, the products they meet below 2^61 + 8.
 __device__ __forceinline__ u64 fp_mul(u64 a, u64 b) {
     const u64 lo = a * b, hi = __umul64hi(a, b);
     const u64 t = (lo & FP_P) + ((lo >> 61) | (hi << 3));
