@@ -121,32 +121,45 @@ constexpr size_t PINNED_TOTAL_MAX = 32ull << 30;   // page-locked host memory he
 constexpr size_t PINNED_KEEP_MAX = 1ull << 30;
 std::mutex pinned_mu;
 std::unordered_map<void *, size_t> pinned_blocks;   // handed out: size class
-std::map<size_t, std::vector<void *>> pinned_free;
+void *pinned_free[4 * 64];                          // kept, by class: each block begins with the next one's address
 size_t pinned_total = 0, pinned_kept = 0;           // total: handed out and kept
 int contexts = 0;
 std::atomic<int64_t> blocks_until_failure{-1};      // for tests: < 0 none
 
+// The list of a size class (Pool::round_size: 4 + q quarters of 2^k), and the class of a list.
+int pinned_list(size_t sz) {
+    const int k = 63 - __builtin_clzll((unsigned long long)sz);
+    return 4 * k + (int)((sz >> (k - 2)) & 3);
+}
+size_t pinned_class(int list) { return (size_t)(4 + list % 4) << (list / 4 - 2); }
+
+// Giving blocks back allocates nothing: it goes on in destructors and in calls that return no status.
 // Takes kept blocks out of the books, largest first, until at most `keep` bytes
 // remain; the caller frees them without the lock.
-std::vector<void *> pinned_trim(size_t keep) {
-    std::vector<void *> out;
-    while (pinned_kept > keep) {
-        auto it = std::prev(pinned_free.end());
-        out.push_back(it->second.back());
-        it->second.pop_back();
-        pinned_kept -= it->first;
-        pinned_total -= it->first;
-        if (it->second.empty()) pinned_free.erase(it);
-    }
+void *pinned_trim(size_t keep) {
+    void *out = nullptr;
+    for (int l = 4 * 64 - 1; pinned_kept > keep; l--)
+        while (pinned_kept > keep && pinned_free[l]) {
+            void *p = pinned_free[l];
+            pinned_free[l] = *(void **)p;
+            *(void **)p = out;
+            out = p;
+            pinned_kept -= pinned_class(l);
+            pinned_total -= pinned_class(l);
+        }
     return out;
 }
-void pinned_release(const std::vector<void *> &blocks) {
-    for (void *p : blocks) (void)hipHostFree(p);
+void pinned_release(void *blocks) {
+    while (blocks) {
+        void *next = *(void **)blocks;
+        (void)hipHostFree(blocks);
+        blocks = next;
+    }
 }
 }  // namespace
 
 void host_contexts(int change) {
-    std::vector<void *> gone;
+    void *gone = nullptr;
     {
         std::lock_guard<std::mutex> lk(pinned_mu);
         contexts += change;
@@ -159,17 +172,16 @@ void *host_block_alloc(size_t bytes) {
     if (blocks_until_failure.load(std::memory_order_relaxed) >= 0 && blocks_until_failure.fetch_sub(1) == 0) return nullptr;
     const size_t sz = Pool::round_size(bytes);
     if (bytes <= PINNED_BLOCK_MAX) {
-        std::vector<void *> gone;
+        void *gone = nullptr;
         bool room;
         {
             std::lock_guard<std::mutex> lk(pinned_mu);
-            auto it = pinned_free.find(sz);
-            if (it != pinned_free.end()) {
-                void *p = it->second.back();
-                it->second.pop_back();
-                if (it->second.empty()) pinned_free.erase(it);
+            void *&head = pinned_free[pinned_list(sz)];
+            if (head) {
+                void *p = head;
+                pinned_blocks.emplace(p, sz);   // may throw: nothing is changed yet
+                head = *(void **)p;
                 pinned_kept -= sz;
-                pinned_blocks[p] = sz;
                 return p;
             }
             if (pinned_total + sz > PINNED_TOTAL_MAX) gone = pinned_trim(0);   // kept blocks make room first
@@ -183,8 +195,12 @@ void *host_block_alloc(size_t bytes) {
             if (!ok) (void)hipGetLastError();
             std::lock_guard<std::mutex> lk(pinned_mu);
             if (ok) {
-                pinned_blocks[p] = sz;
-                return p;
+                try {
+                    pinned_blocks.emplace(p, sz);
+                    return p;
+                } catch (const std::bad_alloc &) {
+                    (void)hipHostFree(p);
+                }
             }
             pinned_total -= sz;
         }
@@ -194,14 +210,16 @@ void *host_block_alloc(size_t bytes) {
 
 void host_block_free(void *p) {
     if (!p) return;
-    std::vector<void *> gone;
+    void *gone = nullptr;
     {
         std::lock_guard<std::mutex> lk(pinned_mu);
         auto it = pinned_blocks.find(p);
         if (it != pinned_blocks.end()) {
             const size_t sz = it->second;
             pinned_blocks.erase(it);
-            pinned_free[sz].push_back(p);
+            void *&head = pinned_free[pinned_list(sz)];
+            *(void **)p = head;
+            head = p;
             pinned_kept += sz;
             gone = pinned_trim(contexts ? PINNED_KEEP_MAX : 0);
             p = nullptr;
