@@ -89,3 +89,19 @@ def test_no_room_for_the_lists(orc):
         got = srv.wait(srv.submit("tc", rows))
     assert (got["iterations"], got["output_size"]) == (want["iterations"], want["output_size"])
     assert np.array_equal(got["rows"], want["rows"])
+
+
+@pytest.mark.parametrize("width", [16_400, 20_000])
+@pytest.mark.parametrize("k", [0, 1, 2, 3, 4, 5])
+def test_few_large_rings(ctx, width, k):
+    """Random neighbours, eight of them: the rings reach most words in a few rounds.  The first buffer has wpr / 4 entries a
+    source (wpr words a row) and takes the rounds of 8 and 56 ends; the second, four times as large, does not take the next
+    two (392 ends in 54 % of the words, 2,744 in nearly all): the run starts again with buffers for two rounds of any size."""
+    rng = np.random.default_rng(width)
+    rows = both(np.concatenate([np.stack([np.arange(width), rng.permutation(width)], 1) for _ in range(4)]))
+    kw = {"keep_output": False, "check_output": 1, **({"max_iterations": k} if k else {})}
+    got, want = ctx.run("tc", rows, **kw), ctx.run("tc", rows, queue=1, **kw)
+    for f in ("iterations", "output_size", "raw_join_rows", "output_sum", "output_order_breaks"):
+        assert got[f] == want[f]
+    if not k:
+        assert got["output_size"] == width * width
