@@ -215,7 +215,7 @@ typedef struct dlg_opts {
                                 least 16,384 ids), 1 never, 2 always.  Same output   */
     int32_t relax;           /* WCC rounds launched one by one: 0 auto (round one read
                                 off the sorted adjacency lists, later rounds pulled
-                                when the frontier's edges are at least half of all
+                                when the frontier's edges are at least an eighth of all
                                 edges, pushed otherwise); 1 push every round (one
                                 thread per frontier edge, atomic minimum at the far
                                 end: the reference's join order); 2 pull every round

@@ -721,7 +721,7 @@ struct WccState {
         : L(c), Ln(c), mark(c), fnode(c), flabel(c), nnode(c), cnt(c), pstart(c), counter(c), offs(c) {}
 };
 void wcc_setup(dlg_ctx *ctx, WccState &s, u64 V);
-// WCC round forms: WCC_AUTO pulls when the frontier's edges are at least half
+// WCC round forms: WCC_AUTO pulls when the frontier's edges are at least an eighth
 // of the graph's, WCC_PUSH walks the frontier's edges, WCC_PULL every node's.
 enum { WCC_AUTO = 0, WCC_PUSH = 1, WCC_PULL = 2 };
 // One round over frontier of size nf; returns the new frontier size.
