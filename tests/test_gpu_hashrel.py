@@ -125,3 +125,17 @@ def test_served_within_its_reservation(ctx, n, m, seed):
         got = srv.wait(srv.submit("tc", rows))
     assert got["status"] == 0 and got["attempts"] == 1
     same(got, ctx.run("tc", rows, strategy=2))
+
+
+@pytest.mark.parametrize("prog,ins,outs", [("tc", 3000, 9000), ("tc", 40, 70_000), ("sg", 10, 6000)])
+def test_star(ctx, prog, ins, outs):
+    """A hub's pairs, nearly all new, from few probes: the set grows past them in a few steps, and the next round, of as many
+    rows and none new, begins with the room there is."""
+    hub = 7
+    rows = np.concatenate([np.stack([100 + np.arange(ins), np.full(ins, hub)], 1),
+                           np.stack([np.full(outs, hub), 100 + ins + np.arange(outs)], 1), [[100 + ins, hub]]])
+    rows = (rows * 20_011).astype(np.int32)
+    kw = {"keep_output": False, "check_output": 1}
+    got, want = ctx.run(prog, rows, **kw), ctx.run(prog, rows, strategy=2, **kw)
+    for f in ("iterations", "output_size", "raw_join_rows", "output_sum", "output_order_breaks"):
+        assert got[f] == want[f]
