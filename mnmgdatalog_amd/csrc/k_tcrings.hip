@@ -446,15 +446,22 @@ __global__ __launch_bounds__(WAVE) void tc_ring_turn_k(TgArgs a, u32 round) {
 }
 
 // Entries per region at most: two rounds of any size, as a workgroup's sources have at most every word each.
-static u64 tg_region_max(u64 W, u64 wpr) {
+static constexpr u64 tg_region_max(u64 W, u64 wpr) {
     const u64 grid = TG_PARTS * (((W + TG_R - 1) / TG_R + TG_PARTS - 1) / TG_PARTS);
     return 2 * ((grid + TG_REGIONS - 1) / TG_REGIONS) * TG_R * wpr;
 }
 
+// Rows of which seven fit a CU's LDS (184,320 ids).  Wider ones leave too few waves for the
+// chain that a round is: parts of paths, 4,500 to 7,200 rounds, against the row kernel 370 and
+// 427 ms at 160,000 ids, 431 and 435 at 180,000, 604 and 568 at 200,000, 1,169 and 776 at 262,016;
+// grids of 8,100 ids each 68 and 84, 84 and 98, 98 and 110, 160 and 147.
+constexpr u64 TG_MAX_WPR = 5760;
+static_assert(TG_REGIONS * tg_region_max(32 * TG_MAX_WPR, TG_MAX_WPR) < 1ull << 32, "list positions are 32-bit");
+
 bool tc_rings_takes(const TcRows &tr, const RowMap &F) {
     if (!tr.ell.p || F.blocks.size() != 1) return false;
     const u64 wpr = F.blocks[0].wpr;
-    return wpr >= TG_D && TG_REGIONS * tg_region_max(F.W, wpr) < 1ull << 32;   // list positions are 32-bit
+    return wpr >= TG_D && wpr <= TG_MAX_WPR;
 }
 
 // One run with buffers of region[i] entries per region to begin with; -1 (F then

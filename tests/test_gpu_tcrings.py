@@ -105,3 +105,9 @@ def test_few_large_rings(ctx, width, k):
         assert got[f] == want[f]
     if not k:
         assert got["output_size"] == width * width
+
+
+# the widest range taken, and the first one that is not
+@pytest.mark.parametrize("width", [184_319, 184_320, 184_321])
+def test_widest(ctx, width):
+    check(ctx, forest(width, 6000, width, extra=2000))
